@@ -1,0 +1,894 @@
+// Flat parallel-beam kernels (included by tsx.hip): scans whose rays stay
+// within a slice of constant z (parallel beam, ray direction perpendicular to
+// z, detector v parallel to z, stepping axis x or y at every angle).
+//
+// There the Joseph weights factor: ray (a, i, j) meets slice n of its stepping
+// axis at the in-slice position q(a, j, n), the same for every detector row i,
+// and at the height t(a, i, j), the same for every slice. So
+//   forward:   G[a, j, z] = sum_n lerp_q x[n, ., z],  y[i, a, j] = l lerp_t G[a, j, .]
+//   backward:  U[a, j, z] = sum_i L(t - z) l y[i, a, j],
+//              x[n, c, z] = sum_a sum_j L(q(a, j, n) - c) U[a, j, z],
+// and the sums over slices and columns have one weight for a whole line along
+// z. The kernels keep z contiguous (volume turned to [x][y][w], G and U as
+// [angle][column][w]; w = (batch entry, z), so that short stacks and 2D
+// slices of a batch fill the lanes), take 64 ZL consecutive w per wave (ZL per
+// lane) and broadcast the weights from the lane that formed them
+// (v_readlane): 2 fma per (ray, slice, z) or (voxel, column) instead of a
+// gather and a bilinear interpolation of their own.
+//
+// Every lane's arithmetic and its order depend only on the plan, never on the
+// position of its w in a wave, so single, batched and fused launches give
+// the same bits.
+#pragma once
+
+#include "tsx_plan.h"
+#include "fp_kernels.h"
+#include "bp_kernels.h"
+
+namespace tsx {
+
+constexpr int FLAT_MAX = MAX_FUSED;  // instances of one launch
+constexpr int FLAT_FW = 8;           // forward projector: waves per block
+constexpr int FLAT_JW = 8;           // forward projector: detector columns per wave
+constexpr int FLAT_NARROW = 40, FLAT_WIDE = 64;  // forward: most voxel columns staged per slice (two kernels)
+// forward: slices (n / FLAT_SUM of the volume) summed before they join the rest of a ray's sum.
+// One running sum over the 256 slices of a slice stack rounds to 3.6e-7 of the result, the
+// padded kernels' two to 1.9e-7, sums of 32 to 1.6e-7 (for 1 to 2 % of the time).
+constexpr int FLAT_SUM = 32;
+constexpr int FLAT_BX = 16, FLAT_BY = 8;  // backprojector: voxel columns per brick (one wave per y)
+constexpr int FLAT_BSC = 64;         // most detector columns staged per angle
+
+// One instance as seen by the kernels of a launch over the angles
+// ang[0 .. kn - 1] of the plan's axis-ordered table.
+struct FlatView {
+    const FlatAngle *ang;
+    int kn;                 // angles of the launch
+    int n_angles, rows, cols, nx, ny, nz;
+    int W, Wp;              // batch entries x nz, and the pitch of a line (a multiple of 4)
+    float *vol, *proj;      // caller's data: read or written, entries vs and ps floats apart
+    int64_t vs, ps;
+    float *turned;          // forward: the volume as [x][y][Wp]
+    float *lines;           // G or U as [kn][cols][Wp]
+    Epilogue ep;
+    int up;                 // backward: pixels per coarse pixel edge (refined detector), else 1
+    int stage;              // columns staged at a time
+    // forward: group[g] .. group[g + 1] - 1 are the angles (of the plan) of
+    // group g, at most ag; k0 the launch's first angle; column tiles
+    const int32_t *group;
+    int groups, ag, k0, tiles;
+    int bx, by, parts, part_len;  // backward: bricks, angle parts
+    float *partial;         // backward: the parts' sums ([entry][part][z][y][x]), null for one part
+    int chunks;             // chunks of 64 ZL of w
+};
+
+struct FlatMulti {
+    FlatView v[FLAT_MAX];
+    int begin[FLAT_MAX + 1];
+    int n;
+    int shift;  // chunk size of the XCD order (xcd_logical)
+};
+
+template <int ZL>
+struct FlatVec {
+    float v[ZL];
+};
+
+
+template <int ZL>
+__device__ __forceinline__ FlatVec<ZL> flat_load(const float *p)
+{
+    FlatVec<ZL> r;
+    if constexpr (ZL == 4) {
+        const float4 t = *reinterpret_cast<const float4 *>(p);
+        r.v[0] = t.x;
+        r.v[1] = t.y;
+        r.v[2] = t.z;
+        r.v[3] = t.w;
+    } else if constexpr (ZL == 2) {
+        const float2 t = *reinterpret_cast<const float2 *>(p);
+        r.v[0] = t.x;
+        r.v[1] = t.y;
+    } else {
+        r.v[0] = *p;
+    }
+    return r;
+}
+
+template <int ZL>
+__device__ __forceinline__ void flat_store(float *p, const FlatVec<ZL> &r)
+{
+    if constexpr (ZL == 4)
+        *reinterpret_cast<float4 *>(p) = make_float4(r.v[0], r.v[1], r.v[2], r.v[3]);
+    else if constexpr (ZL == 2)
+        *reinterpret_cast<float2 *>(p) = make_float2(r.v[0], r.v[1]);
+    else
+        *p = r.v[0];
+}
+
+// A line's values = r (first) or += r; r = 0 after it.
+template <int ZL>
+__device__ __forceinline__ void flat_join(float *p, FlatVec<ZL> &r, bool first)
+{
+    FlatVec<ZL> t;
+#pragma unroll
+    for (int z = 0; z < ZL; ++z) t.v[z] = 0.0f;
+    if (!first) t = flat_load<ZL>(p);
+#pragma unroll
+    for (int z = 0; z < ZL; ++z) {
+        t.v[z] += r.v[z];
+        r.v[z] = 0.0f;
+    }
+    flat_store<ZL>(p, t);
+}
+
+__device__ __forceinline__ float lane_f(float v, int lane)
+{
+    return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), lane));
+}
+
+__device__ __forceinline__ int lane_i(int v, int lane) { return __builtin_amdgcn_readlane(v, lane); }
+
+// ---------------------------------------------------------------------------
+// layout passes: 32 x 32 tiles through LDS, blocks of 32 x 8 threads
+// ---------------------------------------------------------------------------
+
+// turned[x][y][w] from vol[z][y][x] of every entry: a block per tile of 32 x
+// by 32 w of one y.
+__host__ __device__ inline int64_t flat_turn_blocks(const FlatView &v)
+{
+    return (int64_t)((v.nx + 31) / 32) * ((v.W + 31) / 32) * v.ny;
+}
+
+// The line of zeros after `lines` lines of pitch Wp (written by the blocks of
+// a layout pass that start at w0, for the w of their tile).
+__device__ __forceinline__ void flat_zero_line(float *base, int64_t lines, int Wp, int w0)
+{
+    const int w = w0 + threadIdx.x;
+    if (threadIdx.y == 0 && w < Wp) base[lines * Wp + w] = 0.0f;
+}
+
+__global__ void __launch_bounds__(256) flat_turn(FlatMulti M)
+{
+    __shared__ float tile[32][33];
+    const int k = owner_of(M.begin, (int)blockIdx.x);
+    const FlatView &v = M.v[k];
+    const int id = (int)blockIdx.x - M.begin[k];
+    const int tx = threadIdx.x, ty = threadIdx.y;
+    const int tiles_x = (v.nx + 31) / 32, tiles_w = (v.W + 31) / 32;
+    const int x0 = (id % tiles_x) * 32, y = (id / tiles_x) % v.ny, w0 = (id / (tiles_x * v.ny)) * 32;
+    if (w0 >= tiles_w * 32) return;
+    int b = (w0 + ty) / v.nz, z = w0 + ty - b * v.nz;
+    for (int r = ty; r < 32; r += 8) {
+        const int x = x0 + tx;
+        float t = 0.0f;
+        if (w0 + r < v.W && x < v.nx) t = v.vol[b * v.vs + ((int64_t)z * v.ny + y) * v.nx + x];
+        tile[r][tx] = t;
+        for (z += 8; z >= v.nz; z -= v.nz) ++b;
+    }
+    __syncthreads();
+    for (int r = ty; r < 32; r += 8) {
+        const int x = x0 + r, w = w0 + tx;
+        if (x < v.nx && w < v.Wp) v.turned[((int64_t)x * v.ny + y) * v.Wp + w] = tile[tx][r];
+    }
+    if (x0 == 0 && y == 0) flat_zero_line(v.turned, (int64_t)v.nx * v.ny, v.Wp, w0);
+}
+
+// y[i, a, j] = l lerp_t G[a, j, .] through the epilogue: a block per tile of
+// 32 columns by 32 (entry, row) of one angle.
+__host__ __device__ inline int64_t flat_rows_blocks(const FlatView &v)
+{
+    return (int64_t)((v.cols + 31) / 32) * ((v.W / v.nz * v.rows + 31) / 32) * v.kn;
+}
+
+// Interpolation of one detector row in a line: the value at z and the next
+// one with weight w (z = -2: the row misses the volume).
+struct FlatRow {
+    int z;
+    float w;
+};
+
+__device__ __forceinline__ FlatRow flat_row(const FlatAngle &A, int i, int j, int nz)
+{
+    const double t = A.t0 + (double)j * A.tj + (double)i * A.tv;
+    FlatRow r = {-2, 0.0f};
+    if (t > -1.0 && t < (double)nz) {
+        const double f = floor(t);
+        r.z = (int)f;
+        r.w = (float)(t - f);
+    }
+    return r;
+}
+
+__global__ void __launch_bounds__(256) flat_rows(FlatMulti M)
+{
+    __shared__ float tile[32][33];
+    __shared__ FlatRow rows_of[32];
+    __shared__ int entry_of[32], index_of[32];
+    const int q = owner_of(M.begin, (int)blockIdx.x);
+    const FlatView &v = M.v[q];
+    const int id = (int)blockIdx.x - M.begin[q];
+    const int tx = threadIdx.x, ty = threadIdx.y;
+    const int tiles_j = (v.cols + 31) / 32, all = v.W / v.nz * v.rows;
+    const int j0 = (id % tiles_j) * 32, k = (id / tiles_j) % v.kn, r0 = (id / (tiles_j * v.kn)) * 32;
+    if (r0 >= all) return;
+    const FlatAngle &A = v.ang[k];
+    // (the row's place in a line is the same for every column unless the
+    // detector's u axis leaves the slices: formed once per row then, as the
+    // FP64 positions and divisions would otherwise bound this pass)
+    const bool level = A.tj == 0.0;
+    if (ty == 0) {
+        const int b = (r0 + tx) / v.rows, i = r0 + tx - b * v.rows;
+        entry_of[tx] = b;
+        index_of[tx] = i;
+        rows_of[tx] = flat_row(A, i, 0, v.nz);
+    }
+    __syncthreads();
+    const int b = entry_of[tx], i = index_of[tx];
+    const FlatRow fr = rows_of[tx];
+    const float *g0 = v.lines + ((int64_t)k * v.cols + j0) * v.Wp + b * v.nz;
+    for (int c = ty; c < 32; c += 8) {
+        float y = 0.0f;
+        if (j0 + c < v.cols && r0 + tx < all) {
+            const FlatRow r = level ? fr : flat_row(A, i, j0 + c, v.nz);
+            if (r.z > -2) {
+                const float *g = g0 + (int64_t)c * v.Wp + r.z;
+                const float lo = r.z >= 0 ? g[0] : 0.0f, hi = r.z + 1 < v.nz ? g[1] : 0.0f;
+                y = A.len * fmaf(r.w, hi - lo, lo);
+            }
+        }
+        tile[c][tx] = y;
+    }
+    __syncthreads();
+    for (int r = ty; r < 32; r += 8)
+        if (r0 + r < all && j0 + tx < v.cols)
+            emit(v.proj + entry_of[r] * v.ps, ((int64_t)index_of[r] * v.n_angles + A.a) * v.cols + j0 + tx, entry_of[r],
+                 tile[tx][r], v.ep);
+}
+
+// U[a, j, z] = sum_i L(t - z) l y[i, a, j]: a block per tile of 32 columns by
+// 32 w of one angle. The rows i with |t - z| < 1 are found in FP64 (t is
+// affine in i), and read along the columns.
+__host__ __device__ inline int64_t flat_splat_blocks(const FlatView &v)
+{
+    return (int64_t)((v.cols + 31) / 32) * ((v.W + 31) / 32) * v.kn;
+}
+
+// The detector rows i .. i + n - 1 with a weight at height z: row i + e has
+// the weight 1 - |d + e tv| (FP64 position of the first, rows at most a few).
+struct FlatSpan {
+    int i, n;
+    float d;
+};
+
+__device__ __forceinline__ FlatSpan flat_span(const FlatAngle &A, int z, int j, int rows)
+{
+    const double tt = A.t0 + (double)j * A.tj, inv = 1.0 / A.tv, half = fabs(inv), mid = ((double)z - tt) * inv;
+    const int lo = (int)fmax(0.0, ceil(mid - half)), hi = (int)fmin((double)(rows - 1), floor(mid + half));
+    FlatSpan s = {lo, max(0, hi - lo + 1), (float)(tt + (double)lo * A.tv - (double)z)};
+    return s;
+}
+
+__global__ void __launch_bounds__(256) flat_splat(FlatMulti M)
+{
+    __shared__ float tile[32][33];
+    __shared__ FlatSpan spans[32];
+    __shared__ int entry_of[32];
+    const int q = owner_of(M.begin, (int)blockIdx.x);
+    const FlatView &v = M.v[q];
+    const int id = (int)blockIdx.x - M.begin[q];
+    const int tx = threadIdx.x, ty = threadIdx.y;
+    const int tiles_j = (v.cols + 31) / 32;
+    const int j0 = (id % tiles_j) * 32, k = (id / tiles_j) % v.kn, w0 = (id / (tiles_j * v.kn)) * 32;
+    if (w0 >= v.W) return;
+    const FlatAngle &A = v.ang[k];
+    const bool level = A.tj == 0.0;  // (as in flat_rows)
+    if (ty == 0) {
+        entry_of[tx] = (w0 + tx) / v.nz;
+        spans[tx] = flat_span(A, w0 + tx - entry_of[tx] * v.nz, 0, v.rows);
+    }
+    __syncthreads();
+    const int j = j0 + tx, up = v.up, coarse = up == 1 ? v.cols : v.cols / up;
+    const float scale = A.len / (float)(up * up), tv = (float)A.tv;
+    const int64_t line = (int64_t)v.n_angles * coarse;
+    const float *col = v.proj + (int64_t)A.a * coarse + (up == 1 ? j : j / up);
+    for (int r = ty; r < 32; r += 8) {
+        float u = 0.0f;
+        if (j < v.cols && w0 + r < v.W) {
+            const int b = entry_of[r];
+            const FlatSpan s = level ? spans[r] : flat_span(A, w0 + r - b * v.nz, j, v.rows);
+            const float *y = col + b * v.ps;
+            for (int e = 0; e < s.n; ++e) {
+                const float wgt = 1.0f - fabsf(fmaf((float)e, tv, s.d));
+                // (rows of no weight are not read: they may hold infinities)
+                if (wgt > 0.0f) u = fmaf(wgt, scale * y[(up == 1 ? s.i + e : (s.i + e) / up) * line], u);
+            }
+        }
+        tile[r][tx] = u;
+    }
+    __syncthreads();
+    for (int c = ty; c < 32; c += 8) {
+        const int jc = j0 + c, w = w0 + tx;
+        if (jc < v.cols && w < v.Wp) v.lines[((int64_t)k * v.cols + jc) * v.Wp + w] = tile[tx][c];
+    }
+    if (j0 == 0 && k == 0) flat_zero_line(v.lines, (int64_t)v.kn * v.cols, v.Wp, w0);
+}
+
+// ---------------------------------------------------------------------------
+// forward: G[a, j, w]
+// ---------------------------------------------------------------------------
+// A block of 8 waves takes a group of at most `ag` (4 or 2) neighbouring
+// angles, 64 / ag neighbouring detector columns and 64 ZL of w; a wave 8
+// columns of one angle. The block goes through the slices in step: the voxel
+// columns that its rays meet in the next slice are read (coalesced, once for
+// all angles: neighbouring angles meet nearly the same ones) while the present
+// one is summed from LDS (two buffers, one barrier per slice).
+//
+// Bound: vector ALU issue (half of the time) and the staged lines from L2.
+// Per (ray, slice) 3 readlane, 1 address and 2 ZL fma, i.e. 3 instructions
+// per 64 samples at ZL = 4 (19, and a gather that takes 27 cycles of the
+// texture address unit, in fp_padded). Read from global memory directly, a
+// ray's two lines would take 8 cycles of the 64-byte L1 port per 64 samples,
+// hence the staging, and the sharing between angles. Steps of two slices at
+// ZL = 2 halve the blocks per CU (LDS): 3.9 against 2.5 ms at 75 x 441 x 441,
+// 361 angles, 75 x 623 (fp_padded: 2.96 with its layouts). 8 x 128^3, 180
+// angles, 128 x 192: 0.97 ms with both layout passes against 2.56.
+template <int ZL, int SW>
+__global__ void __launch_bounds__(64 * FLAT_FW) fp_flat(FlatMulti M)
+{
+    extern __shared__ __align__(16) float flat_lds[];
+    __shared__ float line_r[FLAT_FW], line_a[FLAT_FW];
+    __shared__ int range_lo[FLAT_FW], range_hi[FLAT_FW];
+    constexpr int CF = 64 * ZL;  // floats per staged column
+    const int logical = xcd_logical(M.shift);
+    if (logical >= M.begin[M.n]) return;
+    const int inst = owner_of(M.begin, logical);
+    const FlatView &v = M.v[inst];
+    const int id = logical - M.begin[inst];
+    const int g = id % v.groups, jt = (id / v.groups) % v.tiles, w0 = (id / (v.groups * v.tiles)) * CF;
+    const int ag = v.ag, Wp = v.Wp, cols = v.cols, SC = v.stage;
+    const int k0 = v.group[g] - v.k0, cnt = v.group[g + 1] - v.group[g];
+    const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int ai = wv % ag;
+    const bool live = ai < cnt;  // (the waves past the group's last angle only stage)
+    const int jb = (jt * (FLAT_FW / ag) + wv / ag) * FLAT_JW;
+    typedef const __attribute__((address_space(4))) FlatAngle ConstAngle;
+    ConstAngle &A = ((ConstAngle *)v.ang)[k0 + min(ai, cnt - 1)];
+    const int m = A.m;
+    const int nm = m == 0 ? v.nx : v.ny, nc = m == 0 ? v.ny : v.nx;
+    // voxel column (n, c) starts at n sn + c sc
+    const int64_t sn = m == 0 ? (int64_t)v.ny * Wp : Wp, sc = m == 0 ? Wp : (int64_t)v.ny * Wp;
+    const int nref = nm / 2;
+    const int jj = lane & 7, nn = lane >> 3;
+    // the ray of column jb + jj: q(n) = R + (n - nref) a2, slices with q in (-1, nc)
+    const double Rd = A.q0 + A.qm * (double)nref + A.qj * (double)min(jb + jj, cols - 1);
+    int lo = 0, hi = nm - 1;
+    if (A.qm != 0.0) {
+        const double t0 = (-1.0 - Rd) / A.qm, t1 = ((double)nc - Rd) / A.qm;
+        lo = max(0, (int)fmax(ceil(fmin(t0, t1) + nref), -1e9));
+        hi = min(nm - 1, (int)fmin(floor(fmax(t0, t1) + nref), 1e9));
+    } else if (!(Rd > -1.0 && Rd < (double)nc)) {
+        lo = nm;
+        hi = -1;
+    }
+    if (lo > hi) {
+        lo = nm;
+        hi = -1;
+    }
+    const float rmin = wave_minf((float)Rd);
+    lo = wave_min(lo);
+    hi = wave_max(hi);
+    if (lane == 0) {
+        line_r[wv] = rmin;
+        line_a[wv] = (float)A.qm;
+        range_lo[wv] = lo;
+        range_hi[wv] = hi;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int e = 0; e < FLAT_FW; ++e) {
+        lo = min(lo, range_lo[e]);
+        hi = max(hi, range_hi[e]);
+    }
+    lo = __builtin_amdgcn_readfirstlane(lo);
+    hi = __builtin_amdgcn_readfirstlane(hi);
+    const int w = w0 + lane * ZL;
+    FlatVec<ZL> acc[FLAT_JW];
+#pragma unroll
+    for (int e = 0; e < FLAT_JW; ++e)
+#pragma unroll
+        for (int z = 0; z < ZL; ++z) acc[e].v[z] = 0.0f;
+    // (lanes past the last w read the line's last values; nothing of theirs is written)
+    const float *src = v.turned + min(w, Wp - ZL);
+    const int64_t sc8 = sc * FLAT_FW;
+    FlatVec<ZL> next[SW];
+    int kbv = 0;  // lane's first staged column of slice lo + 64 i + lane
+    auto bases = [&](int n) {
+        const float dn = (float)(n + lane - nref);
+        float q = fmaf(dn, line_a[0], line_r[0]);
+#pragma unroll
+        for (int e = 1; e < FLAT_FW; ++e) q = fminf(q, fmaf(dn, line_a[e], line_r[e]));
+        // (the margin exceeds the FP32 rounding of the positions)
+        kbv = (int)floorf(fminf(fmaxf(q - 2e-3f, -1e8f), 1e8f));
+    };
+    // the staged columns of slice n: column kb + s in place s, zeros beyond the volume
+    auto load = [&](int n) {
+        const int c0 = lane_i(kbv, (n - lo) & 63) + wv;
+        const float *p = src + ((int64_t)n * sn + (int64_t)c0 * sc);
+#pragma unroll
+        for (int e = 0; e < SW; ++e) {
+            if ((unsigned)(c0 + e * FLAT_FW) < (unsigned)nc) {
+                next[e] = flat_load<ZL>(p + e * sc8);
+            } else {
+#pragma unroll
+                for (int z = 0; z < ZL; ++z) next[e].v[z] = 0.0f;
+            }
+        }
+    };
+    if (lo <= hi) {
+        bases(lo);
+        load(lo);
+    }
+    // the sums of FLAT_SUM slices join the lines in memory
+    float *out = v.lines + ((int64_t)(k0 + ai) * cols + jb) * Wp + w;
+    bool first = true;
+    auto flush = [&]() {
+        if (live && w < Wp) {
+#pragma unroll
+            for (int e = 0; e < FLAT_JW; ++e)
+                if (jb + e < cols) flat_join<ZL>(out + (int64_t)e * Wp, acc[e], first);
+        }
+        first = false;
+    };
+    int off = 0;  // lane (nn, jj): staged place of ray jj's lower column in slice n + nn, in floats
+    float wl = 0.0f, wh = 0.0f;
+    for (int n = lo; n <= hi; ++n) {
+        const int at = n - lo;
+        if ((at & 7) == 0) {
+            const int kb = __shfl(kbv, (at & 63) + nn, 64);
+            const double q = fma((double)(n + nn - nref), A.qm, Rd), f = floor(q);
+            wh = (float)(q - f);
+            wl = 1.0f - wh;
+            off = min(max((int)fmin(fmax(f, -1e8), 1e8) - kb, 0), SC - 2) * CF;
+        }
+        float *buf = flat_lds + (at & 1) * SC * CF + lane * ZL;
+#pragma unroll
+        for (int e = 0; e < SW; ++e)
+            if (wv + e * FLAT_FW < SC) flat_store<ZL>(buf + (wv + e * FLAT_FW) * CF, next[e]);
+        __syncthreads();
+        if (n < hi) {
+            if (((at + 1) & 63) == 0) bases(n + 1);
+            load(n + 1);
+        }
+        if (live) {
+            constexpr int JB = 4;  // rays whose columns are in flight together
+#pragma unroll
+            for (int e0 = 0; e0 < FLAT_JW; e0 += JB) {
+                FlatVec<ZL> a[JB], b[JB];
+#pragma unroll
+                for (int e = 0; e < JB; ++e) {
+                    const float *p = buf + lane_i(off, (at & 7) * 8 + e0 + e);
+                    a[e] = flat_load<ZL>(p);
+                    b[e] = flat_load<ZL>(p + CF);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int e = 0; e < JB; ++e) {
+                    const int ray = (at & 7) * 8 + e0 + e;
+                    const float fl = lane_f(wl, ray), fh = lane_f(wh, ray);
+#pragma unroll
+                    for (int z = 0; z < ZL; ++z)
+                        acc[e0 + e].v[z] = fmaf(fh, b[e].v[z], fmaf(fl, a[e].v[z], acc[e0 + e].v[z]));
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+        if ((n + 1) % FLAT_SUM == 0) flush();
+    }
+    if (lo > hi || (hi + 1) % FLAT_SUM) flush();
+}
+
+// The same without staging, for short lines (64 of w per wave, one per lane),
+// for the reasons given at bp_flat_direct: a wave of one angle and 4 detector
+// columns reads the two voxel columns of every ray and slice from global
+// memory (the line of zeros after the last one where they lie beyond the
+// volume). 64^3, 96 angles, 64 x 96: 22 us against 49 with fp_flat and 39 with
+// fp_padded (and its layouts 10, here 11 in two passes).
+constexpr int FLAT_DJ = 4;  // detector columns per wave of fp_flat_direct
+
+__global__ void __launch_bounds__(256) fp_flat_direct(FlatMulti M)
+{
+    constexpr int JN = FLAT_DJ, NL = 64 / JN;  // slices whose weights a wave holds
+    const int logical = xcd_logical(M.shift);
+    if (logical >= M.begin[M.n]) return;
+    const int inst = owner_of(M.begin, logical);
+    const FlatView &v = M.v[inst];
+    const int id = logical - M.begin[inst];
+    const int tiles = (v.cols + 4 * JN - 1) / (4 * JN), cols = v.cols, Wp = v.Wp;
+    const int k = id % v.kn, jt = (id / v.kn) % tiles, w0 = (id / (v.kn * tiles)) * 64;
+    const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int jb = (jt * 4 + wv) * JN;
+    if (jb >= cols) return;
+    typedef const __attribute__((address_space(4))) FlatAngle ConstAngle;
+    ConstAngle &A = ((ConstAngle *)v.ang)[k];
+    const int m = A.m;
+    const int nm = m == 0 ? v.nx : v.ny, nc = m == 0 ? v.ny : v.nx;
+    const int sn = m == 0 ? v.ny : 1, sc = m == 0 ? 1 : v.ny;  // voxel column (n, c) is n sn + c sc
+    const int nref = nm / 2, zero = v.nx * v.ny;
+    const int jj = lane % JN, nn = lane / JN;
+    const double Rd = A.q0 + A.qm * (double)nref + A.qj * (double)min(jb + jj, cols - 1);
+    int lo = 0, hi = nm - 1;
+    if (A.qm != 0.0) {
+        const double t0 = (-1.0 - Rd) / A.qm, t1 = ((double)nc - Rd) / A.qm;
+        lo = max(0, (int)fmax(ceil(fmin(t0, t1) + nref), -1e9));
+        hi = min(nm - 1, (int)fmin(floor(fmax(t0, t1) + nref), 1e9));
+    } else if (!(Rd > -1.0 && Rd < (double)nc)) {
+        lo = nm;
+        hi = -1;
+    }
+    if (lo > hi) {
+        lo = nm;
+        hi = -1;
+    }
+    lo = __builtin_amdgcn_readfirstlane(wave_min(lo));
+    hi = __builtin_amdgcn_readfirstlane(wave_max(hi));
+    const int w = w0 + lane;
+    const float *src = v.turned + min(w, Wp - 1);
+    FlatVec<1> acc[JN];
+#pragma unroll
+    for (int e = 0; e < JN; ++e) acc[e].v[0] = 0.0f;
+    static_assert(FLAT_SUM % NL == 0, "steps end where sums do");
+    float *out = v.lines + ((int64_t)k * cols + jb) * Wp + w;
+    bool first = true;
+    auto flush = [&]() {
+        if (w < Wp) {
+#pragma unroll
+            for (int e = 0; e < JN; ++e)
+                if (jb + e < cols) flat_join<1>(out + (int64_t)e * Wp, acc[e], first);
+        }
+        first = false;
+    };
+    for (int n0 = lo / NL * NL; n0 <= hi; n0 += NL) {
+        const int n = n0 + nn;
+        const double q = fma((double)(n - nref), A.qm, Rd), f = floor(q);
+        const float wh = (float)(q - f), wl = 1.0f - wh;
+        const int c = (int)fmin(fmax(f, -1e8), 1e8);
+        const int ra = n < nm && (unsigned)c < (unsigned)nc ? n * sn + c * sc : zero;
+        const int rb = n < nm && (unsigned)(c + 1) < (unsigned)nc ? n * sn + (c + 1) * sc : zero;
+        constexpr int UN = 16 / JN;  // slices whose columns are in flight together
+        for (int h = 0; h < NL && n0 + h <= hi; h += UN) {
+            float a[UN * JN], b[UN * JN];
+#pragma unroll
+            for (int e = 0; e < UN * JN; ++e) {
+                a[e] = src[(int64_t)lane_i(ra, h * JN + e) * Wp];
+                b[e] = src[(int64_t)lane_i(rb, h * JN + e) * Wp];
+            }
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int e = 0; e < UN * JN; ++e) {
+                const float fl = lane_f(wl, h * JN + e), fh = lane_f(wh, h * JN + e);
+                acc[e % JN].v[0] = fmaf(fh, b[e], fmaf(fl, a[e], acc[e % JN].v[0]));
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        if ((n0 + NL) % FLAT_SUM == 0) flush();
+    }
+    if (lo > hi || (hi / NL + 1) * NL % FLAT_SUM) flush();
+}
+
+// ---------------------------------------------------------------------------
+// backward: x[n, c, w] from U
+// ---------------------------------------------------------------------------
+// Four neighbouring values of one output row through the epilogue (as emit).
+__device__ __forceinline__ void emit4(float *out, int64_t o, int64_t b, float4 a, const Epilogue &e)
+{
+    float4 *p = reinterpret_cast<float4 *>(out + o);
+    if (e.mode == EP_SET) {
+        *p = a;
+        return;
+    }
+    float4 r = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    if (e.mode != EP_RESIDUAL) r = *p;
+    if (e.mode == EP_ADD) {
+        *p = make_float4(r.x + a.x, r.y + a.y, r.z + a.z, r.w + a.w);
+        return;
+    }
+    const int64_t q = b * e.stride + o;
+    const float4 w = *reinterpret_cast<const float4 *>(e.w + q);
+    if (e.mode == EP_RESIDUAL) {
+        const float4 y = *reinterpret_cast<const float4 *>(e.y + q);
+        r = make_float4(w.x * (y.x - a.x), w.y * (y.y - a.y), w.z * (y.z - a.z), w.w * (y.w - a.w));
+    } else if (e.mode == EP_SCALED_ADD) {
+        r = make_float4(r.x + w.x * a.x, r.y + w.y * a.y, r.z + w.z * a.z, r.w + w.w * a.w);
+    } else {
+        r = make_float4(r.x - w.x * a.x, r.y - w.y * a.y, r.z - w.z * a.z, r.w - w.w * a.w);
+    }
+    *p = r;
+}
+
+// Writes BX neighbouring voxel columns (x0 .., y) of one wave, ZL of w per lane.
+template <int ZL, int BX>
+__device__ __forceinline__ void flat_write(const FlatView &v, int part, int x0, int y, int w, const FlatVec<ZL> (&acc)[BX])
+{
+    if (y >= v.ny) return;
+    const bool quads = (v.nx & 3) == 0 && (((uintptr_t)v.vol | (uintptr_t)v.ep.y | (uintptr_t)v.ep.w) & 15) == 0 &&
+                       ((v.vs | v.ep.stride) & 3) == 0;
+#pragma unroll
+    for (int z = 0; z < ZL; ++z) {
+        if (w + z >= v.W) continue;
+        const int b = (w + z) / v.nz, iz = (w + z) - b * v.nz;
+        const int64_t o = ((int64_t)iz * v.ny + y) * v.nx + x0;
+        Epilogue ep = v.ep;
+        float *out = v.vol + b * v.vs;
+        if (v.partial) {
+            ep.mode = EP_SET;
+            out = v.partial + ((int64_t)b * v.parts + part) * ((int64_t)v.nx * v.ny * v.nz);
+        }
+        if (quads) {
+#pragma unroll
+            for (int c = 0; c < BX; c += 4)
+                if (x0 + c < v.nx)
+                    emit4(out, o + c, b, make_float4(acc[c].v[z], acc[c + 1].v[z], acc[c + 2].v[z], acc[c + 3].v[z]),
+                          ep);
+        } else {
+#pragma unroll
+            for (int c = 0; c < BX; ++c)
+                if (x0 + c < v.nx) emit(out, o + c, b, acc[c].v[z], ep);
+        }
+    }
+}
+
+// Detector column of the ray through the voxel column (x, y); the first one
+// with a weight there; and the weight of the e-th from it on, max(0, 1 - |j -
+// jc| b2), from FP64 positions.
+__device__ __forceinline__ double flat_column(const FlatAngle &A, double x, double y)
+{
+    return A.m == 0 ? fma(A.gc, y, fma(A.gm, x, A.g0)) : fma(A.gc, x, fma(A.gm, y, A.g0));
+}
+
+template <int NC>
+__device__ __forceinline__ double flat_first(const FlatAngle &A, double jc)
+{
+    return fmin(fmax(NC == 2 ? floor(jc) : ceil(jc - fabs(A.gc)), -1e8), 1e8);
+}
+
+__device__ __forceinline__ float flat_weight(const FlatAngle &A, double j0, double jc, int e)
+{
+    return fmaxf(fmaf(-fabsf((float)(j0 - jc) + (float)e), A.b2, 1.0f), 0.0f);
+}
+
+// A block of 8 waves takes a brick of 16 x 8 voxel columns and 64 ZL of w, a
+// wave the 16 columns of one y. Per angle the lines U of the detector columns
+// that meet the brick are staged in LDS (two buffers, one barrier per angle),
+// and every voxel column takes its NC detector columns (|j - jc| < 1 / b2 for
+// b2 = |dq / dj|: two where a detector column is at least a voxel wide, as
+// many as fit otherwise) with their weights, formed by the 64 lanes for four
+// angles at once. A column without weight is taken from a staged line of
+// zeros, so that an infinite or NaN pixel reaches no voxel that its ray does
+// not meet.
+//
+// Bound: vector ALU issue; per (voxel column, angle) NC + 1 readlane, NC
+// addresses and NC ZL fma (bp_wave: about 37 instructions per 64 voxels at
+// pixel pitch 1, where its 16-voxel bricks take two chunks of columns). Two
+// angles per step at ZL = 2 cost a block per CU (registers): 2.4 against 2.2
+// ms at 75 x 441 x 441, 361 angles, 75 x 623 (bp_wave: 6.3); 16 x 16 bricks
+// 3.1. 8 x 128^3, 180 angles, 128 x 192: 0.64 ms with the splat against 3.04.
+template <int ZL, int NC>
+__global__ void __launch_bounds__(64 * FLAT_BY) bp_flat(FlatMulti M)
+{
+    extern __shared__ __align__(16) float flat_lds[];
+    constexpr int CF = 64 * ZL, AL = 4;  // floats per staged column; angles whose weights a wave holds
+    constexpr int SW = 3;  // columns staged by a wave in one pass
+    const int logical = xcd_logical(M.shift);
+    if (logical >= M.begin[M.n]) return;
+    const int inst = owner_of(M.begin, logical);
+    const FlatView &v = M.v[inst];
+    int id = logical - M.begin[inst];
+    const int bx = id % v.bx;
+    id /= v.bx;
+    const int by = id % v.by;
+    id /= v.by;
+    const int w0 = (id % v.chunks) * CF, part = id / v.chunks;
+    const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int x0 = bx * FLAT_BX, y0 = by * FLAT_BY, kn = v.kn, cols = v.cols, Wp = v.Wp;
+    const int ka = part * v.part_len, kb = min(kn, ka + v.part_len);
+    const int w = w0 + lane * ZL;
+    const int SC = v.stage;
+    const FlatAngle *ang = v.ang;
+    FlatVec<ZL> acc[FLAT_BX], next[SW];
+#pragma unroll
+    for (int c = 0; c < FLAT_BX; ++c)
+#pragma unroll
+        for (int z = 0; z < ZL; ++z) acc[c].v[z] = 0.0f;
+    if (wv < 2) {  // the last place of each buffer: a line of zeros
+        FlatVec<ZL> zero;
+#pragma unroll
+        for (int z = 0; z < ZL; ++z) zero.v[z] = 0.0f;
+        flat_store<ZL>(flat_lds + (wv * (SC + 1) + SC) * CF + lane * ZL, zero);
+    }
+    // first staged detector column of angle ka + 64 i + lane
+    int jbv = 0;
+    auto bases = [&](int k) {
+        const FlatAngle &A = ang[min(k + lane, kn - 1)];
+        const double gx = A.m == 0 ? A.gm : A.gc, gy = A.m == 0 ? A.gc : A.gm;
+        const double j = flat_column(A, x0, y0) + fmin(0.0, (FLAT_BX - 1) * gx) + fmin(0.0, (FLAT_BY - 1) * gy);
+        jbv = (int)flat_first<NC>(A, j - 1e-6);
+    };
+    // (lanes past the last w read the line's last values; nothing of theirs is written)
+    const float *src = v.lines + min(w, Wp - ZL);
+    const int64_t line = Wp, line_by = (int64_t)Wp * FLAT_BY;
+    // staged columns of pass e0 (SW columns of every wave) of angle k
+    auto load = [&](int k, int e0) {
+        const int j0 = lane_i(jbv, (k - ka) & 63) + wv + e0 * SW * FLAT_BY;
+        const float *p = src + ((int64_t)k * cols + j0) * line;
+#pragma unroll
+        for (int e = 0; e < SW; ++e) {
+            if ((unsigned)(j0 + e * FLAT_BY) < (unsigned)cols) {
+                next[e] = flat_load<ZL>(p + e * line_by);
+            } else {
+#pragma unroll
+                for (int z = 0; z < ZL; ++z) next[e].v[z] = 0.0f;
+            }
+        }
+    };
+    auto store = [&](float *buf, int e0) {
+#pragma unroll
+        for (int e = 0; e < SW; ++e) {
+            const int s = wv + (e0 * SW + e) * FLAT_BY;
+            if (s < SC) flat_store<ZL>(buf + s * CF, next[e]);
+        }
+    };
+    bases(ka);
+    load(ka, 0);
+    int places = 0;  // lane (angle k % AL, column c): staged places of the voxel's detector columns, 8 bits each
+    float wt[NC];
+#pragma unroll
+    for (int e = 0; e < NC; ++e) wt[e] = 0.0f;
+    for (int k = ka; k < kb; ++k) {
+        const int at = k - ka;
+        if ((at & (AL - 1)) == 0) {
+            const int jb = __shfl(jbv, (at & 63) + lane / FLAT_BX, 64);
+            const FlatAngle &A = ang[min(k + lane / FLAT_BX, kn - 1)];
+            const double jc = flat_column(A, x0 + lane % FLAT_BX, y0 + wv), j0 = flat_first<NC>(A, jc);
+            const int first = min(max((int)j0 - jb, 0), SC - NC);
+            places = 0;
+#pragma unroll
+            for (int e = 0; e < NC; ++e) {
+                wt[e] = flat_weight(A, j0, jc, e);
+                places |= (wt[e] > 0.0f ? first + e : SC) << (8 * e);
+            }
+        }
+        float *buf = flat_lds + (at & 1) * (SC + 1) * CF + lane * ZL;
+        store(buf, 0);
+        for (int e0 = 1; e0 * SW * FLAT_BY < SC; ++e0) {  // (windows wider than one pass)
+            load(k, e0);
+            store(buf, e0);
+        }
+        __syncthreads();
+        if (k + 1 < kb) {
+            if (((at + 1) & 63) == 0) bases(k + 1);
+            load(k + 1, 0);
+        }
+        constexpr int CB = ZL == 4 ? 2 : 4;  // voxel columns whose lines are in flight together
+#pragma unroll
+        for (int c0 = 0; c0 < FLAT_BX; c0 += CB) {
+            FlatVec<ZL> u[CB][NC];
+#pragma unroll
+            for (int c = 0; c < CB; ++c) {
+                const uint32_t at4 = (uint32_t)lane_i(places, (at & (AL - 1)) * FLAT_BX + c0 + c);
+#pragma unroll
+                for (int e = 0; e < NC; ++e) u[c][e] = flat_load<ZL>(buf + ((at4 >> (8 * e)) & 255u) * CF);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int c = 0; c < CB; ++c)
+#pragma unroll
+                for (int e = 0; e < NC; ++e) {
+                    const float f = lane_f(wt[e], (at & (AL - 1)) * FLAT_BX + c0 + c);
+#pragma unroll
+                    for (int z = 0; z < ZL; ++z) acc[c0 + c].v[z] = fmaf(f, u[c][e].v[z], acc[c0 + c].v[z]);
+                }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    }
+    flat_write<ZL, FLAT_BX>(v, part, x0, y0 + wv, w, acc);
+}
+
+// The same without staging, for short lines (64 of w per wave, one per lane):
+// each wave reads the two (or NC) lines of every voxel column from global
+// memory. A line is then 256 bytes or less, its read from L1 takes no longer
+// than the 2 NC + 2 instructions that use it, and no barrier or staging
+// latency is left; the waves of small volumes hide each other's latency only
+// with many loads in flight. Columns without weight read the line of zeros
+// after the last one. 64^3, 96 angles, 64 x 96: 20 us, 16 slices of 256^2, 180
+// angles, 384 columns: 281 us (bp_flat 23 and 334).
+template <int NC>
+__global__ void __launch_bounds__(256) bp_flat_direct(FlatMulti M)
+{
+    constexpr int AL = 4;
+    const int logical = xcd_logical(M.shift);
+    if (logical >= M.begin[M.n]) return;
+    const int inst = owner_of(M.begin, logical);
+    const FlatView &v = M.v[inst];
+    int id = logical - M.begin[inst];
+    const int bx = id % v.bx;
+    id /= v.bx;
+    const int by = id % v.by;
+    id /= v.by;
+    const int w0 = (id % v.chunks) * 64, part = id / v.chunks;
+    const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int x0 = bx * FLAT_BX, y = by * 4 + wv, kn = v.kn, cols = v.cols, Wp = v.Wp;
+    const int ka = part * v.part_len, kb = min(kn, ka + v.part_len);
+    const int w = w0 + lane;
+    const FlatAngle *ang = v.ang;
+    const float *src = v.lines + min(w, Wp - 1);
+    const int zero = kn * cols;
+    FlatVec<1> acc[FLAT_BX];
+#pragma unroll
+    for (int c = 0; c < FLAT_BX; ++c) acc[c].v[0] = 0.0f;
+    for (int k = ka; k < kb; k += AL) {
+        int row[NC];
+        float wt[NC];
+        {
+            const int ke = k + lane / FLAT_BX;
+            const FlatAngle &A = ang[min(ke, kn - 1)];
+            const double jc = flat_column(A, x0 + lane % FLAT_BX, y), j0 = flat_first<NC>(A, jc);
+#pragma unroll
+            for (int e = 0; e < NC; ++e) {
+                const int j = (int)j0 + e;
+                wt[e] = ke < kb && (unsigned)j < (unsigned)cols ? flat_weight(A, j0, jc, e) : 0.0f;
+                row[e] = wt[e] > 0.0f ? ke * cols + j : zero;
+            }
+        }
+#pragma unroll
+        for (int h = 0; h < AL; ++h) {
+            float u[FLAT_BX][NC];
+#pragma unroll
+            for (int c = 0; c < FLAT_BX; ++c)
+#pragma unroll
+                for (int e = 0; e < NC; ++e) u[c][e] = src[(int64_t)lane_i(row[e], h * FLAT_BX + c) * Wp];
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int c = 0; c < FLAT_BX; ++c)
+#pragma unroll
+                for (int e = 0; e < NC; ++e)
+                    acc[c].v[0] = fmaf(lane_f(wt[e], h * FLAT_BX + c), u[c][e], acc[c].v[0]);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    }
+    flat_write<1, FLAT_BX>(v, part, x0, y, w, acc);
+}
+
+// The sums of the angle parts added in order and written through the
+// epilogue: grid (voxels / 256 of the largest instance, entries, instances).
+__global__ void __launch_bounds__(256) flat_parts_reduce(FlatMulti M)
+{
+    const FlatView &v = M.v[blockIdx.z];
+    const int64_t ve = (int64_t)v.nx * v.ny * v.nz, o = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    const int b = blockIdx.y;
+    if (!v.partial || o >= ve || b >= v.W / v.nz) return;
+    const float *pp = v.partial + (int64_t)b * v.parts * ve + o;
+    float t = pp[0];
+    for (int s = 1; s < v.parts; ++s) t += pp[(int64_t)s * ve];
+    emit(v.vol + b * v.vs, o, b, t, v.ep);
+}
+
+using FlatKernel = void (*)(FlatMulti);
+
+inline FlatKernel fp_flat_kernel(int zl, bool wide)
+{
+    if (zl == 4) return wide ? fp_flat<4, FLAT_WIDE / FLAT_FW> : fp_flat<4, FLAT_NARROW / FLAT_FW>;
+    return wide ? fp_flat<2, FLAT_WIDE / FLAT_FW> : fp_flat<2, FLAT_NARROW / FLAT_FW>;
+}
+
+inline FlatKernel bp_flat_kernel(int zl, int nc)
+{
+    if (zl == 4) return nc == 2 ? bp_flat<4, 2> : (nc == 3 ? bp_flat<4, 3> : bp_flat<4, 4>);
+    return nc == 2 ? bp_flat<2, 2> : (nc == 3 ? bp_flat<2, 3> : bp_flat<2, 4>);
+}
+
+inline FlatKernel bp_flat_direct_kernel(int nc)
+{
+    return nc == 2 ? bp_flat_direct<2> : (nc == 3 ? bp_flat_direct<3> : bp_flat_direct<4>);
+}
+
+}  // namespace tsx

@@ -29,6 +29,7 @@
 #include "tsx_plan.h"
 #include "fp_kernels.h"
 #include "bp_kernels.h"
+#include "flat_kernels.h"
 #include "fdk_kernels.h"
 
 using tsx::AngleParams;
@@ -197,6 +198,17 @@ struct tsx_plan {
     // kernel variants chosen by tsx_plan_autotune (-1: library default)
     int32_t fp_variant = -1, bp_bz = -1, fp_by = -1;
     // FDK (cone plans): per-angle quantities and the volume window
+    // flat parallel-beam kernels (fp_flat, bp_flat): the angles ordered by
+    // stepping axis (empty: the plan is not flat), and the columns they stage
+    std::vector<FlatAngle> flat_host;
+    FlatAngle *flat_dev = nullptr;
+    // forward: first angles of the groups of at most flat_ag angles that share
+    // a block, ended by the angle count; voxel columns staged per slice
+    std::vector<int32_t> flat_groups;
+    int32_t *flat_groups_dev = nullptr;
+    int32_t flat_ag = 0, flat_stage_fp = 0;
+    int32_t flat_nc = 0;                // backward: detector columns per voxel column
+    int32_t flat_stage_bp = 0;          // detector columns staged per angle
     std::vector<FdkAngle> fdk_host;
     FdkAngle *fdk_dev = nullptr;
     bool fdk_upright = false;  // every angle: v parallel to z, normal perpendicular to z
@@ -375,6 +387,103 @@ std::vector<AngleParams> device_angle_table(const std::vector<AngleParams> &host
     return t;
 }
 
+// The flat tables of a parallel-beam plan: every ray within a slice of
+// constant z (a drift of less than 1e-9 voxel over the volume counts as
+// none), detector v parallel to z, stepping along x or y.
+void build_flat(tsx_plan *p)
+{
+    p->flat_host.clear();
+    if (p->kind != TSX_PARALLEL3D_VEC || p->ss != 1) return;
+    std::vector<FlatAngle> t;
+    double h_max = 0.0;
+    for (int axis = 0; axis < 2; ++axis) {
+        for (int a = 0; a < p->n_angles; ++a) {
+            const AngleParams &A = p->host[a];
+            if (A.m == 2) return;
+            if (A.m != axis) continue;
+            const double vn = std::fabs(A.V[1]);
+            if (!(vn > 0.0) || std::fabs(A.V[0]) > 1e-12 * vn || std::fabs(A.V[2]) > 1e-12 * vn) return;
+            if (std::fabs(A.S[1]) * (p->nx + p->ny) > 1e-9 * std::fabs(A.S[0])) return;
+            const double r2 = A.S[2] / A.S[0];
+            FlatAngle f;
+            f.q0 = A.P0[2] - A.P0[0] * r2;
+            f.qm = r2;
+            f.qj = A.U[2] - A.U[0] * r2;
+            if (!(std::fabs(f.qj) > 1e-6)) return;
+            f.g0 = -f.q0 / f.qj;
+            f.gm = -f.qm / f.qj;
+            f.gc = 1.0 / f.qj;
+            f.t0 = A.P0[1];
+            f.tj = A.U[1];
+            f.tv = A.V[1];
+            f.b2 = (float)std::fabs(f.qj);
+            f.len = (float)std::sqrt(A.h[0] * A.h[0] + A.h[2] * A.h[2] * r2 * r2);
+            f.m = axis;
+            f.a = a;
+            h_max = std::max(h_max, 1.0 / std::fabs(f.qj));
+            t.push_back(f);
+        }
+    }
+    // detector columns with a weight in a voxel column: |j - jc| < 1 / b2
+    p->flat_nc = (int32_t)std::ceil(std::min(1e6, 2.0 * h_max - 1e-9));
+    if (p->flat_nc < 2) p->flat_nc = 2;
+    // Forward groups: consecutive angles of one axis whose rays meet at most
+    // `limit` voxel columns per slice together (the window of a tile of
+    // columns is widest at the ends of the slices and of the tiles: its lines
+    // are affine in both). Four angles per group where that needs clearly
+    // fewer groups than two, on tiles of 16 instead of 32 columns.
+    const auto window = [&](size_t k0, size_t k1, int jt) {
+        double wide = 0.0;
+        const int nm = t[k0].m == 0 ? p->nx : p->ny;
+        for (double n : {0.0, (double)(nm - 1)})
+            for (double j0 : {0.0, (double)((p->cols - 1) / jt * jt)}) {
+                double lo = 1e300, hi = -1e300;
+                for (size_t k = k0; k < k1; ++k)
+                    for (double j : {j0, std::min(j0 + jt, (double)p->cols) - 1}) {
+                        const double q = t[k].q0 + t[k].qm * n + t[k].qj * j;
+                        lo = std::min(lo, q);
+                        hi = std::max(hi, q);
+                    }
+                wide = std::max(wide, hi - lo);
+            }
+        return (int32_t)std::min(1e6, std::floor(wide + 0.01) + 4.0);
+    };
+    // (No grouping, where a tile of one angle already meets more: the kernels
+    // without staging take those plans, flat_stage_fp = 0.)
+    p->flat_groups.clear();
+    for (int k = 0; k <= (int)t.size(); ++k) p->flat_groups.push_back(k);
+    p->flat_ag = 2;
+    p->flat_stage_fp = 0;
+    for (int ag : {4, 2}) {
+        const int jt = FLAT_FW / ag * FLAT_JW;
+        int32_t most = FLAT_NARROW, stage = 0;
+        for (size_t k = 0; k < t.size(); ++k) most = std::max(most, window(k, k + 1, jt));
+        if (most > FLAT_WIDE) continue;
+        if (ag == 2) most = FLAT_WIDE;
+        std::vector<int32_t> groups;
+        for (size_t k0 = 0; k0 < t.size();) {
+            size_t k1 = k0 + 1;
+            while (k1 < t.size() && (int)(k1 - k0) < ag && t[k1].m == t[k0].m && window(k0, k1 + 1, jt) <= most) ++k1;
+            stage = std::max(stage, window(k0, k1, jt));
+            groups.push_back((int32_t)k0);
+            k0 = k1;
+        }
+        if (p->flat_stage_fp && groups.size() * 10 > (p->flat_groups.size() - 1) * 14) continue;
+        groups.push_back((int32_t)t.size());
+        p->flat_groups = std::move(groups);
+        p->flat_ag = ag;
+        p->flat_stage_fp = stage;
+    }
+    // detector columns that a brick meets
+    double brick = 0.0;
+    for (const FlatAngle &f : t) {
+        const double gx = std::fabs(f.m == 0 ? f.gm : f.gc), gy = std::fabs(f.m == 0 ? f.gc : f.gm);
+        brick = std::max(brick, (FLAT_BX - 1) * gx + (FLAT_BY - 1) * gy);
+    }
+    p->flat_stage_bp = (int32_t)std::min(1e6, std::floor(brick + 0.01) + 2.0 + p->flat_nc);
+    p->flat_host = std::move(t);
+}
+
 int build_angles(const tsx_geometry *g, tsx_plan *p)
 {
     const int64_t n3[3] = {g->grid_col_count, g->grid_row_count, g->grid_slice_count};
@@ -517,6 +626,7 @@ int build_angles(const tsx_geometry *g, tsx_plan *p)
         p->vh[c] = h[c];
     }
     if (cone) build_fdk(g, p);
+    build_flat(p);
     // padded layouts of the forward projector
     const int64_t P2 = 2 * PAD;
     p->layout_elems[0] = (n3[2] + P2) * n3[0] * (n3[1] + P2);
@@ -864,6 +974,132 @@ bool fp_refined(const tsx_plan *p)
            refined_sino(p) * 4 <= REFINED_FP_MAX_BYTES;
 }
 
+// ---------------------------------------------------------------------------
+// flat parallel-beam kernels: choice and sizes
+// ---------------------------------------------------------------------------
+// How a flat plan's projection of `batch` entries runs (ok: whether it does;
+// the variables that force a kernel of the general geometries keep it off).
+// The choice only cuts the work into blocks: no result depends on it.
+struct FlatPlan {
+    bool ok = false;
+    int zl = 1;      // consecutive w per lane
+    bool direct = false;  // short lines: the kernels without staging
+    bool wide = false;    // forward: the kernel of wide windows
+    int stage = 0;   // columns staged at a time
+    int chunks = 1;  // chunks of 64 zl of w
+    int per_launch = 0;  // angles per launch
+    size_t lds = 0;
+};
+
+int64_t flat_pitch(const tsx_plan *p, int64_t batch) { return (p->nz * batch + 3) / 4 * 4; }
+
+// Lanes: the fewest w per lane that cover W in one chunk, at most 4 (W = 64:
+// 1, on the kernels without staging; 128: 2). Fewer w per lane than that cost
+// more instructions per w: 8 x 128^3 (W = 1024) forward 0.80, 0.88 and 1.32 ms
+// with 4, 2 and 1.
+int flat_zl(int64_t W) { return W > 128 ? 4 : (W > 64 ? 2 : 1); }
+
+// The turned volume and its line of zeros.
+int64_t flat_turned_elems(const tsx_plan *p, int64_t batch)
+{
+    return ((int64_t)p->nx * p->ny + 1) * flat_pitch(p, batch);
+}
+
+// Workspace floats of the forward projector. The flat kernels' turned volume
+// and sums G live in that of the padded layouts (which is two to four times
+// the volume), G for as many angles at a time as it holds; it is grown where
+// that would be fewer than 64 (detectors far wider than the volume), unless
+// that took the plan past the static buffer of tsx_direct_fpbp3d_noalloc: it
+// then stays on the padded kernels.
+bool flat_fp_ok(const tsx_plan *p)
+{
+    if (p->flat_host.empty() || force_general() || env_int("TSX_FP_VARIANT") >= 2 || !p->fp_padded) return false;
+    const int64_t need = flat_turned_elems(p, 1) + (int64_t)p->cols * flat_pitch(p, 1) * std::min(p->n_angles, 64);
+    return need * 4 <= TSX_NOALLOC_SCRATCH_BYTES || fp_workspace_elems(p) * 4 > TSX_NOALLOC_SCRATCH_BYTES ||
+           need <= fp_workspace_elems(p);
+}
+
+int64_t fp_elems(const tsx_plan *p, int64_t batch)
+{
+    const int64_t padded = fp_workspace_elems(p) * batch;
+    if (!flat_fp_ok(p)) return padded;
+    return std::max(padded, flat_turned_elems(p, batch) +
+                                (int64_t)p->cols * flat_pitch(p, batch) * std::min(p->n_angles, 64));
+}
+
+FlatPlan flat_fp(const tsx_plan *p, int64_t batch)
+{
+    FlatPlan f;
+    const int64_t W = p->nz * batch, Wp = flat_pitch(p, batch);
+    if (!flat_fp_ok(p) || W > (1 << 28)) return f;
+    f.per_launch = (int)std::min<int64_t>(
+        p->n_angles, (fp_elems(p, batch) - flat_turned_elems(p, batch)) / ((int64_t)p->cols * Wp));
+    f.stage = p->flat_stage_fp;
+    f.wide = f.stage > FLAT_NARROW;
+    f.zl = f.stage ? flat_zl(W) : 1;
+    f.direct = f.zl == 1;
+    f.lds = f.direct ? 0 : (size_t)2 * f.stage * f.zl * 256;
+    f.ok = true;
+    f.chunks = (int)((W + 64 * f.zl - 1) / (64 * std::max(f.zl, 1)));
+    return f;
+}
+
+// The backprojector's lines U take the workspace of the transposed
+// projections (grown where the volume is higher than the detector).
+// Where that growth would take a plan past the static buffer of
+// tsx_direct_fpbp3d_noalloc, the plan keeps the separable kernel and the buffer.
+bool flat_bp_ok(const tsx_plan *p)
+{
+    if (p->flat_host.empty() || !p->bp_separable || force_general() || env_int("TSX_BP_BRICK_Z") >= 0 ||
+        p->flat_nc > 4 || p->flat_stage_bp > FLAT_BSC)
+        return false;
+    const int64_t sums = bp_parts_of(p) > 1 ? (int64_t)bp_parts_of(p) * p->nx * p->ny * p->nz * 4 + 256 : 0;
+    const int64_t lines = ((int64_t)bp_chunk_of(p) * p->cols + 1) * flat_pitch(p, 1) * 4;
+    return lines + sums <= TSX_NOALLOC_SCRATCH_BYTES || bp_workspace_elems(p) * 4 + sums > TSX_NOALLOC_SCRATCH_BYTES;
+}
+
+int64_t flat_line_elems(const tsx_plan *p, int64_t batch)
+{
+    return flat_bp_ok(p) ? ((int64_t)bp_chunk_of(p) * p->cols + 1) * flat_pitch(p, batch) : 0;
+}
+
+// Blocks of the backprojector (by: voxel columns per block along y).
+int64_t flat_blocks(const tsx_plan *p, int by, int chunks)
+{
+    return (int64_t)((p->nx + FLAT_BX - 1) / FLAT_BX) * ((p->ny + by - 1) / by) * chunks;
+}
+
+FlatPlan flat_bp(const tsx_plan *p, int64_t batch)
+{
+    FlatPlan f;
+    const int64_t W = p->nz * batch;
+    if (!flat_bp_ok(p) || W > (1 << 28)) return f;
+    f.zl = flat_zl(W);
+    f.direct = f.zl == 1;
+    f.chunks = (int)((W + 64 * f.zl - 1) / (64 * f.zl));
+    f.stage = p->flat_stage_bp;
+    f.lds = f.direct ? 0 : (size_t)2 * (f.stage + 1) * f.zl * 256;
+    f.per_launch = bp_chunk_of(p);
+    f.ok = true;
+    return f;
+}
+
+// Angle parts of the flat backprojector, for the plans that bp_part_len_of
+// cuts into parts (never more of them: they use its workspace): two halves,
+// which round less than one running sum (180 angles: 1.7e-7 of the result
+// against 2.7e-7; the separable kernel's four parts 1.9e-7), or parts of at
+// least 4 angles, about 256 blocks of 8 waves per launch of one entry, where
+// the bricks alone give fewer than 128.
+int flat_part_len(const tsx_plan *p)
+{
+    const int cut = bp_part_len_of(p);
+    if (cut == p->n_angles) return cut;
+    const int zl = flat_zl(p->nz);
+    const int64_t blocks = std::min<int64_t>(128, flat_blocks(p, 8, (p->nz + 64 * zl - 1) / (64 * zl)));
+    const int64_t len = std::max<int64_t>(4, ((int64_t)p->n_angles * blocks + 255) / 256);
+    return (int)std::min<int64_t>(std::max<int64_t>(len, cut), p->n_angles);
+}
+
 int64_t workspace_bytes(const tsx_plan *p, int op, int64_t batch)
 {
     if (force_general()) return 0;
@@ -873,14 +1109,14 @@ int64_t workspace_bytes(const tsx_plan *p, int op, int64_t batch)
     // the refined detector's projections, then that plan's workspace
     if (op == TSX_OP_FP && fp_refined(p))
         return align_ws(refined_sino(p) * batch * 4) + workspace_bytes(p->fine, op, batch);
-    if (op == TSX_OP_FP) return p->fp_padded ? fp_workspace_elems(p) * batch * 4 : 0;
+    if (op == TSX_OP_FP) return p->fp_padded ? fp_elems(p, batch) * 4 : 0;
     if (op == TSX_OP_BP && bp_refined(p)) return workspace_bytes(p->fine, op, batch);
     if (p->perm)
         return align_ws((int64_t)p->nx * p->ny * p->nz * batch * 4) + workspace_bytes(p->perm, op, batch);
     if (p->bp_separable) {
         // transposed projections, then the sums of the angle parts
         const int parts = bp_parts_of(p);
-        const int64_t t = bp_workspace_elems(p) * batch * 4;
+        const int64_t t = std::max(bp_workspace_elems(p) * batch, flat_line_elems(p, batch)) * 4;
         return parts > 1 ? align_ws(t) + (int64_t)parts * p->nx * p->ny * p->nz * batch * 4 : t;
     }
     return bp_general_prescaled(p, batch) ? bp_workspace_elems(p) * batch * 4 : 0;
@@ -1231,6 +1467,195 @@ int launch_unswap(const float *src, int64_t ss, float *out, int64_t os, int nx, 
     return TSX_OK;
 }
 
+// ---------------------------------------------------------------------------
+// flat parallel-beam kernels: launches
+// ---------------------------------------------------------------------------
+FlatView flat_view(const tsx_plan *p, const FlatPlan &f, int64_t batch, int k0, int kn, Epilogue ep)
+{
+    FlatView v = {};
+    v.ang = p->flat_dev + k0;
+    v.kn = kn;
+    v.n_angles = p->n_angles;
+    v.rows = p->rows;
+    v.cols = p->cols;
+    v.nx = p->nx;
+    v.ny = p->ny;
+    v.nz = p->nz;
+    v.W = (int)(p->nz * batch);
+    v.Wp = (int)flat_pitch(p, batch);
+    v.ep = ep;
+    v.up = 1;
+    v.stage = f.stage;
+    v.chunks = f.chunks;
+    v.parts = 1;
+    v.part_len = kn;
+    return v;
+}
+
+// The instances of one flat launch and the block counts of its passes.
+struct FlatBatch {
+    FlatMulti m = {};
+    size_t lds = 0;
+    hipStream_t stream;
+    explicit FlatBatch(hipStream_t s) : stream(s) {}
+    // begin[] from each instance's block count; -1 where they exceed a launch
+    template <typename F>
+    int64_t lay(F &&blocks, int threads)
+    {
+        int64_t n = 0;
+        for (int k = 0; k < m.n; ++k) {
+            m.begin[k] = (int)n;
+            n += blocks(m.v[k]);
+            if (n > max_blocks(threads)) return -1;
+        }
+        m.begin[m.n] = (int)n;
+        pad_begin(m.begin, m.n);
+        return n;
+    }
+    template <typename K, typename F>
+    int pass(K kernel, F &&blocks)
+    {
+        const int64_t n = lay(blocks, 256);
+        if (n < 0) return fail(TSX_ERR_UNSUPPORTED, "flat kernels: too many blocks for one launch");
+        if (n > 0) hipLaunchKernelGGL(kernel, dim3((unsigned)n), dim3(32, 8), 0, stream, m);
+        TSX_HIP_CHECK(hipGetLastError());
+        return TSX_OK;
+    }
+    template <typename F>
+    int main_pass(FlatKernel kernel, int waves, F &&blocks)
+    {
+        const int64_t n = lay(blocks, 64 * waves);
+        if (n < 0) return fail(TSX_ERR_UNSUPPORTED, "flat kernels: too many blocks for one launch");
+        const unsigned grid = xcd_grid(n, &m.shift);
+        if (lds > 64 * 1024)
+            TSX_HIP_CHECK(hipFuncSetAttribute((const void *)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+        hipLaunchKernelGGL(kernel, dim3(grid), dim3(64 * waves), lds, stream, m);
+        TSX_HIP_CHECK(hipGetLastError());
+        return TSX_OK;
+    }
+    int forward(const FlatPlan &f, bool turn)
+    {
+        int rc = turn ? pass(flat_turn, flat_turn_blocks) : TSX_OK;
+        if (rc) return rc;
+        if (f.direct)
+            rc = main_pass(fp_flat_direct, 4, [](const FlatView &v) {
+                return (int64_t)v.kn * ((v.cols + 4 * FLAT_DJ - 1) / (4 * FLAT_DJ)) * v.chunks;
+            });
+        else
+            rc = main_pass(fp_flat_kernel(f.zl, f.wide), FLAT_FW,
+                           [](const FlatView &v) { return (int64_t)v.groups * v.tiles * v.chunks; });
+        return rc ? rc : pass(flat_rows, flat_rows_blocks);
+    }
+    int backward(const FlatPlan &f, int nc)
+    {
+        int rc = pass(flat_splat, flat_splat_blocks);
+        if (rc) return rc;
+        int64_t ve = 0;
+        int entries = 0;
+        bool sums = false;
+        const int by = f.direct ? 4 : FLAT_BY;
+        for (int k = 0; k < m.n; ++k) {
+            FlatView &v = m.v[k];
+            v.bx = (v.nx + FLAT_BX - 1) / FLAT_BX;
+            v.by = (v.ny + by - 1) / by;
+            sums = sums || v.partial;
+            ve = std::max(ve, (int64_t)v.nx * v.ny * v.nz);
+            entries = std::max(entries, v.W / v.nz);
+        }
+        rc = main_pass(f.direct ? bp_flat_direct_kernel(nc) : bp_flat_kernel(f.zl, nc), by,
+                       [](const FlatView &v) { return (int64_t)v.bx * v.by * v.chunks * v.parts; });
+        if (rc || !sums) return rc;
+        hipLaunchKernelGGL(flat_parts_reduce, dim3((unsigned)((ve + 255) / 256), (unsigned)entries, (unsigned)m.n),
+                           dim3(256), 0, stream, m);
+        TSX_HIP_CHECK(hipGetLastError());
+        return TSX_OK;
+    }
+};
+
+// The forward groups g0 .. g1 - 1 of a plan in a view (whose angles are theirs).
+void flat_groups(const tsx_plan *p, int g0, int g1, FlatView &v)
+{
+    const int jt = FLAT_FW / p->flat_ag * FLAT_JW;
+    v.group = p->flat_groups_dev + g0;
+    v.groups = g1 - g0;
+    v.ag = p->flat_ag;
+    v.k0 = p->flat_groups[g0];
+    v.tiles = (p->cols + jt - 1) / jt;
+}
+
+// Batch entries of one flat launch: w stays far below 2^28, the blocks below
+// the dispatch limit.
+int64_t flat_entries(const tsx_plan *p)
+{
+    const int64_t per = std::max<int64_t>(p->nz, p->rows);
+    return std::max<int64_t>(1, std::min<int64_t>(65535, ((int64_t)1 << 16) / per));
+}
+
+int launch_fp_flat(const tsx_plan *p, const float *vol, int64_t vs, float *proj, int64_t ps, int64_t batch,
+                   Epilogue ep, float *base, hipStream_t stream)
+{
+    const int64_t bc = flat_entries(p);
+    for (int64_t b0 = 0; b0 < batch; b0 += bc) {
+        const int64_t nb = std::min(bc, batch - b0);
+        const FlatPlan f = flat_fp(p, nb);
+        const int ng = (int)p->flat_groups.size() - 1;
+        for (int g0 = 0, g1; g0 < ng; g0 = g1) {
+            const int k0 = p->flat_groups[g0];
+            for (g1 = g0 + 1; g1 < ng && p->flat_groups[g1 + 1] - k0 <= f.per_launch;) ++g1;
+            FlatBatch fb(stream);
+            FlatView v = flat_view(p, f, nb, k0, p->flat_groups[g1] - k0, ep_from(ep, b0));
+            flat_groups(p, g0, g1, v);
+            v.vol = const_cast<float *>(vol) + b0 * vs;
+            v.vs = vs;
+            v.proj = proj + b0 * ps;
+            v.ps = ps;
+            v.turned = base;
+            v.lines = base + flat_turned_elems(p, nb);
+            fb.m.v[0] = v;
+            fb.m.n = 1;
+            fb.lds = f.lds;
+            const int rc = fb.forward(f, g0 == 0);
+            if (rc) return rc;
+        }
+    }
+    return TSX_OK;
+}
+
+// up: pixels of this plan per pixel edge of the caller's detector; `partial`:
+// room for the sums of bp_parts_of(p) angle parts of every entry (null: one part).
+int launch_bp_flat(const tsx_plan *p, float *vol, int64_t vs, const float *proj, int64_t ps, int64_t batch,
+                   Epilogue ep, float *lines, float *partial, int up, hipStream_t stream)
+{
+    const int64_t bc = flat_entries(p);
+    const int len = partial ? flat_part_len(p) : p->n_angles;
+    for (int64_t b0 = 0; b0 < batch; b0 += bc) {
+        const int64_t nb = std::min(bc, batch - b0);
+        const FlatPlan f = flat_bp(p, nb);
+        for (int k0 = 0; k0 < p->n_angles; k0 += f.per_launch) {
+            FlatBatch fb(stream);
+            FlatView v = flat_view(p, f, nb, k0, std::min(f.per_launch, p->n_angles - k0),
+                                   ep_from(k0 == 0 ? ep : later_chunk(ep), b0));
+            v.vol = vol + b0 * vs;
+            v.vs = vs;
+            v.proj = const_cast<float *>(proj) + b0 * ps;
+            v.ps = ps;
+            v.up = up;
+            v.lines = lines;
+            if (len < p->n_angles) {
+                v.part_len = len;
+                v.parts = (p->n_angles + len - 1) / len;
+                v.partial = partial;
+            }
+            fb.m.v[0] = v;
+            fb.m.n = 1;
+            fb.lds = f.lds;
+            const int rc = fb.backward(f, p->flat_nc);
+            if (rc) return rc;
+        }
+    }
+    return TSX_OK;
+}
+
 // Forward projection of `batch` volumes: the padded kernels on the whole
 // volume or slab by slab (each slab's sums added to the projections of the
 // previous ones), else the general kernel.
@@ -1285,8 +1710,10 @@ int launch_fp(const tsx_plan *p, const float *vol, int64_t vs, float *proj, int6
     const int variant = fp_variant_of(p), by = fp_tile_rows_of(p);
     Scratch owned;
     void *wptr = nullptr;
-    int rc = get_workspace(p, fp_workspace_elems(p) * batch * 4, wsp, ws_bytes, stream, owned, &wptr);
+    int rc = get_workspace(p, fp_elems(p, batch) * 4, wsp, ws_bytes, stream, owned, &wptr);
     if (rc) return rc;
+    if (flat_fp(p, 1).ok && flat_fp(p, std::min(batch, flat_entries(p))).ok)
+        return launch_fp_flat(p, vol, vs, proj, ps, batch, ep, (float *)wptr, stream);
     const bool shear = fp_shear_on(p);  // (slabs: each with its own row offset bound)
     if (p->slabs.empty())
         return launch_fp_padded(p, variant, by, shear, vol, vs, proj, ps, batch, ep, (float *)wptr, stream);
@@ -1406,7 +1833,9 @@ int launch_bp(const tsx_plan *p, float *vol, int64_t vs, const float *proj, int6
     int rc = get_workspace(p, workspace_bytes(p, TSX_OP_BP, batch), wsp, ws_bytes, stream, owned, &wptr);
     if (rc) return rc;
     float *ly = (float *)wptr;
-    float *partial = parts > 1 ? (float *)((char *)wptr + align_ws(sino_t * batch * 4)) : nullptr;
+    const int64_t ly_elems = std::max(sino_t * batch, flat_line_elems(p, batch));
+    float *partial = parts > 1 ? (float *)((char *)wptr + align_ws(ly_elems * 4)) : nullptr;
+    if (flat_bp(p, 1).ok) return launch_bp_flat(p, vol, vs, proj, ps, batch, ep, ly, partial, up, stream);
     const int BZ = bp_brick_z_of(p);
     const int64_t bricks = (int64_t)((p->nx + BR - 1) / BR) * ((p->ny + BR - 1) / BR) * ((p->nz + BZ - 1) / BZ);
     if (bricks * parts > max_blocks(BR * BR)) return fail(TSX_ERR_UNSUPPORTED, "volume too large for one launch");
@@ -1473,6 +1902,20 @@ int check_multi(const tsx_plan *const *plans, int n)
     return TSX_OK;
 }
 
+// Whether an instance of a fused call is flat and its angles fit one launch
+// (with the block counts of every pass far below the dispatch limit).
+bool flat_one_launch(const tsx_plan *p, int op)
+{
+    const FlatPlan f = op == TSX_OP_FP ? flat_fp(p, 1) : flat_bp(p, 1);
+    const int64_t tiles = (int64_t)((p->cols + 31) / 32) * ((std::max(p->rows, p->nz) + 31) / 32) * p->n_angles;
+    const int64_t turn = (int64_t)((p->nx + 31) / 32) * ((p->nz + 31) / 32) * p->ny;
+    const int64_t most = max_blocks(1024) / FLAT_MAX;
+    if (op == TSX_OP_FP && (fp_refined(p) || fp_swapped(p))) return false;
+    if (op == TSX_OP_BP && (bp_refined(p) || p->perm)) return false;
+    return f.ok && f.per_launch >= p->n_angles && std::max(tiles, turn) <= most &&
+           flat_blocks(p, 4, f.chunks) * bp_parts_of(p) <= most;
+}
+
 // Scratch of a fused launch: each instance's workspace.
 int64_t multi_workspace_bytes(const tsx_plan *const *plans, int n, int op)
 {
@@ -1527,8 +1970,32 @@ int multi_fp(const tsx_plan *const *plans, const float *const *vols, float *cons
         const std::pair<int, int> key(fp_variant_of(plans[k]), fp_tile_rows_of(plans[k]));
         if (std::find(keys.begin(), keys.end(), key) == keys.end()) keys.push_back(key);
     }
+    // flat parallel-beam instances, by their choice of kernel
+    std::vector<char> taken(n, 0);
+    for (int k = 0; k < n && fast; ++k) {
+        if (taken[k] || !flat_one_launch(plans[k], TSX_OP_FP)) continue;
+        const FlatPlan f = flat_fp(plans[k], 1);
+        FlatBatch fb(stream);
+        for (int e = k; e < n && fb.m.n < FLAT_MAX; ++e) {
+            if (taken[e] || !flat_one_launch(plans[e], TSX_OP_FP)) continue;
+            const FlatPlan fe = flat_fp(plans[e], 1);
+            if (fe.zl != f.zl || fe.wide != f.wide) continue;
+            taken[e] = 1;
+            FlatView &v = fb.m.v[fb.m.n++];
+            v = flat_view(plans[e], fe, 1, 0, plans[e]->n_angles, eps[e]);
+            flat_groups(plans[e], 0, (int)plans[e]->flat_groups.size() - 1, v);
+            v.vol = const_cast<float *>(vols[e]);
+            v.proj = projs[e];
+            v.turned = (float *)((char *)wptr + off[e]);
+            v.lines = v.turned + flat_turned_elems(plans[e], 1);
+            fb.lds = std::max(fb.lds, fe.lds);
+        }
+        const int rc = fb.forward(f, true);
+        if (rc) return rc;
+    }
     for (size_t pass = 0; pass < keys.size(); ++pass)
     for (int k = 0; k < n; ++k) {
+        if (taken[k]) continue;
         const tsx_plan *p = plans[k];
         const int64_t wb = off[k + 1] - off[k];
         const int64_t woff = off[k];
@@ -1539,7 +2006,7 @@ int multi_fp(const tsx_plan *const *plans, const float *const *vols, float *cons
         const int64_t blocks = (int64_t)tiles_u * tiles_v * p->n_angles;
         const int64_t cap = max_blocks(FP_BX * pby);
         if (!(fast && p->fp_padded && p->ss == 1 && p->slabs.empty() && !fp_swapped(p) && !p->fp_wide) ||
-            blocks > cap) {
+            blocks > cap || flat_fp(p, 1).ok) {
             // this instance takes its own launch(es), in the first pass
             if (pass > 0) continue;
             int rc = launch_fp(p, vols[k], 0, projs[k], 0, 1, eps[k], stream, wptr ? (char *)wptr + woff : nullptr, wb);
@@ -1635,8 +2102,38 @@ int multi_bp(const tsx_plan *const *plans, float *const *vols, const float *cons
         const std::pair<int, bool> key(bp_brick_z_of(plans[k]), bp_parts_of(plans[k]) > 1);
         if (std::find(keys.begin(), keys.end(), key) == keys.end()) keys.push_back(key);
     }
+    // flat parallel-beam instances, by their choice of kernel
+    std::vector<char> taken(n, 0);
+    for (int k = 0; k < n && fast; ++k) {
+        if (taken[k] || !flat_one_launch(plans[k], TSX_OP_BP)) continue;
+        const FlatPlan f = flat_bp(plans[k], 1);
+        FlatBatch fb(stream);
+        for (int e = k; e < n && fb.m.n < FLAT_MAX; ++e) {
+            if (taken[e] || !flat_one_launch(plans[e], TSX_OP_BP)) continue;
+            const tsx_plan *p = plans[e];
+            const FlatPlan fe = flat_bp(p, 1);
+            if (fe.zl != f.zl || p->flat_nc != plans[k]->flat_nc) continue;
+            taken[e] = 1;
+            FlatView &v = fb.m.v[fb.m.n++];
+            v = flat_view(p, fe, 1, 0, p->n_angles, eps[e]);
+            v.vol = vols[e];
+            v.proj = const_cast<float *>(projs[e]);
+            v.lines = (float *)((char *)wptr + off[e]);
+            const int len = bp_parts_of(p) > 1 ? flat_part_len(p) : p->n_angles;
+            if (len < p->n_angles) {
+                v.part_len = len;
+                v.parts = (p->n_angles + len - 1) / len;
+                v.partial = (float *)((char *)wptr + off[e] +
+                                      align_ws(std::max(bp_workspace_elems(p), flat_line_elems(p, 1)) * 4));
+            }
+            fb.lds = std::max(fb.lds, fe.lds);
+        }
+        const int rc = fb.backward(f, plans[k]->flat_nc);
+        if (rc) return rc;
+    }
     for (size_t pass = 0; pass < keys.size(); ++pass)
     for (int k = 0; k < n; ++k) {
+        if (taken[k]) continue;
         const tsx_plan *p = plans[k];
         const int64_t wb = off[k + 1] - off[k];
         const int64_t woff = off[k];
@@ -1652,7 +2149,7 @@ int multi_bp(const tsx_plan *const *plans, float *const *vols, const float *cons
         const int64_t tblocks = scale_job_blocks(job);
         const int64_t cap = max_blocks(BR * BR);
         if (!(fast && p->bp_separable && bp_chunk_of(p) == p->n_angles) || blocks > cap ||
-            tblocks > max_blocks(256)) {
+            tblocks > max_blocks(256) || flat_bp(p, 1).ok) {
             if (pass > 0) continue;  // (its own launch, in the first pass)
             int rc = launch_bp(p, vols[k], 0, projs[k], 0, 1, eps[k], stream, wptr ? (char *)wptr + woff : nullptr, wb);
             if (rc) return rc;
@@ -1715,7 +2212,7 @@ std::string tune_key(const tsx_plan *p)
            ":" + std::to_string(p->rows) + "x" + std::to_string(p->cols) + ":" + std::to_string(p->nx) +
            "x" + std::to_string(p->ny) + "x" + std::to_string(p->nz) + ":" + std::to_string(p->ss) + ":" +
            std::to_string((int)p->fp_padded) + std::to_string((int)p->fp_pair) +
-           std::to_string((int)p->bp_separable) + ":" +
+           std::to_string((int)p->bp_separable) + (flat_fp(p, 1).ok ? "f" : "") + (flat_bp(p, 1).ok ? "b" : "") + ":" +
            std::to_string(angle_bucket(p->n_angles)) + ":" + std::to_string(p->fp_shear_rows) +
            (p->fp_column_waves ? "c" : "r");
 }
@@ -1780,6 +2277,14 @@ int autotune(tsx_plan *p, hipStream_t stream)
             return TSX_OK;
         }
     }
+    // Flat parallel-beam projections have no variants to choose from
+    const bool fp_flat_used = flat_fp(p, 1).ok, bp_flat_used = flat_bp(p, 1).ok;
+    if (fp_flat_used && bp_flat_used) {
+        p->fp_variant = p->fp_pair ? 4 : 3;
+        p->fp_by = 8;
+        p->bp_bz = 32;
+        return TSX_OK;
+    }
     // Backprojector trials: a sub-plan of at most 64 of the plan's angles, in
     // four runs of 16 consecutive angles (the plan's own angular spacing, so that
     // the cache reuse between neighbouring angles is as in the full launch)
@@ -1841,7 +2346,7 @@ int autotune(tsx_plan *p, hipStream_t stream)
     // (a plan whose forward projection runs on its axis-swapped plan leaves the
     // choice to that plan's own tuning)
     const bool fp_choices =
-        p->fp_padded && p->ss >= 1 && p->ss <= 4 && !force_general() && !fp_swapped(p) && !fp_refined(p);
+        p->fp_padded && p->ss >= 1 && p->ss <= 4 && !force_general() && !fp_swapped(p) && !fp_refined(p) && !fp_flat_used;
     if (fp_choices) {
         // The forward kernel walks all angles of one detector tile before the
         // next tile, so its cache reuse depends on the angle count: the
@@ -1956,7 +2461,7 @@ int autotune(tsx_plan *p, hipStream_t stream)
             best.fp_shear = off_ms * 1.02f < on_ms ? 0 : 1;
         }
     }
-    if (p->bp_separable && !force_general()) {
+    if (p->bp_separable && !force_general() && !bp_flat_used) {
         float best_ms = 1e30f;
         for (int bz : {32, 24, 16}) {
             sub.bp_bz = bz;
@@ -2187,11 +2692,23 @@ int tsx_plan_create(const tsx_geometry *g, int device, tsx_plan **out)
                 return fail(TSX_ERR_OUT_OF_MEMORY, std::string("FDK tables: ") + hipGetErrorString(e));
             }
         }
-        int rc = build_range_table(p, nullptr, &p->bp_rt);
+        int rc = TSX_OK;
+        if (!p->flat_host.empty()) {
+            const size_t fb = sizeof(FlatAngle) * p->flat_host.size();
+            e = hipMalloc((void **)&p->flat_dev, fb);
+            if (e == hipSuccess) e = hipMemcpy(p->flat_dev, p->flat_host.data(), fb, hipMemcpyHostToDevice);
+            const size_t gb = sizeof(int32_t) * p->flat_groups.size();
+            if (e == hipSuccess && gb) e = hipMalloc((void **)&p->flat_groups_dev, gb);
+            if (e == hipSuccess && gb) e = hipMemcpy(p->flat_groups_dev, p->flat_groups.data(), gb, hipMemcpyHostToDevice);
+            if (e != hipSuccess) rc = fail(TSX_ERR_OUT_OF_MEMORY, std::string("flat tables: ") + hipGetErrorString(e));
+        }
+        if (rc == TSX_OK) rc = build_range_table(p, nullptr, &p->bp_rt);
         if (rc == TSX_OK && hipStreamSynchronize(nullptr) != hipSuccess)
             rc = fail(TSX_ERR_HIP, "slice-range table: synchronisation failed");
         if (rc) {
             if (p->bp_rt) (void)hipFree(p->bp_rt);
+            if (p->flat_dev) (void)hipFree(p->flat_dev);
+            if (p->flat_groups_dev) (void)hipFree(p->flat_groups_dev);
             if (p->fdk_dev) (void)hipFree(p->fdk_dev);
             (void)hipFree(p->dev);
             delete p;
@@ -2255,6 +2772,8 @@ int tsx_plan_destroy(tsx_plan *p)
         DeviceGuard guard(p->device);
         (void)hipFree(p->dev);
         if (p->fdk_dev) (void)hipFree(p->fdk_dev);
+        if (p->flat_dev) (void)hipFree(p->flat_dev);
+        if (p->flat_groups_dev) (void)hipFree(p->flat_groups_dev);
         if (p->bp_rt) (void)hipFree(p->bp_rt);
     }
     delete p;
@@ -2276,7 +2795,9 @@ int tsx_plan_info_get(const tsx_plan *p, tsx_plan_info *info)
     if (p->fine && tsx_plan_info_get(p->fine, &sub) == TSX_OK) sub_bytes += sub.plan_bytes;
     info->plan_bytes = sub_bytes + (p->dev ? (int64_t)(sizeof(AngleParams) * 2 * p->host.size()) *
                                         (1 + (int64_t)p->slabs.size()) +
-                                    (p->bp_rt ? p->bp_rt_stride * p->n_angles * 4 : 0)
+                                    (p->bp_rt ? p->bp_rt_stride * p->n_angles * 4 : 0) +
+                                    (p->flat_dev ? (int64_t)(sizeof(FlatAngle) * p->flat_host.size() +
+                                                             sizeof(int32_t) * p->flat_groups.size()) : 0)
                               : 0);
     for (int c = 0; c < 3; ++c) info->axis_count[c] = p->axis_count[c];
     // the plan whose forward kernels run

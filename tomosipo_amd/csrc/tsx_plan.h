@@ -44,6 +44,18 @@ struct AngleParams {
     float shear;
 };
 
+// Per-angle quantities of a flat parallel-beam plan (rays within slices of
+// constant z, detector v parallel to z), the angles ordered by stepping axis.
+// In-slice coordinates n (along m) and c (the other horizontal axis).
+struct FlatAngle {
+    double g0, gm, gc;  // detector column of the ray through (n, c): g0 + gm n + gc c
+    double q0, qm, qj;  // position c of column j's ray in slice n: q0 + qm n + qj j
+    double t0, tj, tv;  // height z of pixel (i, j): t0 + tj j + tv i
+    float b2;           // |qj|
+    float len;          // world length per slice step
+    int32_t m, a;       // stepping axis (0 = x, 1 = y), index of the angle in the projections
+};
+
 // Per-angle FDK quantities of a cone-beam plan, world (x, y, z) coordinates.
 // The detector is moved to the parallel plane through the volume centre c
 // (virtual detector: pixel (i, j) centre at s + P0s + j*U + i*V).
