@@ -66,11 +66,9 @@ struct GeneralMath<double> {
     static __device__ __forceinline__ double v(const AngleParams &A, int k) { return A.V[k]; }
 };
 
-// With PRESCALED (detector supersampling 1 only), proj holds the
-// length-weighted projections l(a, i, j) * y[i, a, j] and the per-pixel ray
-// length is not recomputed. CONE: the plan's beam (every angle of a plan is
-// of the same kind), so that each kernel holds only its own set-up.
-template <typename T, bool PRESCALED, bool CONE>
+// CONE: the plan's beam (every angle of a plan is of the same kind), so that
+// each kernel holds only its own set-up.
+template <typename T, bool CONE>
 __global__ void __launch_bounds__(BP_BX *BP_BY)
 bp_general(const AngleParams *__restrict__ angles, int n_angles, int rows, int cols, int ss,
            int nx, int ny, int nz, T *__restrict__ vol, int64_t vol_stride,
@@ -106,10 +104,8 @@ bp_general(const AngleParams *__restrict__ angles, int n_angles, int rows, int c
             A2i = A.par_a[3];
             bj = A.par_b[0];
             bi = A.par_b[1];
-            if constexpr (!PRESCALED) {
-                r1 = (T)(A.S[1] * A.inv_S0);
-                r2 = (T)(A.S[2] * A.inv_S0);
-            }
+            r1 = (T)(A.S[1] * A.inv_S0);
+            r2 = (T)(A.S[2] * A.inv_S0);
         } else {
             T Tc, Bjc = T(0), Bic = T(0);
             if constexpr (CONE) {
@@ -181,27 +177,6 @@ bp_general(const AngleParams *__restrict__ angles, int n_angles, int rows, int c
         }
         if (j0 > j1 || i0 > i1) continue;
         const T dj0 = (T)((double)j0 - cj), di0 = (T)((double)i0 - ci);
-        if constexpr (PRESCALED) {
-            // detector supersampling 1 (the only case with length-weighted
-            // projections): one ray per pixel, through its centre
-            T acc_a = T(0);
-            for (int i = i0; i <= i1; ++i) {
-                const T *row = pr + ((int64_t)i * n_angles + a) * cols;
-                const T di = di0 + (T)(i - i0);
-                const T e = di * fBi + T(1), b1 = di * A1i, b2 = di * A2i;
-                for (int j = j0; j <= j1; ++j) {
-                    const T dj = dj0 + (T)(j - j0);
-                    const T iden = GeneralMath<T>::recip(dj * fBj + e);
-                    const T dq1 = (dj * A1j + b1) * iden;
-                    const T dq2 = (dj * A2j + b2) * iden;
-                    const T w1 = T(1) - fabs(dq1), w2 = T(1) - fabs(dq2);
-                    const T w = (w1 > T(0) ? w1 : T(0)) * (w2 > T(0) ? w2 : T(0));
-                    acc_a += w * row[j];
-                }
-            }
-            acc += acc_a;
-            continue;
-        }
         const T fr1 = r1, fr2 = r2, fg = g;
         const T h0 = (T)(A.h[0] * A.h[0]), h1 = (T)(A.h[1] * A.h[1]), h2 = (T)(A.h[2] * A.h[2]);
         const T len_par = GeneralMath<T>::root(h0 + h1 * fr1 * fr1 + h2 * fr2 * fr2);
@@ -238,7 +213,8 @@ bp_general(const AngleParams *__restrict__ angles, int n_angles, int rows, int c
     emit(vol + (int64_t)b * vol_stride, ((int64_t)z * ny + y) * nx + x, b, acc, ep);
 }
 
-// ly[i, a, j] = l(a, i, j) * y[i, a, j] (detector supersampling 1). Block
+// ly[a, i, j] = l(a, i, j) * y[i, a, j] (detector supersampling 1), an angle's
+// rows together so that bp_tilted addresses them with 32-bit offsets. Block
 // (x, y) takes columns 256 x .. 256 x + 255 of the detector lines y,
 // y + gridDim.y, ... of the `lines` = batch * rows * n_angles lines (line
 // (b, i, a) is b * rows * n_angles + i * n_angles + a).
@@ -270,9 +246,261 @@ __global__ void scale_by_length(const AngleParams *__restrict__ angles, int n_an
         const int64_t ia = line - b * per_entry;
         const int i = (int)(ia / n_angles), a = (int)(ia - (int64_t)i * n_angles);
         const float len = ray_length(angles[a], i, j);
-        const int64_t o = ia * cols + j;
-        out[b * out_stride + o] = len * proj[b * proj_stride + o];
+        out[b * out_stride + ((int64_t)a * rows + i) * cols + j] = len * proj[b * proj_stride + ia * cols + j];
     }
+}
+
+// bp_tilted: the float backprojector of detectors that the separable kernels do
+// not take (tilted or rolled ones, angles stepping along z), detector
+// supersampling 1, from length-weighted projections ly[a][i][j]. One thread
+// per ZV voxels along z. A voxel X maps to the detector position
+//   p(X) = p0 + kappa (W . B) / (W . N),  W = X - S,
+// a ratio of affine functions: formed in FP64 for the first voxel, for the
+// next ones from its differences,
+//   p(X + k e) - p(X) = k lam_k (B_e - N_e (W . B) / (W . N)),  lam_k = kappa / (W_k . N),
+// which are a few pixels and exact in FP32. The derivatives M of the same
+// ratio bound the image of the voxel's +-1 square,
+//   |dj| <= (|M00| + |M01|) / (1 - c),  c = (|N1| + |N2|) / |W . N|,
+// without the inverse of a local map; along the thread's voxels both factors
+// are largest at an end, so that one box size, from the two ends, serves all
+// of them. A pixel's weight takes its ray's in-slice offset, as in bp_general:
+// (dj A1j + di A1i) / (1 + dj fBj + di fBi) along c1, likewise along c2.
+// Angles stepping along z and voxels near the source's planes (W . N under 16
+// times its steps, |W_m| under 16) take the FP64 set-up for each voxel.
+//
+// Bound: vector ALU issue (1.2 per CU-cycle). 192^3 cone, 240 angles, 192 x
+// 288 tilted by 0.2 rad: 4.17 ms (103 instructions per 64 voxels and angle); with the set-up of every voxel in FP64 and
+// a loop over the pixels of each box 7.46 (234).
+struct TiltedVoxel {
+    int j0, i0;     // pixel near the voxel's position
+    float pj, pi;   // position relative to it
+    float tj, ti;   // (W . B) / (W . N)
+    float dn, W0, W1, W2;
+};
+
+// Local map of one voxel and its box of pixels (offsets from j0, i0).
+struct TiltedMap {
+    float pj, pi, A1j, A1i, A2j, A2i, fBj, fBi;
+    int jl, jh, il, ih;
+};
+
+// Weight of a pixel from its ray's in-slice offsets (q1, q2) / den.
+template <bool CONE>
+__device__ __forceinline__ float tilted_weight(float q1, float q2, float den)
+{
+    const float iden = CONE ? fabsf(__builtin_amdgcn_rcpf(den)) : 1.0f;
+    const float w1 = __builtin_amdgcn_fmed3f(fmaf(-fabsf(q1), iden, 1.0f), 0.0f, 1.0f);
+    const float w2 = __builtin_amdgcn_fmed3f(fmaf(-fabsf(q2), iden, 1.0f), 0.0f, 1.0f);
+    return w1 * w2;
+}
+
+// Sum of the pixels of a voxel's box; `o`: byte offset of pixel (j0, i0).
+// Boxes of at most 2 x 2 pixels throughout a wave (nearly all where a pixel is
+// larger than a voxel) take two 8-byte loads and no loop.
+template <bool CONE>
+__device__ __forceinline__ float tilted_sum(__amdgpu_buffer_rsrc_t rs, const TiltedMap &T, uint32_t o, uint32_t pitch)
+{
+    const float djl = (float)T.jl - T.pj;
+    float di = (float)T.il - T.pi;
+    const float a1 = djl * T.A1j, a2 = djl * T.A2j, ad = CONE ? fmaf(djl, T.fBj, 1.0f) : 1.0f;
+    o += (uint32_t)T.il * pitch + (uint32_t)T.jl * 4u;
+    const int nj = T.jh - T.jl, ni = T.ih - T.il;
+    float sum = 0.0f;
+    if (__builtin_amdgcn_ballot_w64(max(nj, ni) > 1) == 0) {
+        const float2 ya = __builtin_bit_cast(float2, __builtin_amdgcn_raw_buffer_load_b64(rs, o, 0, 0));
+        const float2 yb = __builtin_bit_cast(float2, __builtin_amdgcn_raw_buffer_load_b64(rs, o + pitch, 0, 0));
+        const float q1 = fmaf(di, T.A1i, a1), q2 = fmaf(di, T.A2i, a2), den = CONE ? fmaf(di, T.fBi, ad) : 1.0f;
+        const float r1 = q1 + T.A1i, r2 = q2 + T.A2i, rd = den + T.fBi;
+        const float w00 = tilted_weight<CONE>(q1, q2, den);
+        const float w01 = tilted_weight<CONE>(q1 + T.A1j, q2 + T.A2j, den + T.fBj);
+        const float w10 = tilted_weight<CONE>(r1, r2, rd);
+        const float w11 = tilted_weight<CONE>(r1 + T.A1j, r2 + T.A2j, rd + T.fBj);
+        const bool some = min(nj, ni) >= 0, j1 = nj > 0, i1 = ni > 0;
+        sum = w00 * (some ? ya.x : 0.0f);
+        sum = fmaf(w01, some && j1 ? ya.y : 0.0f, sum);
+        sum = fmaf(w10, some && i1 ? yb.x : 0.0f, sum);
+        return fmaf(w11, some && i1 && j1 ? yb.y : 0.0f, sum);
+    }
+    for (int i = 0; i <= ni; ++i) {
+        float q1 = fmaf(di, T.A1i, a1), q2 = fmaf(di, T.A2i, a2), den = CONE ? fmaf(di, T.fBi, ad) : 1.0f;
+        uint32_t oj = o;
+        for (int j = 0; j <= nj; ++j) {
+            sum = fmaf(tilted_weight<CONE>(q1, q2, den), bload(rs, oj), sum);
+            q1 += T.A1j;
+            q2 += T.A2j;
+            den += T.fBj;
+            oj += 4u;
+        }
+        di += 1.0f;
+        o += pitch;
+    }
+    return sum;
+}
+
+template <bool CONE, int ZV>
+__global__ void __launch_bounds__(BP_BX *BP_BY)
+bp_tilted(const AngleParams *__restrict__ angles, int n_angles, int rows, int cols, int nx, int ny, int nz,
+          float *__restrict__ vol, int64_t vol_stride, const float *__restrict__ ly, int64_t ly_stride, Epilogue ep)
+{
+    const int x = blockIdx.x * BP_BX + threadIdx.x;
+    const int y = blockIdx.y * BP_BY + threadIdx.y;
+    const int zb = (nz + ZV - 1) / ZV;
+    const int z0 = (blockIdx.z % zb) * ZV, b = blockIdx.z / zb;
+    typedef const __attribute__((address_space(4))) AngleParams ConstAngle;
+    ConstAngle *table = (ConstAngle *)angles;
+    const float *entry = uniform_ptr(ly + (int64_t)b * ly_stride);
+    const uint32_t bytes = (uint32_t)rows * (uint32_t)cols * 4u, pitch = (uint32_t)cols * 4u;
+    float acc[ZV];
+#pragma unroll
+    for (int k = 0; k < ZV; ++k) acc[k] = 0.0f;
+    for (int a = 0; a < n_angles; ++a) {
+        ConstAngle &A = table[a];
+        const int m = A.m;
+        if (!CONE && !(A.par_b[0] >= 0.0f)) continue;  // singular map
+        const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
+            (void *)(entry + (int64_t)a * rows * cols), (short)0, (int)bytes, 0x00020000);
+        // FP64 set-up of the voxel z; false: no position
+        auto setup = [&](int z, TiltedVoxel &V) {
+            const double km = sel3(m, x, y, z), k1 = sel3(m == 2 ? 1 : 2, x, y, z), k2 = sel3(m == 0 ? 1 : 0, x, y, z);
+            double cj, ci;
+            V.tj = V.ti = V.dn = V.W0 = V.W1 = V.W2 = 0.0f;
+            if constexpr (CONE) {
+                const double W0 = km - A.S[0], W1 = k1 - A.S[1], W2 = k2 - A.S[2];
+                const double dn = W0 * A.N[0] + W1 * A.N[1] + W2 * A.N[2];
+                const double r = rcp64(dn);
+                const double tj = (W0 * A.Bj[0] + W1 * A.Bj[1] + W2 * A.Bj[2]) * r;
+                const double ti = (W0 * A.Bi[0] + W1 * A.Bi[1] + W2 * A.Bi[2]) * r;
+                cj = fma(A.kappa, tj, A.sBj);
+                ci = fma(A.kappa, ti, A.sBi);
+                V.tj = (float)tj;
+                V.ti = (float)ti;
+                V.dn = (float)dn;
+                V.W0 = (float)W0;
+                V.W1 = (float)W1;
+                V.W2 = (float)W2;
+                if (dn == 0.0 || W0 == 0.0) return false;
+            } else {
+                cj = fma(k2, A.par_c[3], fma(k1, A.par_c[2], fma(km, A.par_c[1], A.par_c[0])));
+                ci = fma(k2, A.par_c[7], fma(k1, A.par_c[6], fma(km, A.par_c[5], A.par_c[4])));
+            }
+            const double fj = floor(fmin(fmax(cj, -1e9), 1e9)), fi = floor(fmin(fmax(ci, -1e9), 1e9));
+            V.j0 = (int)fj;
+            V.i0 = (int)fi;
+            V.pj = (float)(cj - fj);
+            V.pi = (float)(ci - fi);
+            return true;
+        };
+        // the box of half-widths (mj, mi) around the position, cut to the detector
+        auto box = [&](const TiltedVoxel &V, float mj, float mi, TiltedMap &T) {
+            T.jl = -min(floor_to_int(mj - T.pj), V.j0);
+            T.jh = min(floor_to_int(T.pj + mj), cols - 1 - V.j0);
+            T.il = -min(floor_to_int(mi - T.pi), V.i0);
+            T.ih = min(floor_to_int(T.pi + mi), rows - 1 - V.i0);
+        };
+        // (offsets of pixels far outside the detector wrap around; their boxes are empty)
+        auto origin = [&](const TiltedVoxel &V) { return (uint32_t)V.i0 * pitch + (uint32_t)V.j0 * 4u; };
+        TiltedVoxel V;
+        const bool ok = setup(z0, V);
+        const bool near = CONE && (!ok || m == 2 || !(fabsf(V.dn) > A.freach) || !(fabsf(V.W0) > 16.0f));
+        TiltedMap T;
+        if (!CONE) {
+            T.A1j = A.par_a[0];
+            T.A1i = A.par_a[1];
+            T.A2j = A.par_a[2];
+            T.A2i = A.par_a[3];
+            T.fBj = T.fBi = 0.0f;
+            const int zc = m == 2 ? 0 : 1;
+            const float gj = A.fBj[zc], gi = A.fBi[zc], mj = A.par_b[0] + 1e-3f, mi = A.par_b[1] + 1e-3f;
+            const uint32_t o = origin(V);
+#pragma unroll
+            for (int k = 0; k < ZV; ++k) {
+                T.pj = fmaf((float)k, gj, V.pj);
+                T.pi = fmaf((float)k, gi, V.pi);
+                box(V, mj, mi, T);
+                acc[k] += tilted_sum<CONE>(rs, T, o, pitch);
+            }
+        } else if (__builtin_amdgcn_ballot_w64(near) == 0) {
+            // (m = 0 or 1: the voxels differ along c1)
+            const float Nz = A.fN[1];
+            const float gj = fmaf(-Nz, V.tj, A.fBj[1]), gi = fmaf(-Nz, V.ti, A.fBi[1]);
+            // box size from the two ends
+            float mj = 0.0f, mi = 0.0f, s = 0.0f;
+#pragma unroll
+            for (int e = 0; e < 2; ++e) {
+                if (e == 1 && ZV == 1) break;
+                const float fk = e ? (float)(ZV - 1) : 0.0f;
+                const float lam = A.fkappa * __builtin_amdgcn_rcpf(fmaf(fk, Nz, V.dn)), kl = fk * lam * A.finv_kappa;
+                const float tj = fmaf(kl, gj, V.tj), ti = fmaf(kl, gi, V.ti);
+                const float M00 = fmaf(-A.fN[1], tj, A.fBj[1]), M01 = fmaf(-A.fN[2], tj, A.fBj[2]);
+                const float M10 = fmaf(-A.fN[1], ti, A.fBi[1]), M11 = fmaf(-A.fN[2], ti, A.fBi[2]);
+                mj = fmaxf(mj, fabsf(M00) + fabsf(M01));
+                mi = fmaxf(mi, fabsf(M10) + fabsf(M11));
+                s = fmaxf(s, fabsf(lam));
+            }
+            s *= fmaf(1.1f * A.fspan, s, 1.0f);  // 1 / (1 - c) <= 1 + 1.1 c for c <= 1 / 16
+            mj = fmaf(mj, s, 1e-3f);
+            mi = fmaf(mi, s, 1e-3f);
+            const float iW0 = __builtin_amdgcn_rcpf(V.W0), r1 = V.W1 * iW0, r2 = V.W2 * iW0;
+            const float uj = A.fU[0] * iW0, ui = A.fV[0] * iW0;
+            const float c1j = fmaf(-r1, A.fU[0], A.fU[1]), c1i = fmaf(-r1, A.fV[0], A.fV[1]);
+            const float c2j = fmaf(-r2, A.fU[0], A.fU[2]), c2i = fmaf(-r2, A.fV[0], A.fV[2]);
+            const uint32_t o = origin(V);
+#pragma unroll
+            for (int k = 0; k < ZV; ++k) {
+                const float fk = (float)k, dn = k ? fmaf(fk, Nz, V.dn) : V.dn, Tc = dn * A.finv_kappa;
+                T.pj = V.pj;
+                T.pi = V.pi;
+                if (k) {
+                    const float kl = fk * A.fkappa * __builtin_amdgcn_rcpf(dn);
+                    T.pj = fmaf(kl, gj, V.pj);
+                    T.pi = fmaf(kl, gi, V.pi);
+                }
+                T.A1j = Tc * fmaf(-fk, uj, c1j);
+                T.A1i = Tc * fmaf(-fk, ui, c1i);
+                T.A2j = Tc * c2j;
+                T.A2i = Tc * c2i;
+                T.fBj = Tc * uj;
+                T.fBi = Tc * ui;
+                box(V, mj, mi, T);
+                acc[k] += tilted_sum<CONE>(rs, T, o, pitch);
+            }
+        } else {
+#pragma unroll 1
+            for (int k = 0; k < ZV; ++k) {
+                float sum = 0.0f;
+                if (setup(z0 + k, V)) {
+                    const float lam = A.fkappa * __builtin_amdgcn_rcpf(V.dn), c = A.fspan * fabsf(lam);
+                    const float M00 = fmaf(-A.fN[1], V.tj, A.fBj[1]), M01 = fmaf(-A.fN[2], V.tj, A.fBj[2]);
+                    const float M10 = fmaf(-A.fN[1], V.ti, A.fBi[1]), M11 = fmaf(-A.fN[2], V.ti, A.fBi[2]);
+                    const float s = fabsf(lam) * __builtin_amdgcn_rcpf(1.0f - c);
+                    const float iW0 = __builtin_amdgcn_rcpf(V.W0), r1 = V.W1 * iW0, r2 = V.W2 * iW0;
+                    const float Tc = V.dn * A.finv_kappa, TW = Tc * iW0;
+                    T.pj = V.pj;
+                    T.pi = V.pi;
+                    T.A1j = Tc * fmaf(-r1, A.fU[0], A.fU[1]);
+                    T.A1i = Tc * fmaf(-r1, A.fV[0], A.fV[1]);
+                    T.A2j = Tc * fmaf(-r2, A.fU[0], A.fU[2]);
+                    T.A2i = Tc * fmaf(-r2, A.fV[0], A.fV[2]);
+                    T.fBj = A.fU[0] * TW;
+                    T.fBi = A.fV[0] * TW;
+                    box(V, fmaf(fabsf(M00) + fabsf(M01), s, 1e-3f), fmaf(fabsf(M10) + fabsf(M11), s, 1e-3f), T);
+                    if (!(c < 1.0f - 1e-6f)) {  // an unbounded image
+                        T.jl = -V.j0;
+                        T.jh = cols - 1 - V.j0;
+                        T.il = -V.i0;
+                        T.ih = rows - 1 - V.i0;
+                    }
+                    sum = tilted_sum<CONE>(rs, T, origin(V), pitch);
+                }
+#pragma unroll
+                for (int e = 0; e < ZV; ++e) acc[e] += e == k ? sum : 0.0f;
+            }
+        }
+    }
+    if (x >= nx || y >= ny) return;
+#pragma unroll
+    for (int k = 0; k < ZV; ++k)
+        if (z0 + k < nz) emit(vol + (int64_t)b * vol_stride, ((int64_t)(z0 + k) * ny + y) * nx + x, b, acc[k], ep);
 }
 
 // Length-weighted projections for the separable backprojector, transposed so

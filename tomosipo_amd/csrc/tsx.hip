@@ -596,6 +596,11 @@ int build_angles(const tsx_geometry *g, tsx_plan *p)
         A.kappa = cone ? dot(P0 - S, N) : 0.0;
         A.EN = cone ? 0.0 : dot(S, N);
         A.inv_kappa = A.kappa != 0.0 ? 1.0 / A.kappa : 0.0;
+        A.sBj = A.sBi = 0.0;
+        for (int k = 0; k < 3 && cone; ++k) {
+            A.sBj += (A.S[k] - A.P0[k]) * A.Bj[k];
+            A.sBi += (A.S[k] - A.P0[k]) * A.Bi[k];
+        }
         A.inv_EN = A.EN != 0.0 ? 1.0 / A.EN : 0.0;
         A.inv_S0 = !cone && A.S[0] != 0.0 ? 1.0 / A.S[0] : 0.0;
         for (int k = 0; k < 3; ++k) {
@@ -603,6 +608,15 @@ int build_angles(const tsx_geometry *g, tsx_plan *p)
             A.fV[k] = (float)A.V[k];
         }
         parallel_map(A);
+        for (int k = 0; k < 3; ++k) {
+            A.fN[k] = (float)A.N[k];
+            A.fBj[k] = (float)(cone ? A.Bj[k] : A.par_c[1 + k]);
+            A.fBi[k] = (float)(cone ? A.Bi[k] : A.par_c[5 + k]);
+        }
+        A.fkappa = (float)A.kappa;
+        A.finv_kappa = (float)A.inv_kappa;
+        A.fspan = (float)((std::fabs(A.N[1]) + std::fabs(A.N[2])) * std::fabs(A.inv_kappa));
+        A.freach = (float)(16.0 * (std::fabs(A.N[0]) + std::fabs(A.N[1]) + std::fabs(A.N[2])));
         tile_slopes(A, g->det_row_count, g->det_col_count, &slope_j[a], &slope_i[a]);
         p->axis_count[m] += 1;
     }
@@ -932,12 +946,12 @@ int64_t bp_workspace_elems(const tsx_plan *p)
     return (int64_t)p->rows * p->n_angles * p->cols;
 }
 
-// The general backprojector takes length-weighted projections (like the
-// separable one) for detector supersampling 1, within the launch limits of
-// the weighting pass.
+// Plans without the separable backprojector take bp_tilted, on length-weighted
+// projections, for detector supersampling 1 (an angle's projections are
+// addressed with 32-bit offsets).
 bool bp_general_prescaled(const tsx_plan *p, int64_t /*batch*/)
 {
-    return !p->bp_separable && p->ss == 1;
+    return !p->bp_separable && p->ss == 1 && (int64_t)p->rows * p->cols * 4 < ((int64_t)1 << 32);
 }
 
 // Scratch sizes rounded up to 256 bytes.
@@ -1757,8 +1771,8 @@ BpView bp_view(const tsx_plan *p, int BZ, float *vol, int64_t vs, const float *l
 }
 
 // bp_general over every batch entry, in launches of at most 65535 slices x
-// entries (grid z); `ly` non-null: length-weighted projections (PRESCALED).
-template <typename T, bool PRESCALED>
+// entries (grid z).
+template <typename T>
 int launch_bp_general(const tsx_plan *p, T *vol, int64_t vs, const T *proj, int64_t ps, int64_t batch,
                       Epilogue ep, hipStream_t stream)
 {
@@ -1768,7 +1782,7 @@ int launch_bp_general(const tsx_plan *p, T *vol, int64_t vs, const T *proj, int6
         const int64_t nb = std::min(bc, batch - b0);
         dim3 grid((unsigned)((p->nx + BP_BX - 1) / BP_BX), (unsigned)((p->ny + BP_BY - 1) / BP_BY),
                   (unsigned)(p->nz * nb));
-        auto kernel = p->kind == TSX_CONE_VEC ? bp_general<T, PRESCALED, true> : bp_general<T, PRESCALED, false>;
+        auto kernel = p->kind == TSX_CONE_VEC ? bp_general<T, true> : bp_general<T, false>;
         hipLaunchKernelGGL(kernel, grid, dim3(BP_BX, BP_BY), 0, stream, p->dev,
                            p->n_angles, p->rows, p->cols, p->ss, p->nx, p->ny, p->nz, vol + b0 * vs, vs,
                            proj + b0 * ps, ps, ep_from(ep, b0));
@@ -1777,6 +1791,39 @@ int launch_bp_general(const tsx_plan *p, T *vol, int64_t vs, const T *proj, int6
     return TSX_OK;
 }
 
+// Voxels per thread of bp_tilted: eight share a set-up, or two, or none where
+// more would leave fewer than four blocks per CU (of one entry: the choice
+// changes the rounding of positions, so it depends on the plan alone).
+int tilted_voxels(const tsx_plan *p)
+{
+    const int64_t columns = (int64_t)((p->nx + BP_BX - 1) / BP_BX) * ((p->ny + BP_BY - 1) / BP_BY);
+    for (int zv : {8, 2})
+        if (columns * ((p->nz + zv - 1) / zv) >= 1024) return zv;
+    return 1;
+}
+
+// bp_tilted over every batch entry of the length-weighted projections `ly`,
+// in launches of at most 65535 groups of slices x entries (grid z).
+int launch_bp_tilted(const tsx_plan *p, float *vol, int64_t vs, const float *ly, int64_t ly_stride, int64_t batch,
+                     Epilogue ep, hipStream_t stream)
+{
+    if (p->nz > GRID_DIM_MAX) return fail(TSX_ERR_UNSUPPORTED, "volume depth exceeds 65535 slices");
+    const int zv = tilted_voxels(p);
+    const int64_t groups = (p->nz + zv - 1) / zv, bc = GRID_DIM_MAX / groups;  // entries per launch
+    const bool cone = p->kind == TSX_CONE_VEC;
+    auto kernel = zv == 8   ? (cone ? bp_tilted<true, 8> : bp_tilted<false, 8>)
+                  : zv == 2 ? (cone ? bp_tilted<true, 2> : bp_tilted<false, 2>)
+                            : (cone ? bp_tilted<true, 1> : bp_tilted<false, 1>);
+    for (int64_t b0 = 0; b0 < batch; b0 += bc) {
+        const int64_t nb = std::min(bc, batch - b0);
+        dim3 grid((unsigned)((p->nx + BP_BX - 1) / BP_BX), (unsigned)((p->ny + BP_BY - 1) / BP_BY),
+                  (unsigned)(groups * nb));
+        hipLaunchKernelGGL(kernel, grid, dim3(BP_BX, BP_BY), 0, stream, p->dev, p->n_angles, p->rows, p->cols, p->nx,
+                           p->ny, p->nz, vol + b0 * vs, vs, ly + b0 * ly_stride, ly_stride, ep_from(ep, b0));
+    }
+    TSX_HIP_CHECK(hipGetLastError());
+    return TSX_OK;
+}
 
 // up > 1: p is the refined-detector plan of a plan with detector
 // supersampling up, and proj holds that plan's (coarse) projections.
@@ -1817,9 +1864,9 @@ int launch_bp(const tsx_plan *p, float *vol, int64_t vs, const float *proj, int6
             if (rc) return rc;
             float *ly = (float *)wptr;
             launch_scale_by_length(p, proj, ps, ly, sino, batch, stream);
-            return launch_bp_general<float, true>(p, vol, vs, ly, sino, batch, ep, stream);
+            return launch_bp_tilted(p, vol, vs, ly, sino, batch, ep, stream);
         }
-        return launch_bp_general<float, false>(p, vol, vs, proj, ps, batch, ep, stream);
+        return launch_bp_general<float>(p, vol, vs, proj, ps, batch, ep, stream);
     }
     // transposed, padded projections of the angles of one launch (all of them
     // unless they reach chunk_bytes: then ranges of sorted angles, each range's
@@ -1880,7 +1927,7 @@ int launch_general(const tsx_plan *p, bool forward, T *vol, int64_t vs, T *proj,
 {
     if (batch <= 0) return TSX_OK;
     if (forward) return launch_fp_general<T>(p, (const T *)vol, vs, proj, ps, batch, ep, stream);
-    return launch_bp_general<T, false>(p, vol, vs, (const T *)proj, ps, batch, ep, stream);
+    return launch_bp_general<T>(p, vol, vs, (const T *)proj, ps, batch, ep, stream);
 }
 
 // ---------------------------------------------------------------------------

@@ -30,6 +30,11 @@ struct AngleParams {
     double inv_EN;        // parallel: 1 / EN
     double inv_S0;        // parallel: 1 / S[0] (the ray's component along m)
     float fU[3], fV[3];   // U and V rounded to float
+    double sBj, sBi;      // cone: (S - P0) . Bj, (S - P0) . Bi
+    // cone: floats of N, Bj, Bi, kappa and 1 / kappa; (|N1| + |N2|) / |kappa|;
+    // 16 (|N0| + |N1| + |N2|). parallel: the position's steps (fBj, fBi)
+    // along (m, c1, c2)
+    float fN[3], fBj[3], fBi[3], fkappa, finv_kappa, fspan, freach;
     // parallel beam: detector position of grid point k = (k_m, k_c1, k_c2),
     // j = par_c[0] + k . par_c[1..3], i = par_c[4] + k . par_c[5..7]; the
     // local map's terms (A1j, A1i, A2j, A2i) and the half-widths (in
