@@ -1770,22 +1770,22 @@ BpView bp_view(const tsx_plan *p, int BZ, float *vol, int64_t vs, const float *l
     return v;
 }
 
-// bp_general over every batch entry, in launches of at most 65535 slices x
-// entries (grid z).
+// bp_general over every batch entry, in launches of at most 65535 entries.
 template <typename T>
 int launch_bp_general(const tsx_plan *p, T *vol, int64_t vs, const T *proj, int64_t ps, int64_t batch,
                       Epilogue ep, hipStream_t stream)
 {
     if (p->nz > GRID_DIM_MAX) return fail(TSX_ERR_UNSUPPORTED, "volume depth exceeds 65535 slices");
-    const int64_t bc = GRID_DIM_MAX / p->nz;  // entries per launch
+    const int64_t blocks = ((int64_t)p->nx * p->ny * p->nz + BP_BX - 1) / BP_BX;
+    // (work-items of a launch stay below 2^32: ranges of voxels of one entry, or whole entries)
+    const int64_t cap = max_blocks(BP_BX * BP_BY), bc = std::max<int64_t>(1, std::min(GRID_DIM_MAX, cap / blocks));
+    auto kernel = p->kind == TSX_CONE_VEC ? bp_general<T, true> : bp_general<T, false>;
     for (int64_t b0 = 0; b0 < batch; b0 += bc) {
         const int64_t nb = std::min(bc, batch - b0);
-        dim3 grid((unsigned)((p->nx + BP_BX - 1) / BP_BX), (unsigned)((p->ny + BP_BY - 1) / BP_BY),
-                  (unsigned)(p->nz * nb));
-        auto kernel = p->kind == TSX_CONE_VEC ? bp_general<T, true> : bp_general<T, false>;
-        hipLaunchKernelGGL(kernel, grid, dim3(BP_BX, BP_BY), 0, stream, p->dev,
-                           p->n_angles, p->rows, p->cols, p->ss, p->nx, p->ny, p->nz, vol + b0 * vs, vs,
-                           proj + b0 * ps, ps, ep_from(ep, b0));
+        for (int64_t f = 0; f < blocks; f += cap)
+            hipLaunchKernelGGL(kernel, dim3((unsigned)std::min(cap, blocks - f), (unsigned)nb), dim3(BP_BX, BP_BY), 0,
+                               stream, p->dev, p->n_angles, p->rows, p->cols, p->ss, p->nx, p->ny, p->nz, f,
+                               vol + b0 * vs, vs, proj + b0 * ps, ps, ep_from(ep, b0));
     }
     TSX_HIP_CHECK(hipGetLastError());
     return TSX_OK;
