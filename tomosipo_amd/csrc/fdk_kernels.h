@@ -1,9 +1,9 @@
 // FDK reconstruction kernels (included by tsx.hip); cone-beam plans only.
 //
-// fdk_filter: one block per (detector row i, angle a). The row is weighted by
-//   the cosine of each pixel's ray against the detector normal, staged in LDS
-//   between zero margins, and convolved with the sampled Ram-Lak kernel
-//   g[0] = 1/4, g[odd m] = -1/(pi^2 m^2) over every lag of the row (the linear
+// fdk_filter: one block per angle and 16 detector rows. The rows are weighted
+//   by the cosine of each pixel's ray against the detector normal and convolved
+//   on the matrix cores (FP32) with the sampled Ram-Lak kernel g[0] = 1/4,
+//   g[odd m] = -1/(pi^2 m^2) over every lag of the row (the linear
 //   convolution of the zero-padded row), scaled by 1 / |U|.
 // fdk_bp: one thread per voxel; for every angle the voxel centre is projected
 //   from the source onto the virtual detector (FP64), the filtered
@@ -16,119 +16,175 @@
 
 namespace tsx {
 
-constexpr int FDK_FILTER_THREADS = 128;
-constexpr int FDK_FR = 6;   // consecutive outputs per filter thread
-constexpr int FDK_FK = 8;   // odd lags per register chunk
 constexpr int FDK_MAX_COLS = 4096;
-constexpr int FDK_FW = FDK_FR + 2 * FDK_FK;  // window of one side per chunk, floats
-constexpr int FDK_PASS = FDK_FILTER_THREADS * FDK_FR;  // outputs per pass over a row
-
-// LDS layout of fdk_filter for a row of `cols` pixels: the weighted row at
-// offset fdk_zl(cols) between zeros (wide enough for every lag of every
-// output of the last pass), then the lag coefficients.
-__host__ __device__ inline int fdk_nodd_pad(int cols)
-{
-    return (cols / 2 + FDK_FK - 1) / FDK_FK * FDK_FK;
-}
-__host__ __device__ inline int fdk_zl(int cols) { return 2 * fdk_nodd_pad(cols) + 2; }
-__host__ __device__ inline int fdk_lds_floats(int cols)
-{
-    const int passes = (cols + FDK_PASS - 1) / FDK_PASS;
-    return fdk_zl(cols) + passes * FDK_PASS + 2 * fdk_nodd_pad(cols) + FDK_FW + fdk_nodd_pad(cols);
-}
-
 constexpr int FDK_BX = 64, FDK_BY = 4;
+
+// fdk_filter<NT> computes 64 NT outputs of 16 rows in a pass, wave w those of
+// parity w & 1 in NT tiles of 16, from 64 NT columns at a time in LDS.
+constexpr int FDK_ROWS = 16, FDK_FILTER_THREADS = 256;
+
+// Tiles per wave: the multiplications are passes^2 NT^2, and the loading and
+// weighting of the columns for each of passes^2 parts about 5 NT of them.
+__host__ __device__ inline int fdk_tiles(int cols)
+{
+    int best = 12, least = 1 << 30;
+    for (int nt = 12; nt >= 2; nt = nt > 8 ? 8 : nt / 2) {
+        const int passes = (cols + 64 * nt - 1) / (64 * nt), cost = passes * passes * nt * (nt + 5);
+        if (cost < least) {
+            least = cost;
+            best = nt;
+        }
+    }
+    return best;
+}
+// Entries of the factor tables on either side of lag 0.
+__host__ __device__ inline int fdk_factor_reach(int cols)
+{
+    const int half = 32 * fdk_tiles(cols);
+    return ((cols + 1) / 2 + half - 1) / half * half + 16;
+}
+constexpr int fdk_filter_floats(int nt) { return 2 * (FDK_ROWS * (32 * nt + 4) + 16) + 64 * nt + 16; }
 
 // With `pair`, q is written row-paired: element (i, a, j) holds the filtered
 // values of rows i and i + 1 (0 past the last row), 8 bytes.
 //
-// The convolution is register-tiled: thread t computes the outputs
-// j0 .. j0 + FDK_FR - 1 (j0 = FDK_FR t within a pass) over the odd lags
-// m = 2k + 1 in chunks of FDK_FK, from two windows of the row that it reads
-// once per chunk (the samples j - m and j + m of all its outputs and lags in
-// the chunk), as 8-byte LDS reads; thread starts FDK_FR = 6 floats apart keep
-// them free of bank conflicts. One LDS read per output and lag instead of
-// three.
+// The ramp filter couples columns of opposite parity only. With c_p[y] the
+// weighted pixel 2 y + p, and E[y] = c_p[y] - c_p[y - 1] the differences of
+// the other parity p's pixels (zeros outside the row),
+//   q[j] = (2 c[j] - c[j - 1] - c[j + 1]) / 8 + sum_y F(y - j / 2 - (j & 1)) E[y],
+//   F(t) = -sign(t) * (sum of 1 / (pi^2 m^2) over the odd m > 2 |t|), F(0) = 0:
+// summation by parts of the plain sum, exact because the kernel has no DC
+// response. A row that is smooth on the pixel scale has small differences,
+// while the terms of the plain sum nearly cancel c[j] / 4. Where a pixel of
+// the rows is infinite or NaN, the block takes the plain sum, q[j] = c[j] / 4
+// + sum_y H(y - j / 2 - (j & 1)) c_p[y - 1], H(t) = -1 / (pi^2 (2 t - 1)^2),
+// which spreads it as the filter's definition says.
 //
-// The sum is taken in difference form: the kernel has no DC response
-// (g[0] + 2 sum of g[odd m] = 0 over all lags), so
-//   q[j] = (0.25 - 2 sum_k coef_k) c[j] - sum_k coef_k (c[j - m] + c[j + m] - 2 c[j]),
-// with the first factor (`tail`, over the lags summed here) computed in FP64
-// by the caller. For a row that is smooth on the pixel scale the plain sum
-// nearly cancels 0.25 c[j] and loses about ten times more to FP32 rounding.
-__global__ void __launch_bounds__(FDK_FILTER_THREADS)
-fdk_filter(const FdkAngle *__restrict__ angles, int n_angles, int rows, int cols,
-           const float *__restrict__ proj, float *__restrict__ q, int pair, float tail)
+// Either sum is a product of 16 rows with a Toeplitz matrix: MFMA 16x16x4 in
+// FP32, A = the rows (lane: row lane % 16, the slots 4 (lane / 16) + s, s = 0 ..
+// 3, of each 16 as one 16-byte LDS read), B = the factors, read from the
+// 64 NT + 16 of them that the pass and columns at hand meet. Rows S = 32 NT + 4
+// floats apart keep both reads free of bank conflicts; the results go through
+// LDS to be written in rows.
+//
+// Bound: the matrix cores' FP32 rate (157 TFLOP/s; 2 cols FLOP per output,
+// half of the full product), with three blocks per CU at 768 columns so that
+// one loads while another multiplies. 512 x 720 rows of 768 columns: FIGURE ms (the sum
+// of factor (c[j - m] + c[j + m] - 2 c[j]) on the vector ALUs, register-tiled:
+// 10.4 ms; in this form there: 9.5 ms).
+template <int NT>
+__global__ void __launch_bounds__(FDK_FILTER_THREADS, NT > 8 ? 3 : 4)
+fdk_filter(const FdkAngle *__restrict__ angles, int n_angles, int rows, int cols, const float *__restrict__ factors,
+           const float *__restrict__ proj, float *__restrict__ q, int pair)
 {
-    extern __shared__ __align__(16) float lds[];
-    const int nodd_pad = fdk_nodd_pad(cols), zl = fdk_zl(cols), nbuf = fdk_lds_floats(cols) - nodd_pad;
-    float *buf = lds;           // buf[zl + j]: weighted pixel j; zeros elsewhere
-    float *coef = lds + nbuf;   // coef[k] = 1 / (pi^2 (2k + 1)^2)
-    const int i = blockIdx.x, a = blockIdx.y;
+    typedef float f4 __attribute__((ext_vector_type(4)));
+    constexpr int HALF = 32 * NT, S = HALF + 4, PAR = FDK_ROWS * S + 16, W = 2 * HALF + 4, OUT = 2 * HALF + 4;
+    __shared__ __align__(16) float lds[fdk_filter_floats(NT)];
+    float *tab = lds + 2 * PAR;
+    const int i0 = blockIdx.x * FDK_ROWS, a = blockIdx.y;
     const FdkAngle &A = angles[a];
-    const int64_t row = ((int64_t)i * n_angles + a) * cols;
-    for (int k = threadIdx.x; k < nbuf; k += blockDim.x) {
-        const int j = k - zl;
-        float v = 0.0f;
-        if (j >= 0 && j < cols) {
-            const double px = A.P0s[0] + j * A.U[0] + i * A.V[0];
-            const double py = A.P0s[1] + j * A.U[1] + i * A.V[1];
-            const double pz = A.P0s[2] + j * A.U[2] + i * A.V[2];
-            v = (float)(A.D / sqrt(px * px + py * py + pz * pz) * (double)proj[row + j]);
-        }
-        buf[k] = v;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int p = wave & 1, u0 = (wave >> 1) * 16 * NT, n = lane & 15, h = lane >> 4;
+    const int passes = ((cols + 1) / 2 + HALF - 1) / HALF;
+    const int64_t pitch = (int64_t)n_angles * cols;
+    const float *src = proj + (int64_t)i0 * pitch + (int64_t)a * cols;
+    int plain = 0;
+    if (passes > 1) {  // every pass and every part of a row has to take the same sum
+        bool bad = false;
+        for (int r = 0; r < FDK_ROWS && i0 + r < rows; ++r)
+            for (int k = threadIdx.x; k < cols; k += FDK_FILTER_THREADS)
+                bad |= !(fabsf(src[r * pitch + k]) <= 3.402823466e38f);
+        plain = __syncthreads_or(bad);
     }
-    for (int k = threadIdx.x; k < nodd_pad; k += blockDim.x) {
-        const double m = 2.0 * k + 1.0;
-        coef[k] = (float)(1.0 / (M_PI * M_PI * m * m));
-    }
-    __syncthreads();
-    const float inv_du = (float)A.inv_du;
-    for (int base = 0; base < cols; base += FDK_PASS) {
-        const int j0 = base + FDK_FR * (int)threadIdx.x;  // even
-        float part[FDK_FR], c2[FDK_FR];
+    for (int pass = 0; pass < passes; ++pass) {
+        const int ub = pass * HALF;
+        f4 acc[NT];
 #pragma unroll
-        for (int r = 0; r < FDK_FR; ++r) {
-            part[r] = 0.0f;
-            c2[r] = 2.0f * buf[zl + j0 + r];
-        }
-        for (int k0 = 0; k0 < nodd_pad; k0 += FDK_FK) {
-            // left window from j0 - 2 (k0 + FDK_FK), right window from j0 + 2 k0 (both even)
-            const float2 *lw = reinterpret_cast<const float2 *>(buf + zl + j0 - 2 * (k0 + FDK_FK));
-            const float2 *rw = reinterpret_cast<const float2 *>(buf + zl + j0 + 2 * k0);
-            float L[FDK_FW], R[FDK_FW], ck[FDK_FK];
-#pragma unroll
-            for (int x = 0; x < FDK_FW / 2; ++x) {
-                const float2 l2 = lw[x], r2 = rw[x];
-                L[2 * x] = l2.x;
-                L[2 * x + 1] = l2.y;
-                R[2 * x] = r2.x;
-                R[2 * x + 1] = r2.y;
+        for (int t = 0; t < NT; ++t) acc[t] = f4{0.0f, 0.0f, 0.0f, 0.0f};
+        for (int k = 0; k < passes; ++k) {
+            // (the pass's own columns come last: the outputs need them)
+            const int part = (pass + 1 + k) % passes, yb = part * HALF;
+            // slot s of row r and parity p: c_p[yb - 1 + s], s = 0 .. HALF + 1
+            bool bad = false;
+            __syncthreads();
+#pragma unroll 2
+            for (int e = threadIdx.x; e < FDK_ROWS * W; e += FDK_FILTER_THREADS) {
+                const int r = e / W, kk = e - r * W, j = 2 * yb - 2 + kk, i = i0 + r;
+                float v = 0.0f;
+                if (j >= 0 && j < cols && i < rows) {
+                    const double px = A.P0s[0] + j * A.U[0] + i * A.V[0];
+                    const double py = A.P0s[1] + j * A.U[1] + i * A.V[1];
+                    const double pz = A.P0s[2] + j * A.U[2] + i * A.V[2];
+                    v = (float)(A.D / sqrt(px * px + py * py + pz * pz) * (double)src[r * pitch + j]);
+                }
+                bad |= !(fabsf(v) <= 3.402823466e38f);
+                lds[(kk & 1) * PAR + r * S + (kk >> 1)] = v;
             }
+            plain |= __syncthreads_or(bad);
+            const int reach = passes * HALF + 16;
+            const float *f = factors + (plain ? 2 * reach + 1 : 0) + reach + (yb - ub) - HALF;
+            for (int e = threadIdx.x; e < 2 * HALF + 16; e += FDK_FILTER_THREADS) tab[e] = f[e];
+            __syncthreads();
+            // the other parity's differences (or pixels) yb .. yb + nd - 1
+            const int nd = part == passes - 1 ? (p ? (cols + 1) / 2 : cols / 2) + 1 - yb : HALF;
+            const float *line = lds + (1 - p) * PAR + n * S + 4 * h;
+            const float *fac = tab + HALF - u0 - p + 4 * h - n;
+            for (int kb = 0; kb < nd; kb += 16) {
+                const float4 c = *reinterpret_cast<const float4 *>(line + kb);
+                const float next = line[kb + 4];
+                float e[4];
+                e[0] = plain ? c.x : c.y - c.x;
+                e[1] = plain ? c.y : c.z - c.y;
+                e[2] = plain ? c.z : c.w - c.z;
+                e[3] = plain ? c.w : next - c.w;
+                if (kb + 16 > nd) {
 #pragma unroll
-            for (int kk = 0; kk < FDK_FK; ++kk) ck[kk] = coef[k0 + kk];
+                    for (int s = 0; s < 4; ++s)
+                        if (kb + 4 * h + s >= nd) e[s] = 0.0f;
+                }
 #pragma unroll
-            for (int kk = 0; kk < FDK_FK; ++kk) {
+                for (int s = 0; s < 4; ++s) {
 #pragma unroll
-                for (int r = 0; r < FDK_FR; ++r) {
-                    // samples j - m and j + m, j = j0 + r, m = 2 (k0 + kk) + 1
-                    const float sum = (L[r - 2 * kk - 1 + 2 * FDK_FK] + R[r + 2 * kk + 1]) - c2[r];
-                    part[r] = fmaf(ck[kk], sum, part[r]);
+                    for (int t = 0; t < NT; ++t)
+                        acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(e[s], fac[kb - 16 * t + s], acc[t], 0, 0, 0);
+                    __builtin_amdgcn_sched_barrier(0);
                 }
             }
         }
+        // acc[t][g]: row 4 h + g, column 2 (ub + u0 + 16 t + n) + p
+        const float inv_du = (float)A.inv_du;
 #pragma unroll
-        for (int r = 0; r < FDK_FR; ++r) {
-            const int j = j0 + r;
-            if (j >= cols) break;
-            const float v = inv_du * fmaf(tail, buf[zl + j], -part[r]);
+        for (int t = 0; t < NT; ++t) {
+            const int u = u0 + 16 * t + n;
+#pragma unroll
+            for (int g = 0; g < 4; ++g) {
+                const float *even = lds + (4 * h + g) * S + u, *odd = even + PAR;
+                const float c = p ? odd[1] : even[1], l = p ? even[1] : odd[0], r = p ? even[2] : odd[1];
+                acc[t][g] = inv_du * (plain ? fmaf(0.25f, c, acc[t][g]) : fmaf(0.125f, (c - l) + (c - r), acc[t][g]));
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        __syncthreads();
+#pragma unroll
+        for (int t = 0; t < NT; ++t)
+#pragma unroll
+            for (int g = 0; g < 4; ++g) lds[(4 * h + g) * OUT + 2 * (u0 + 16 * t + n) + p] = acc[t][g];
+        __syncthreads();
+        for (int e = threadIdx.x; e < FDK_ROWS * 2 * HALF; e += FDK_FILTER_THREADS) {
+            const int r = e / (2 * HALF), k = e - r * 2 * HALF, j = 2 * ub + k, i = i0 + r;
+            if (j >= cols || i >= rows) continue;
+            const float v = lds[r * OUT + k];
+            const int64_t o = (int64_t)i * pitch + (int64_t)a * cols + j;
             if (!pair) {
-                q[row + j] = v;
+                q[o] = v;
             } else {
-                const int64_t prev = ((int64_t)(i - 1) * n_angles + a) * cols;
-                q[2 * (row + j)] = v;
-                if (i > 0) q[2 * (prev + j) + 1] = v;
-                if (i == rows - 1) q[2 * (row + j) + 1] = 0.0f;
+                if (i == rows - 1)
+                    reinterpret_cast<float2 *>(q)[o] = make_float2(v, 0.0f);
+                else if (r < FDK_ROWS - 1)
+                    reinterpret_cast<float2 *>(q)[o] = make_float2(v, lds[(r + 1) * OUT + k]);
+                else
+                    q[2 * o] = v;
+                if (r == 0 && i > 0) q[2 * (o - pitch) + 1] = v;
             }
         }
     }
@@ -152,12 +208,12 @@ fdk_bp(const FdkAngle *__restrict__ angles, int n_angles, int rows, int cols,
         const double den = wx * A.n[0] + wy * A.n[1] + wz * A.n[2];
         if (!(den > 0.0)) continue;  // voxel not in front of the source
         const double lam = A.D * rcp64(den);
-        const float fj = (float)(A.cj + lam * (wx * A.Bj[0] + wy * A.Bj[1] + wz * A.Bj[2]));
-        const float fi = (float)(A.ci + lam * (wx * A.Bi[0] + wy * A.Bi[1] + wz * A.Bi[2]));
-        if (!(fj > -1.0f && fj < (float)cols && fi > -1.0f && fi < (float)rows)) continue;
-        const float fj0 = floorf(fj), fi0 = floorf(fi);
+        const double fj = A.cj + lam * (wx * A.Bj[0] + wy * A.Bj[1] + wz * A.Bj[2]);
+        const double fi = A.ci + lam * (wx * A.Bi[0] + wy * A.Bi[1] + wz * A.Bi[2]);
+        if (!(fj > -1.0 && fj < (double)cols && fi > -1.0 && fi < (double)rows)) continue;
+        const double fj0 = floor(fj), fi0 = floor(fi);
         const int j0 = (int)fj0, i0 = (int)fi0;
-        const float wj = fj - fj0, wi = fi - fi0;
+        const float wj = (float)(fj - fj0), wi = (float)(fi - fi0);
         // corners outside the detector read a clamped (in-bounds) pixel and count 0
         const float *base = q + (int64_t)a * astride;
         const bool j_lo = j0 >= 0, j_hi = j0 + 1 < cols, i_lo = i0 >= 0, i_hi = i0 + 1 < rows;
@@ -207,14 +263,17 @@ fdk_bp_upright(const FdkAngle *__restrict__ angles, int n_angles, int rows, int 
             const double den = wx * A.n[0] + wy * A.n[1];
             if (!(den > 0.0)) return;
             const double lam = A.D * rcp64(den);
-            const float fj = (float)(A.cj + lam * (wx * A.Bj[0] + wy * A.Bj[1]));
-            if (!(fj > -1.0f && fj < (float)cols)) return;
-            const float fi0 = (float)(A.ci + lam * (wx * A.Bi[0] + wy * A.Bi[1] + wz * A.Bi[2]));
+            const double fj = A.cj + lam * (wx * A.Bj[0] + wy * A.Bj[1]);
+            if (!(fj > -1.0 && fj < (double)cols)) return;
+            // rows relative to the first voxel's, floor(fi): FP32 holds their fractions
+            const double fi = fmin(fmax(A.ci + lam * (wx * A.Bi[0] + wy * A.Bi[1] + wz * A.Bi[2]), -1e9), 1e9);
+            const int ib = (int)floor(fi);
+            const float fi0 = (float)(fi - ib);
             const float dfi = (float)(lam * h_z * A.Bi[2]);
             const float wgt = (float)(A.half_dbeta * lam * lam);
-            const float fj0 = floorf(fj);
+            const double fj0 = floor(fj);
             const int j0 = (int)fj0;
-            const float wj = fj - fj0;
+            const float wj = (float)(fj - fj0);
             // columns (jb, jb + 1), jb = j0 clamped into [0, cols - 2], read as one
             // 8-byte pair; the weights of columns outside the detector are 0
             const int jb = min(max(j0, 0), max(cols - 2, 0));
@@ -236,7 +295,7 @@ fdk_bp_upright(const FdkAngle *__restrict__ angles, int n_angles, int rows, int 
             for (int k = 0; k < FDK_ZC; ++k) {
                 const float fi = fmaf((float)k, dfi, fi0);
                 const float fi0f = floorf(fi);
-                const int i0 = (int)fi0f;
+                const int i0 = ib + (int)fi0f;
                 const float wi = fi - fi0f;
                 // rows i0, i0 + 1 from the element of row max(i0, 0) (inside the
                 // buffer); for i0 = -1 that element's first row is row i0 + 1

@@ -211,6 +211,7 @@ struct tsx_plan {
     int32_t flat_stage_bp = 0;          // detector columns staged per angle
     std::vector<FdkAngle> fdk_host;
     FdkAngle *fdk_dev = nullptr;
+    const float *fdk_factors = nullptr;  // the ramp filter's factors (after fdk_dev's entries)
     bool fdk_upright = false;  // every angle: v parallel to z, normal perpendicular to z
     double vlo[3] = {0, 0, 0}, vh[3] = {0, 0, 0};
 };
@@ -371,6 +372,25 @@ void build_fdk(const tsx_geometry *g, tsx_plan *p)
         F.half_dbeta = 0.5 * db;
         F.inv_du = 1.0 / std::sqrt(dot(U, U));
     }
+}
+
+// The ramp filter's factors F(t), then H(t), t = -reach .. reach (fdk_filter).
+std::vector<float> fdk_filter_factors(int cols)
+{
+    const int reach = fdk_factor_reach(std::min(cols, FDK_MAX_COLS));
+    std::vector<float> f(2 * (2 * (size_t)reach + 1));
+    double k = 0.125;  // the sum of 1 / (pi^2 m^2) over the odd m > 2 t
+    for (int t = 1; t <= reach; ++t) {
+        const double m = 2.0 * t - 1.0;
+        k -= 1.0 / (M_PI * M_PI * m * m);
+        f[reach + t] = (float)-k;
+        f[reach - t] = (float)k;
+    }
+    for (int t = -reach; t <= reach; ++t) {
+        const double m = 2.0 * t - 1.0;
+        f[3 * (size_t)reach + 1 + t] = (float)(-1.0 / (M_PI * M_PI * m * m));
+    }
+    return f;
 }
 
 // The device angle table of a plan: the angles in order, then ordered by
@@ -2730,8 +2750,12 @@ int tsx_plan_create(const tsx_geometry *g, int device, tsx_plan **out)
         }
         if (!p->fdk_host.empty()) {
             const size_t fb = sizeof(FdkAngle) * p->fdk_host.size();
-            e = hipMalloc((void **)&p->fdk_dev, fb);
+            const std::vector<float> factors = fdk_filter_factors(p->cols);
+            e = hipMalloc((void **)&p->fdk_dev, fb + factors.size() * 4);
             if (e == hipSuccess) e = hipMemcpy(p->fdk_dev, p->fdk_host.data(), fb, hipMemcpyHostToDevice);
+            p->fdk_factors = (const float *)((const char *)p->fdk_dev + fb);
+            if (e == hipSuccess)
+                e = hipMemcpy((void *)p->fdk_factors, factors.data(), factors.size() * 4, hipMemcpyHostToDevice);
             if (e != hipSuccess) {
                 if (p->fdk_dev) (void)hipFree(p->fdk_dev);
                 (void)hipFree(p->dev);
@@ -2903,15 +2927,11 @@ int tsx_fdk(const tsx_plan *p, float *vol, const float *proj, int additive, void
     rc = get_workspace(p, need, workspace, workspace_bytes, s, owned, &wptr);
     if (rc) return rc;
     float *q = (float *)wptr;
-    const size_t lds = (size_t)fdk_lds_floats(p->cols) * sizeof(float);
-    double tail = 0.25;  // 0.25 - 2 * sum of the filter's lag coefficients
-    for (int k = fdk_nodd_pad(p->cols) - 1; k >= 0; --k) {
-        const double m = 2.0 * k + 1.0;
-        tail -= 2.0 / (M_PI * M_PI * m * m);
-    }
-    hipLaunchKernelGGL(fdk_filter, dim3((unsigned)p->rows, (unsigned)p->n_angles), dim3(FDK_FILTER_THREADS),
-                       lds, s, p->fdk_dev, p->n_angles, p->rows, p->cols, proj, q, upright ? 1 : 0,
-                       (float)tail);
+    const int nt = fdk_tiles(p->cols);
+    auto filter = nt == 12 ? fdk_filter<12> : nt == 8 ? fdk_filter<8> : nt == 4 ? fdk_filter<4> : fdk_filter<2>;
+    hipLaunchKernelGGL(filter, dim3((unsigned)((p->rows + FDK_ROWS - 1) / FDK_ROWS), (unsigned)p->n_angles),
+                       dim3(FDK_FILTER_THREADS), 0, s, p->fdk_dev, p->n_angles, p->rows, p->cols, p->fdk_factors, proj,
+                       q, upright ? 1 : 0);
     TSX_HIP_CHECK(hipGetLastError());
     const unsigned gx = (unsigned)((p->nx + FDK_BX - 1) / FDK_BX), gy = (unsigned)((p->ny + FDK_BY - 1) / FDK_BY);
     if (upright)
