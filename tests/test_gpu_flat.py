@@ -63,6 +63,10 @@ CASES = {
     "skewed": dict(shape=(66, 24, 24), det=(70, 36), angles=13, skew=0.2),
     "voxels": dict(shape=(66, 24, 30), det=(70, 45), angles=13, voxel=(0.7, 1.2, 0.9), pitch=1.1),
     "narrow": dict(shape=(70, 48, 48), det=(20, 7), angles=17),
+    "three_slices": dict(shape=(3, 40, 44), det=(3, 131), angles=33),
+    "eight_slices": dict(shape=(8, 70, 66), det=(9, 300), angles=66),
+    "longest_chunk": dict(shape=(127, 20, 24), det=(131, 33), angles=11),
+    "aligned_chunks": dict(shape=(192, 20, 24), det=(180, 150), angles=35),
     "many_angles": dict(shape=(4, 16, 16), det=(4, 24), angles=300),
     "many_angles_long": dict(shape=(150, 8, 8), det=(150, 40), angles=170),
 }

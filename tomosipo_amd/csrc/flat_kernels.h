@@ -11,10 +11,10 @@
 // and the sums over slices and columns have one weight for a whole line along
 // z. The kernels keep z contiguous (volume turned to [x][y][w], G and U as
 // [angle][column][w]; w = (batch entry, z), so that short stacks and 2D
-// slices of a batch fill the lanes), take 64 ZL consecutive w per wave (ZL per
-// lane) and broadcast the weights from the lane that formed them
-// (v_readlane): 2 fma per (ray, slice, z) or (voxel, column) instead of a
-// gather and a bilinear interpolation of their own.
+// slices of a batch fill the lanes), take consecutive w per lane and share the
+// weights that one lane formed (through LDS or v_readlane): 2 fma per (ray,
+// slice, z) or (voxel, column) instead of a gather and a bilinear
+// interpolation of their own.
 //
 // Every lane's arithmetic and its order depend only on the plan, never on the
 // position of its w in a wave, so single, batched and fused launches give
@@ -28,9 +28,8 @@
 namespace tsx {
 
 constexpr int FLAT_MAX = MAX_FUSED;  // instances of one launch
-constexpr int FLAT_FW = 8;           // forward projector: waves per block
-constexpr int FLAT_JW = 8;           // forward projector: detector columns per wave
-constexpr int FLAT_NARROW = 40, FLAT_WIDE = 64;  // forward: most voxel columns staged per slice (two kernels)
+constexpr int FLAT_RAYS = 32;        // forward projector: most rays per wave
+constexpr int FLAT_STRIP = 8;        // forward projector: column tiles per strip
 // forward: slices (n / FLAT_SUM of the volume) summed before they join the rest of a ray's sum.
 // One running sum over the 256 slices of a slice stack rounds to 3.6e-7 of the result, the
 // padded kernels' two to 1.9e-7, sums of 32 to 1.6e-7 (for 1 to 2 % of the time).
@@ -44,21 +43,18 @@ struct FlatView {
     const FlatAngle *ang;
     int kn;                 // angles of the launch
     int n_angles, rows, cols, nx, ny, nz;
-    int W, Wp;              // batch entries x nz, and the pitch of a line (a multiple of 4)
+    int W, Wp;              // batch entries x nz, and the pitch of a line
     float *vol, *proj;      // caller's data: read or written, entries vs and ps floats apart
     int64_t vs, ps;
     float *turned;          // forward: the volume as [x][y][Wp]
     float *lines;           // G or U as [kn][cols][Wp]
     Epilogue ep;
     int up;                 // backward: pixels per coarse pixel edge (refined detector), else 1
-    int stage;              // columns staged at a time
-    // forward: group[g] .. group[g + 1] - 1 are the angles (of the plan) of
-    // group g, at most ag; k0 the launch's first angle; column tiles
-    const int32_t *group;
-    int groups, ag, k0, tiles;
+    int stage;              // backward: columns staged at a time
+    int quads, rays;        // forward: lanes per ray (V of w each) and rays per wave
     int bx, by, parts, part_len;  // backward: bricks, angle parts
     float *partial;         // backward: the parts' sums ([entry][part][z][y][x]), null for one part
-    int chunks;             // chunks of 64 ZL of w
+    int chunks;             // chunks of w
 };
 
 struct FlatMulti {
@@ -316,263 +312,149 @@ __global__ void __launch_bounds__(256) flat_splat(FlatMulti M)
 // ---------------------------------------------------------------------------
 // forward: G[a, j, w]
 // ---------------------------------------------------------------------------
-// A block of 8 waves takes a group of at most `ag` (4 or 2) neighbouring
-// angles, 64 / ag neighbouring detector columns and 64 ZL of w; a wave 8
-// columns of one angle. The block goes through the slices in step: the voxel
-// columns that its rays meet in the next slice are read (coalesced, once for
-// all angles: neighbouring angles meet nearly the same ones) while the present
-// one is summed from LDS (two buffers, one barrier per slice).
-//
-// Bound: vector ALU issue (half of the time) and the staged lines from L2.
-// Per (ray, slice) 3 readlane, 1 address and 2 ZL fma, i.e. 3 instructions
-// per 64 samples at ZL = 4 (19, and a gather that takes 27 cycles of the
-// texture address unit, in fp_padded). Read from global memory directly, a
-// ray's two lines would take 8 cycles of the 64-byte L1 port per 64 samples,
-// hence the staging, and the sharing between angles. Steps of two slices at
-// ZL = 2 halve the blocks per CU (LDS): 3.9 against 2.5 ms at 75 x 441 x 441,
-// 361 angles, 75 x 623 (fp_padded: 2.96 with its layouts). 8 x 128^3, 180
-// angles, 128 x 192: 0.97 ms with both layout passes against 2.56.
-template <int ZL, int SW>
-__global__ void __launch_bounds__(64 * FLAT_FW) fp_flat(FlatMulti M)
+template <int V>
+__device__ __forceinline__ FlatVec<V> flat_bload(__amdgpu_buffer_rsrc_t rs, uint32_t bytes)
 {
-    extern __shared__ __align__(16) float flat_lds[];
-    __shared__ float line_r[FLAT_FW], line_a[FLAT_FW];
-    __shared__ int range_lo[FLAT_FW], range_hi[FLAT_FW];
-    constexpr int CF = 64 * ZL;  // floats per staged column
-    const int logical = xcd_logical(M.shift);
-    if (logical >= M.begin[M.n]) return;
-    const int inst = owner_of(M.begin, logical);
-    const FlatView &v = M.v[inst];
-    const int id = logical - M.begin[inst];
-    const int g = id % v.groups, jt = (id / v.groups) % v.tiles, w0 = (id / (v.groups * v.tiles)) * CF;
-    const int ag = v.ag, Wp = v.Wp, cols = v.cols, SC = v.stage;
-    const int k0 = v.group[g] - v.k0, cnt = v.group[g + 1] - v.group[g];
-    const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int ai = wv % ag;
-    const bool live = ai < cnt;  // (the waves past the group's last angle only stage)
-    const int jb = (jt * (FLAT_FW / ag) + wv / ag) * FLAT_JW;
-    typedef const __attribute__((address_space(4))) FlatAngle ConstAngle;
-    ConstAngle &A = ((ConstAngle *)v.ang)[k0 + min(ai, cnt - 1)];
-    const int m = A.m;
-    const int nm = m == 0 ? v.nx : v.ny, nc = m == 0 ? v.ny : v.nx;
-    // voxel column (n, c) starts at n sn + c sc
-    const int64_t sn = m == 0 ? (int64_t)v.ny * Wp : Wp, sc = m == 0 ? Wp : (int64_t)v.ny * Wp;
-    const int nref = nm / 2;
-    const int jj = lane & 7, nn = lane >> 3;
-    // the ray of column jb + jj: q(n) = R + (n - nref) a2, slices with q in (-1, nc)
-    const double Rd = A.q0 + A.qm * (double)nref + A.qj * (double)min(jb + jj, cols - 1);
-    int lo = 0, hi = nm - 1;
-    if (A.qm != 0.0) {
-        const double t0 = (-1.0 - Rd) / A.qm, t1 = ((double)nc - Rd) / A.qm;
-        lo = max(0, (int)fmax(ceil(fmin(t0, t1) + nref), -1e9));
-        hi = min(nm - 1, (int)fmin(floor(fmax(t0, t1) + nref), 1e9));
-    } else if (!(Rd > -1.0 && Rd < (double)nc)) {
-        lo = nm;
-        hi = -1;
-    }
-    if (lo > hi) {
-        lo = nm;
-        hi = -1;
-    }
-    const float rmin = wave_minf((float)Rd);
-    lo = wave_min(lo);
-    hi = wave_max(hi);
-    if (lane == 0) {
-        line_r[wv] = rmin;
-        line_a[wv] = (float)A.qm;
-        range_lo[wv] = lo;
-        range_hi[wv] = hi;
-    }
-    __syncthreads();
-#pragma unroll
-    for (int e = 0; e < FLAT_FW; ++e) {
-        lo = min(lo, range_lo[e]);
-        hi = max(hi, range_hi[e]);
-    }
-    lo = __builtin_amdgcn_readfirstlane(lo);
-    hi = __builtin_amdgcn_readfirstlane(hi);
-    const int w = w0 + lane * ZL;
-    FlatVec<ZL> acc[FLAT_JW];
-#pragma unroll
-    for (int e = 0; e < FLAT_JW; ++e)
-#pragma unroll
-        for (int z = 0; z < ZL; ++z) acc[e].v[z] = 0.0f;
-    // (lanes past the last w read the line's last values; nothing of theirs is written)
-    const float *src = v.turned + min(w, Wp - ZL);
-    const int64_t sc8 = sc * FLAT_FW;
-    FlatVec<ZL> next[SW];
-    int kbv = 0;  // lane's first staged column of slice lo + 64 i + lane
-    auto bases = [&](int n) {
-        const float dn = (float)(n + lane - nref);
-        float q = fmaf(dn, line_a[0], line_r[0]);
-#pragma unroll
-        for (int e = 1; e < FLAT_FW; ++e) q = fminf(q, fmaf(dn, line_a[e], line_r[e]));
-        // (the margin exceeds the FP32 rounding of the positions)
-        kbv = (int)floorf(fminf(fmaxf(q - 2e-3f, -1e8f), 1e8f));
-    };
-    // the staged columns of slice n: column kb + s in place s, zeros beyond the volume
-    auto load = [&](int n) {
-        const int c0 = lane_i(kbv, (n - lo) & 63) + wv;
-        const float *p = src + ((int64_t)n * sn + (int64_t)c0 * sc);
-#pragma unroll
-        for (int e = 0; e < SW; ++e) {
-            if ((unsigned)(c0 + e * FLAT_FW) < (unsigned)nc) {
-                next[e] = flat_load<ZL>(p + e * sc8);
-            } else {
-#pragma unroll
-                for (int z = 0; z < ZL; ++z) next[e].v[z] = 0.0f;
-            }
-        }
-    };
-    if (lo <= hi) {
-        bases(lo);
-        load(lo);
-    }
-    // the sums of FLAT_SUM slices join the lines in memory
-    float *out = v.lines + ((int64_t)(k0 + ai) * cols + jb) * Wp + w;
-    bool first = true;
-    auto flush = [&]() {
-        if (live && w < Wp) {
-#pragma unroll
-            for (int e = 0; e < FLAT_JW; ++e)
-                if (jb + e < cols) flat_join<ZL>(out + (int64_t)e * Wp, acc[e], first);
-        }
-        first = false;
-    };
-    int off = 0;  // lane (nn, jj): staged place of ray jj's lower column in slice n + nn, in floats
-    float wl = 0.0f, wh = 0.0f;
-    for (int n = lo; n <= hi; ++n) {
-        const int at = n - lo;
-        if ((at & 7) == 0) {
-            const int kb = __shfl(kbv, (at & 63) + nn, 64);
-            const double q = fma((double)(n + nn - nref), A.qm, Rd), f = floor(q);
-            wh = (float)(q - f);
-            wl = 1.0f - wh;
-            off = min(max((int)fmin(fmax(f, -1e8), 1e8) - kb, 0), SC - 2) * CF;
-        }
-        float *buf = flat_lds + (at & 1) * SC * CF + lane * ZL;
-#pragma unroll
-        for (int e = 0; e < SW; ++e)
-            if (wv + e * FLAT_FW < SC) flat_store<ZL>(buf + (wv + e * FLAT_FW) * CF, next[e]);
-        __syncthreads();
-        if (n < hi) {
-            if (((at + 1) & 63) == 0) bases(n + 1);
-            load(n + 1);
-        }
-        if (live) {
-            constexpr int JB = 4;  // rays whose columns are in flight together
-#pragma unroll
-            for (int e0 = 0; e0 < FLAT_JW; e0 += JB) {
-                FlatVec<ZL> a[JB], b[JB];
-#pragma unroll
-                for (int e = 0; e < JB; ++e) {
-                    const float *p = buf + lane_i(off, (at & 7) * 8 + e0 + e);
-                    a[e] = flat_load<ZL>(p);
-                    b[e] = flat_load<ZL>(p + CF);
-                }
-                __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-                for (int e = 0; e < JB; ++e) {
-                    const int ray = (at & 7) * 8 + e0 + e;
-                    const float fl = lane_f(wl, ray), fh = lane_f(wh, ray);
-#pragma unroll
-                    for (int z = 0; z < ZL; ++z)
-                        acc[e0 + e].v[z] = fmaf(fh, b[e].v[z], fmaf(fl, a[e].v[z], acc[e0 + e].v[z]));
-                }
-                __builtin_amdgcn_sched_barrier(0);
-            }
-        }
-        if ((n + 1) % FLAT_SUM == 0) flush();
-    }
-    if (lo > hi || (hi + 1) % FLAT_SUM) flush();
+    if constexpr (V == 4)
+        return __builtin_bit_cast(FlatVec<4>, __builtin_amdgcn_raw_buffer_load_b128(rs, bytes, 0, 0));
+    else
+        return __builtin_bit_cast(FlatVec<1>, __builtin_amdgcn_raw_buffer_load_b32(rs, bytes, 0, 0));
 }
 
-// The same without staging, for short lines (64 of w per wave, one per lane),
-// for the reasons given at bp_flat_direct: a wave of one angle and 4 detector
-// columns reads the two voxel columns of every ray and slice from global
-// memory (the line of zeros after the last one where they lie beyond the
-// volume). 64^3, 96 angles, 64 x 96: 22 us against 49 with fp_flat and 39 with
-// fp_padded (and its layouts 10, here 11 in two passes).
-constexpr int FLAT_DJ = 4;  // detector columns per wave of fp_flat_direct
-
-__global__ void __launch_bounds__(256) fp_flat_direct(FlatMulti M)
+// A wave takes `rays` neighbouring detector columns of one angle and 4 quads
+// of w (lane: ray lane / quads, V = 4 consecutive w at 4 (lane % quads); V = 1
+// on lines of fewer than 4 w), a block four neighbouring angles, whose rays
+// meet nearly the same voxel columns. Slice by slice every ray takes the two
+// voxel columns beside it straight from memory (the line of zeros after the
+// last one where they lie beyond the volume), with the weights and addresses
+// of up to 32 slices formed by all lanes (FP64 positions) and passed on through
+// LDS. The launch goes through chunks of at most 80 of w, in a chunk through strips
+// of 8 column tiles, in a strip through the angles: the blocks that an XCD runs
+// together meet few voxel columns, so that its L2 holds them (512^3, 360
+// angles: 9.9 ms; angles before tiles, chunks of 256 of w: 19.4 ms).
+//
+// Bound: the L1 port and L2 (two 16-byte loads per lane, 8 fma, one LDS read
+// for 4 samples). fp_padded with its layouts against this with both layout
+// passes, pixel pitch sqrt 2 (in brackets 1):
+//   64^3, 180 angles      58 (72) and 35 (36) us
+//   128^3, 360 angles    0.40 (0.55) and 0.17 (0.21) ms
+//   256^3, 360 angles    2.17 (3.39) and 1.11 (1.43) ms
+//   512^3, 360 angles    15.4 and 10.0 ms
+//   75 x 441 x 441, 361  1.79 (2.81) and 1.28 (1.44) ms
+//   16 x (256 x 256), 180 angles 0.64 and 0.09 ms; one slice 69 and 74 us
+// Taken back: lines staged in LDS by blocks that go through the slices in step
+// (a barrier per slice: 200^3, 360 angles, pitch sqrt 2 1.07 ms against 0.72
+// here; few blocks on small volumes: 80^3, 60 angles 0.09 against 0.03); one ray
+// per wave with weights from readlane (1.15 ms).
+template <int V>
+__global__ void __launch_bounds__(256) fp_flat(FlatMulti M)
 {
-    constexpr int JN = FLAT_DJ, NL = 64 / JN;  // slices whose weights a wave holds
+    constexpr int EN = 256;  // (ray, slice) entries of a wave at a time
+    constexpr int UN = 8;    // slices whose columns are in flight together
+    __shared__ float4 entry[4][EN];
     const int logical = xcd_logical(M.shift);
     if (logical >= M.begin[M.n]) return;
     const int inst = owner_of(M.begin, logical);
     const FlatView &v = M.v[inst];
     const int id = logical - M.begin[inst];
-    const int tiles = (v.cols + 4 * JN - 1) / (4 * JN), cols = v.cols, Wp = v.Wp;
-    const int k = id % v.kn, jt = (id / v.kn) % tiles, w0 = (id / (v.kn * tiles)) * 64;
+    const int cols = v.cols, Wp = v.Wp, L = v.quads, R = v.rays;
+    const int tiles = (cols + R - 1) / R, ks = (v.kn + 3) / 4;
     const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int jb = (jt * 4 + wv) * JN;
-    if (jb >= cols) return;
+    constexpr int T = FLAT_STRIP;
+    const int per = ks * tiles, chunk = id / per, in_chunk = id - chunk * per;
+    const int strip = in_chunk / (ks * T), width = min(T, tiles - strip * T), in_strip = in_chunk - strip * ks * T;
+    const int jb = (strip * T + in_strip % width) * R, w0 = chunk * V * L, k = in_strip / width * 4 + wv;
+    if (k >= v.kn) return;
     typedef const __attribute__((address_space(4))) FlatAngle ConstAngle;
     ConstAngle &A = ((ConstAngle *)v.ang)[k];
     const int m = A.m;
     const int nm = m == 0 ? v.nx : v.ny, nc = m == 0 ? v.ny : v.nx;
     const int sn = m == 0 ? v.ny : 1, sc = m == 0 ? 1 : v.ny;  // voxel column (n, c) is n sn + c sc
     const int nref = nm / 2, zero = v.nx * v.ny;
-    const int jj = lane % JN, nn = lane / JN;
-    const double Rd = A.q0 + A.qm * (double)nref + A.qj * (double)min(jb + jj, cols - 1);
+    // the ray of column j: q(n) = base + j qj + (n - nref) qm, slices with q in (-1, nc)
+    const double base = fma(A.qm, (double)nref, A.q0);
     int lo = 0, hi = nm - 1;
-    if (A.qm != 0.0) {
-        const double t0 = (-1.0 - Rd) / A.qm, t1 = ((double)nc - Rd) / A.qm;
-        lo = max(0, (int)fmax(ceil(fmin(t0, t1) + nref), -1e9));
-        hi = min(nm - 1, (int)fmin(floor(fmax(t0, t1) + nref), 1e9));
-    } else if (!(Rd > -1.0 && Rd < (double)nc)) {
-        lo = nm;
-        hi = -1;
-    }
-    if (lo > hi) {
-        lo = nm;
-        hi = -1;
+    {
+        const double Rd = fma(A.qj, (double)min(jb + lane % R, cols - 1), base);
+        if (A.qm != 0.0) {
+            const double t0 = (-1.0 - Rd) / A.qm, t1 = ((double)nc - Rd) / A.qm;
+            lo = max(0, (int)fmax(ceil(fmin(t0, t1) + nref), -1e9));
+            hi = min(nm - 1, (int)fmin(floor(fmax(t0, t1) + nref), 1e9));
+        } else if (!(Rd > -1.0 && Rd < (double)nc)) {
+            lo = nm;
+            hi = -1;
+        }
+        if (lo > hi) {
+            lo = nm;
+            hi = -1;
+        }
     }
     lo = __builtin_amdgcn_readfirstlane(wave_min(lo));
     hi = __builtin_amdgcn_readfirstlane(wave_max(hi));
-    const int w = w0 + lane;
-    const float *src = v.turned + min(w, Wp - 1);
-    FlatVec<1> acc[JN];
+    const int r = lane / L, w = w0 + (lane - r * L) * V;
+    const bool live = r < R && w < Wp;
+    const uint32_t lane_bytes = (uint32_t)w * 4u, line_bytes = (uint32_t)Wp * 4u;
+    const __amdgpu_buffer_rsrc_t rs =
+        __builtin_amdgcn_make_buffer_rsrc((void *)v.turned, (short)0, (int)((uint32_t)(zero + 1) * line_bytes), 0x00020000);
+    FlatVec<V> acc;
 #pragma unroll
-    for (int e = 0; e < JN; ++e) acc[e].v[0] = 0.0f;
-    static_assert(FLAT_SUM % NL == 0, "steps end where sums do");
-    float *out = v.lines + ((int64_t)k * cols + jb) * Wp + w;
+    for (int z = 0; z < V; ++z) acc.v[z] = 0.0f;
+    float *out = v.lines + ((int64_t)k * cols + jb + r) * Wp + w;
     bool first = true;
     auto flush = [&]() {
-        if (w < Wp) {
-#pragma unroll
-            for (int e = 0; e < JN; ++e)
-                if (jb + e < cols) flat_join<1>(out + (int64_t)e * Wp, acc[e], first);
-        }
+        if (live && jb + r < cols) flat_join<V>(out, acc, first);
         first = false;
     };
-    for (int n0 = lo / NL * NL; n0 <= hi; n0 += NL) {
-        const int n = n0 + nn;
-        const double q = fma((double)(n - nref), A.qm, Rd), f = floor(q);
-        const float wh = (float)(q - f), wl = 1.0f - wh;
-        const int c = (int)fmin(fmax(f, -1e8), 1e8);
-        const int ra = n < nm && (unsigned)c < (unsigned)nc ? n * sn + c * sc : zero;
-        const int rb = n < nm && (unsigned)(c + 1) < (unsigned)nc ? n * sn + (c + 1) * sc : zero;
-        constexpr int UN = 16 / JN;  // slices whose columns are in flight together
-        for (int h = 0; h < NL && n0 + h <= hi; h += UN) {
-            float a[UN * JN], b[UN * JN];
-#pragma unroll
-            for (int e = 0; e < UN * JN; ++e) {
-                a[e] = src[(int64_t)lane_i(ra, h * JN + e) * Wp];
-                b[e] = src[(int64_t)lane_i(rb, h * JN + e) * Wp];
+    // slices whose entries are formed together (a power of two from UN to FLAT_SUM; NS R <= EN)
+    const int NS = R <= 8 ? 32 : (R <= 16 ? 16 : 8);
+    // (ray, slice) of the lane's first entry of a step, and the way from one to the next
+    const int h0 = lane / R, ray0 = lane - h0 * R, step_h = 64 / R, step_r = 64 - step_h * R;
+    for (int n0 = lo / NS * NS; n0 <= hi; n0 += NS) {
+        int h = h0, ray = ray0;
+        for (int e = lane; e < NS * R; e += 64) {
+            const int n = n0 + h;
+            const double Rd = fma(A.qj, (double)min(jb + ray, cols - 1), base);
+            const double q = fma((double)(n - nref), A.qm, Rd), f = floor(q);
+            ray += step_r;
+            h += step_h;
+            if (ray >= R) {
+                ray -= R;
+                ++h;
             }
-            __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-            for (int e = 0; e < UN * JN; ++e) {
-                const float fl = lane_f(wl, h * JN + e), fh = lane_f(wh, h * JN + e);
-                acc[e % JN].v[0] = fmaf(fh, b[e], fmaf(fl, a[e], acc[e % JN].v[0]));
-            }
-            __builtin_amdgcn_sched_barrier(0);
+            const float wh = (float)(q - f);
+            const int c = (int)fmin(fmax(f, -1e8), 1e8);
+            const uint32_t ra = (uint32_t)(n < nm && (unsigned)c < (unsigned)nc ? n * sn + c * sc : zero) * line_bytes;
+            const uint32_t rb =
+                (uint32_t)(n < nm && (unsigned)(c + 1) < (unsigned)nc ? n * sn + (c + 1) * sc : zero) * line_bytes;
+            entry[wv][e] = make_float4(1.0f - wh, wh, __builtin_bit_cast(float, ra), __builtin_bit_cast(float, rb));
         }
-        if ((n0 + NL) % FLAT_SUM == 0) flush();
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        if (live) {
+            const float4 *in = entry[wv] + r;
+            for (int h = 0; h < NS && n0 + h <= hi; h += UN) {
+                float4 t[UN];
+                FlatVec<V> a[UN], b[UN];
+#pragma unroll
+                for (int e = 0; e < UN; ++e) t[e] = in[(h + e) * R];
+#pragma unroll
+                for (int e = 0; e < UN; ++e) {
+                    a[e] = flat_bload<V>(rs, __builtin_bit_cast(uint32_t, t[e].z) + lane_bytes);
+                    b[e] = flat_bload<V>(rs, __builtin_bit_cast(uint32_t, t[e].w) + lane_bytes);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int e = 0; e < UN; ++e)
+#pragma unroll
+                    for (int z = 0; z < V; ++z) acc.v[z] = fmaf(t[e].y, b[e].v[z], fmaf(t[e].x, a[e].v[z], acc.v[z]));
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        if ((n0 + NS) % FLAT_SUM == 0) flush();
     }
-    if (lo > hi || (hi / NL + 1) * NL % FLAT_SUM) flush();
+    if (lo > hi || (hi / NS + 1) * NS % FLAT_SUM) flush();
 }
 
 // ---------------------------------------------------------------------------
@@ -873,12 +755,6 @@ __global__ void __launch_bounds__(256) flat_parts_reduce(FlatMulti M)
 }
 
 using FlatKernel = void (*)(FlatMulti);
-
-inline FlatKernel fp_flat_kernel(int zl, bool wide)
-{
-    if (zl == 4) return wide ? fp_flat<4, FLAT_WIDE / FLAT_FW> : fp_flat<4, FLAT_NARROW / FLAT_FW>;
-    return wide ? fp_flat<2, FLAT_WIDE / FLAT_FW> : fp_flat<2, FLAT_NARROW / FLAT_FW>;
-}
 
 inline FlatKernel bp_flat_kernel(int zl, int nc)
 {

@@ -202,11 +202,6 @@ struct tsx_plan {
     // stepping axis (empty: the plan is not flat), and the columns they stage
     std::vector<FlatAngle> flat_host;
     FlatAngle *flat_dev = nullptr;
-    // forward: first angles of the groups of at most flat_ag angles that share
-    // a block, ended by the angle count; voxel columns staged per slice
-    std::vector<int32_t> flat_groups;
-    int32_t *flat_groups_dev = nullptr;
-    int32_t flat_ag = 0, flat_stage_fp = 0;
     int32_t flat_nc = 0;                // backward: detector columns per voxel column
     int32_t flat_stage_bp = 0;          // detector columns staged per angle
     std::vector<FdkAngle> fdk_host;
@@ -447,53 +442,6 @@ void build_flat(tsx_plan *p)
     // detector columns with a weight in a voxel column: |j - jc| < 1 / b2
     p->flat_nc = (int32_t)std::ceil(std::min(1e6, 2.0 * h_max - 1e-9));
     if (p->flat_nc < 2) p->flat_nc = 2;
-    // Forward groups: consecutive angles of one axis whose rays meet at most
-    // `limit` voxel columns per slice together (the window of a tile of
-    // columns is widest at the ends of the slices and of the tiles: its lines
-    // are affine in both). Four angles per group where that needs clearly
-    // fewer groups than two, on tiles of 16 instead of 32 columns.
-    const auto window = [&](size_t k0, size_t k1, int jt) {
-        double wide = 0.0;
-        const int nm = t[k0].m == 0 ? p->nx : p->ny;
-        for (double n : {0.0, (double)(nm - 1)})
-            for (double j0 : {0.0, (double)((p->cols - 1) / jt * jt)}) {
-                double lo = 1e300, hi = -1e300;
-                for (size_t k = k0; k < k1; ++k)
-                    for (double j : {j0, std::min(j0 + jt, (double)p->cols) - 1}) {
-                        const double q = t[k].q0 + t[k].qm * n + t[k].qj * j;
-                        lo = std::min(lo, q);
-                        hi = std::max(hi, q);
-                    }
-                wide = std::max(wide, hi - lo);
-            }
-        return (int32_t)std::min(1e6, std::floor(wide + 0.01) + 4.0);
-    };
-    // (No grouping, where a tile of one angle already meets more: the kernels
-    // without staging take those plans, flat_stage_fp = 0.)
-    p->flat_groups.clear();
-    for (int k = 0; k <= (int)t.size(); ++k) p->flat_groups.push_back(k);
-    p->flat_ag = 2;
-    p->flat_stage_fp = 0;
-    for (int ag : {4, 2}) {
-        const int jt = FLAT_FW / ag * FLAT_JW;
-        int32_t most = FLAT_NARROW, stage = 0;
-        for (size_t k = 0; k < t.size(); ++k) most = std::max(most, window(k, k + 1, jt));
-        if (most > FLAT_WIDE) continue;
-        if (ag == 2) most = FLAT_WIDE;
-        std::vector<int32_t> groups;
-        for (size_t k0 = 0; k0 < t.size();) {
-            size_t k1 = k0 + 1;
-            while (k1 < t.size() && (int)(k1 - k0) < ag && t[k1].m == t[k0].m && window(k0, k1 + 1, jt) <= most) ++k1;
-            stage = std::max(stage, window(k0, k1, jt));
-            groups.push_back((int32_t)k0);
-            k0 = k1;
-        }
-        if (p->flat_stage_fp && groups.size() * 10 > (p->flat_groups.size() - 1) * 14) continue;
-        groups.push_back((int32_t)t.size());
-        p->flat_groups = std::move(groups);
-        p->flat_ag = ag;
-        p->flat_stage_fp = stage;
-    }
     // detector columns that a brick meets
     double brick = 0.0;
     for (const FlatAngle &f : t) {
@@ -1016,21 +964,26 @@ bool fp_refined(const tsx_plan *p)
 // The choice only cuts the work into blocks: no result depends on it.
 struct FlatPlan {
     bool ok = false;
-    int zl = 1;      // consecutive w per lane
-    bool direct = false;  // short lines: the kernels without staging
-    bool wide = false;    // forward: the kernel of wide windows
-    int stage = 0;   // columns staged at a time
-    int chunks = 1;  // chunks of 64 zl of w
+    int v = 4, quads = 1, rays = 1;  // forward: w per lane, lanes per ray, rays per wave
+    int zl = 1;      // backward: consecutive w per lane
+    bool direct = false;  // backward, short lines: the kernel without staging
+    int stage = 0;   // backward: columns staged at a time
+    int chunks = 1;  // chunks of w
     int per_launch = 0;  // angles per launch
     size_t lds = 0;
 };
 
-int64_t flat_pitch(const tsx_plan *p, int64_t batch) { return (p->nz * batch + 3) / 4 * 4; }
+// Pitch of a line of w: a multiple of 4, and of the forward projector's 16-byte
+// loads, unless the line is shorter.
+int64_t flat_pitch(const tsx_plan *p, int64_t batch)
+{
+    const int64_t W = p->nz * batch;
+    return W < 4 ? W : (W + 3) / 4 * 4;
+}
 
-// Lanes: the fewest w per lane that cover W in one chunk, at most 4 (W = 64:
-// 1, on the kernels without staging; 128: 2). Fewer w per lane than that cost
-// more instructions per w: 8 x 128^3 (W = 1024) forward 0.80, 0.88 and 1.32 ms
-// with 4, 2 and 1.
+// Backward, lanes: the fewest w per lane that cover W in one chunk, at most 4
+// (W = 64: 1, on the kernels without staging; 128: 2). Fewer w per lane than
+// that cost more instructions per w.
 int flat_zl(int64_t W) { return W > 128 ? 4 : (W > 64 ? 2 : 1); }
 
 // The turned volume and its line of zeros.
@@ -1041,24 +994,38 @@ int64_t flat_turned_elems(const tsx_plan *p, int64_t batch)
 
 // Workspace floats of the forward projector. The flat kernels' turned volume
 // and sums G live in that of the padded layouts (which is two to four times
-// the volume), G for as many angles at a time as it holds; it is grown where
-// that would be fewer than 64 (detectors far wider than the volume), unless
-// that took the plan past the static buffer of tsx_direct_fpbp3d_noalloc: it
-// then stays on the padded kernels.
+// the volume), G for as many angles at a time as it holds; it is grown to
+// flat_angles of them, unless 64 took the plan past the static buffer of
+// tsx_direct_fpbp3d_noalloc: it then stays on the padded kernels.
 bool flat_fp_ok(const tsx_plan *p)
 {
     if (p->flat_host.empty() || force_general() || env_int("TSX_FP_VARIANT") >= 2 || !p->fp_padded) return false;
+    if (flat_turned_elems(p, 1) * 4 >= (int64_t)1 << 32) return false;  // 32-bit byte offsets
     const int64_t need = flat_turned_elems(p, 1) + (int64_t)p->cols * flat_pitch(p, 1) * std::min(p->n_angles, 64);
     return need * 4 <= TSX_NOALLOC_SCRATCH_BYTES || fp_workspace_elems(p) * 4 > TSX_NOALLOC_SCRATCH_BYTES ||
            need <= fp_workspace_elems(p);
+}
+
+// Angles whose sums G the workspace has to hold: all of them within 64 MiB per
+// batch entry (a launch of few angles leaves most of the chip idle: 48^3, 360
+// angles in four launches 90 us, in one 52), or 64.
+int64_t flat_angles(const tsx_plan *p)
+{
+    const int64_t room = ((int64_t)1 << 24) - flat_turned_elems(p, 1);
+    return std::min<int64_t>(p->n_angles, std::max<int64_t>(64, room / ((int64_t)p->cols * flat_pitch(p, 1))));
 }
 
 int64_t fp_elems(const tsx_plan *p, int64_t batch)
 {
     const int64_t padded = fp_workspace_elems(p) * batch;
     if (!flat_fp_ok(p)) return padded;
-    return std::max(padded, flat_turned_elems(p, batch) +
-                                (int64_t)p->cols * flat_pitch(p, batch) * std::min(p->n_angles, 64));
+    return std::max(padded, flat_turned_elems(p, batch) + (int64_t)p->cols * flat_pitch(p, batch) * flat_angles(p));
+}
+
+// Blocks of the forward projector (four angles and `rays` columns each).
+int64_t flat_fp_blocks(int angles, int cols, int rays, int chunks)
+{
+    return (int64_t)((angles + 3) / 4) * ((cols + rays - 1) / rays) * chunks;
 }
 
 FlatPlan flat_fp(const tsx_plan *p, int64_t batch)
@@ -1068,13 +1035,19 @@ FlatPlan flat_fp(const tsx_plan *p, int64_t batch)
     if (!flat_fp_ok(p) || W > (1 << 28)) return f;
     f.per_launch = (int)std::min<int64_t>(
         p->n_angles, (fp_elems(p, batch) - flat_turned_elems(p, batch)) / ((int64_t)p->cols * Wp));
-    f.stage = p->flat_stage_fp;
-    f.wide = f.stage > FLAT_NARROW;
-    f.zl = f.stage ? flat_zl(W) : 1;
-    f.direct = f.zl == 1;
-    f.lds = f.direct ? 0 : (size_t)2 * f.stage * f.zl * 256;
+    // Chunks of w: one up to 127; of 64, whole cache lines, where they fit
+    // (512^3, 360 angles: 9.9 ms, chunks of 76 17.1); else at most 80 (134^3,
+    // 360 angles: chunks of 68 0.26 ms, one 0.32). As many rays as fill a wave;
+    // fewer where that leaves fewer than 512 blocks (one slice, whose waves
+    // spend most of their time on weights: 2048. 512 x 512, 360 angles: 0.41
+    // ms with 64 rays, 0.35 so).
+    f.v = W < 4 ? 1 : 4;
+    f.chunks = (int)(W < 128 ? 1 : (W % 64 == 0 ? W / 64 : (W + 79) / 80));
+    f.quads = (int)((Wp / f.v + f.chunks - 1) / f.chunks);
+    f.rays = std::min(FLAT_RAYS, 64 / f.quads);
+    while (f.rays > 8 && flat_fp_blocks(std::min(p->n_angles, f.per_launch), p->cols, f.rays, f.chunks) < (f.v == 1 ? 2048 : 512))
+        f.rays = (f.rays + 1) / 2;
     f.ok = true;
-    f.chunks = (int)((W + 64 * f.zl - 1) / (64 * std::max(f.zl, 1)));
     return f;
 }
 
@@ -1173,10 +1146,10 @@ int64_t max_blocks(int threads_per_block)
     return std::min(MAX_LOGICAL, (int64_t)(0xffffffffLL / threads_per_block) - 9 * 1024);
 }
 
-unsigned xcd_grid(int64_t n, int *shift)
+unsigned xcd_grid(int64_t n, int *shift, int most = 10, int64_t chunks_wanted = 2048)
 {
     int s = 0;
-    while (s < 10 && ((int64_t)2048 << (s + 1)) <= n) ++s;
+    while (s < most && (chunks_wanted << (s + 1)) <= n) ++s;
     const int64_t c = (int64_t)1 << s;
     const int64_t chunks = (n + c - 1) / c;
     *shift = s;
@@ -1520,6 +1493,8 @@ FlatView flat_view(const tsx_plan *p, const FlatPlan &f, int64_t batch, int k0, 
     v.ep = ep;
     v.up = 1;
     v.stage = f.stage;
+    v.quads = f.quads;
+    v.rays = f.rays;
     v.chunks = f.chunks;
     v.parts = 1;
     v.part_len = kn;
@@ -1556,11 +1531,11 @@ struct FlatBatch {
         return TSX_OK;
     }
     template <typename F>
-    int main_pass(FlatKernel kernel, int waves, F &&blocks)
+    int main_pass(FlatKernel kernel, int waves, int most, int64_t chunks, F &&blocks)
     {
         const int64_t n = lay(blocks, 64 * waves);
         if (n < 0) return fail(TSX_ERR_UNSUPPORTED, "flat kernels: too many blocks for one launch");
-        const unsigned grid = xcd_grid(n, &m.shift);
+        const unsigned grid = xcd_grid(n, &m.shift, most, chunks);
         if (lds > 64 * 1024)
             TSX_HIP_CHECK(hipFuncSetAttribute((const void *)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
         hipLaunchKernelGGL(kernel, dim3(grid), dim3(64 * waves), lds, stream, m);
@@ -1571,13 +1546,9 @@ struct FlatBatch {
     {
         int rc = turn ? pass(flat_turn, flat_turn_blocks) : TSX_OK;
         if (rc) return rc;
-        if (f.direct)
-            rc = main_pass(fp_flat_direct, 4, [](const FlatView &v) {
-                return (int64_t)v.kn * ((v.cols + 4 * FLAT_DJ - 1) / (4 * FLAT_DJ)) * v.chunks;
-            });
-        else
-            rc = main_pass(fp_flat_kernel(f.zl, f.wide), FLAT_FW,
-                           [](const FlatView &v) { return (int64_t)v.groups * v.tiles * v.chunks; });
+        rc = main_pass(f.v == 4 ? fp_flat<4> : fp_flat<1>, 4, 8, 128, [](const FlatView &v) {  // (large runs of blocks per XCD: whole strips share its L2)
+            return flat_fp_blocks(v.kn, v.cols, v.rays, v.chunks);
+        });
         return rc ? rc : pass(flat_rows, flat_rows_blocks);
     }
     int backward(const FlatPlan &f, int nc)
@@ -1596,7 +1567,7 @@ struct FlatBatch {
             ve = std::max(ve, (int64_t)v.nx * v.ny * v.nz);
             entries = std::max(entries, v.W / v.nz);
         }
-        rc = main_pass(f.direct ? bp_flat_direct_kernel(nc) : bp_flat_kernel(f.zl, nc), by,
+        rc = main_pass(f.direct ? bp_flat_direct_kernel(nc) : bp_flat_kernel(f.zl, nc), by, 10, 2048,
                        [](const FlatView &v) { return (int64_t)v.bx * v.by * v.chunks * v.parts; });
         if (rc || !sums) return rc;
         hipLaunchKernelGGL(flat_parts_reduce, dim3((unsigned)((ve + 255) / 256), (unsigned)entries, (unsigned)m.n),
@@ -1605,17 +1576,6 @@ struct FlatBatch {
         return TSX_OK;
     }
 };
-
-// The forward groups g0 .. g1 - 1 of a plan in a view (whose angles are theirs).
-void flat_groups(const tsx_plan *p, int g0, int g1, FlatView &v)
-{
-    const int jt = FLAT_FW / p->flat_ag * FLAT_JW;
-    v.group = p->flat_groups_dev + g0;
-    v.groups = g1 - g0;
-    v.ag = p->flat_ag;
-    v.k0 = p->flat_groups[g0];
-    v.tiles = (p->cols + jt - 1) / jt;
-}
 
 // Batch entries of one flat launch: w stays far below 2^28, the blocks below
 // the dispatch limit.
@@ -1628,17 +1588,15 @@ int64_t flat_entries(const tsx_plan *p)
 int launch_fp_flat(const tsx_plan *p, const float *vol, int64_t vs, float *proj, int64_t ps, int64_t batch,
                    Epilogue ep, float *base, hipStream_t stream)
 {
-    const int64_t bc = flat_entries(p);
+    // (the turned volume of a launch is addressed with 32-bit byte offsets)
+    const int64_t room = (((int64_t)1 << 30) - 1) / ((int64_t)p->nx * p->ny + 1) - 3;
+    const int64_t bc = std::max<int64_t>(1, std::min(flat_entries(p), room / p->nz));
     for (int64_t b0 = 0; b0 < batch; b0 += bc) {
         const int64_t nb = std::min(bc, batch - b0);
         const FlatPlan f = flat_fp(p, nb);
-        const int ng = (int)p->flat_groups.size() - 1;
-        for (int g0 = 0, g1; g0 < ng; g0 = g1) {
-            const int k0 = p->flat_groups[g0];
-            for (g1 = g0 + 1; g1 < ng && p->flat_groups[g1 + 1] - k0 <= f.per_launch;) ++g1;
+        for (int k0 = 0; k0 < p->n_angles; k0 += f.per_launch) {
             FlatBatch fb(stream);
-            FlatView v = flat_view(p, f, nb, k0, p->flat_groups[g1] - k0, ep_from(ep, b0));
-            flat_groups(p, g0, g1, v);
+            FlatView v = flat_view(p, f, nb, k0, std::min(f.per_launch, p->n_angles - k0), ep_from(ep, b0));
             v.vol = const_cast<float *>(vol) + b0 * vs;
             v.vs = vs;
             v.proj = proj + b0 * ps;
@@ -1647,8 +1605,7 @@ int launch_fp_flat(const tsx_plan *p, const float *vol, int64_t vs, float *proj,
             v.lines = base + flat_turned_elems(p, nb);
             fb.m.v[0] = v;
             fb.m.n = 1;
-            fb.lds = f.lds;
-            const int rc = fb.forward(f, g0 == 0);
+            const int rc = fb.forward(f, k0 == 0);
             if (rc) return rc;
         }
     }
@@ -2046,16 +2003,14 @@ int multi_fp(const tsx_plan *const *plans, const float *const *vols, float *cons
         for (int e = k; e < n && fb.m.n < FLAT_MAX; ++e) {
             if (taken[e] || !flat_one_launch(plans[e], TSX_OP_FP)) continue;
             const FlatPlan fe = flat_fp(plans[e], 1);
-            if (fe.zl != f.zl || fe.wide != f.wide) continue;
+            if (fe.v != f.v) continue;
             taken[e] = 1;
             FlatView &v = fb.m.v[fb.m.n++];
             v = flat_view(plans[e], fe, 1, 0, plans[e]->n_angles, eps[e]);
-            flat_groups(plans[e], 0, (int)plans[e]->flat_groups.size() - 1, v);
             v.vol = const_cast<float *>(vols[e]);
             v.proj = projs[e];
             v.turned = (float *)((char *)wptr + off[e]);
             v.lines = v.turned + flat_turned_elems(plans[e], 1);
-            fb.lds = std::max(fb.lds, fe.lds);
         }
         const int rc = fb.forward(f, true);
         if (rc) return rc;
@@ -2768,9 +2723,6 @@ int tsx_plan_create(const tsx_geometry *g, int device, tsx_plan **out)
             const size_t fb = sizeof(FlatAngle) * p->flat_host.size();
             e = hipMalloc((void **)&p->flat_dev, fb);
             if (e == hipSuccess) e = hipMemcpy(p->flat_dev, p->flat_host.data(), fb, hipMemcpyHostToDevice);
-            const size_t gb = sizeof(int32_t) * p->flat_groups.size();
-            if (e == hipSuccess && gb) e = hipMalloc((void **)&p->flat_groups_dev, gb);
-            if (e == hipSuccess && gb) e = hipMemcpy(p->flat_groups_dev, p->flat_groups.data(), gb, hipMemcpyHostToDevice);
             if (e != hipSuccess) rc = fail(TSX_ERR_OUT_OF_MEMORY, std::string("flat tables: ") + hipGetErrorString(e));
         }
         if (rc == TSX_OK) rc = build_range_table(p, nullptr, &p->bp_rt);
@@ -2779,7 +2731,6 @@ int tsx_plan_create(const tsx_geometry *g, int device, tsx_plan **out)
         if (rc) {
             if (p->bp_rt) (void)hipFree(p->bp_rt);
             if (p->flat_dev) (void)hipFree(p->flat_dev);
-            if (p->flat_groups_dev) (void)hipFree(p->flat_groups_dev);
             if (p->fdk_dev) (void)hipFree(p->fdk_dev);
             (void)hipFree(p->dev);
             delete p;
@@ -2844,7 +2795,6 @@ int tsx_plan_destroy(tsx_plan *p)
         (void)hipFree(p->dev);
         if (p->fdk_dev) (void)hipFree(p->fdk_dev);
         if (p->flat_dev) (void)hipFree(p->flat_dev);
-        if (p->flat_groups_dev) (void)hipFree(p->flat_groups_dev);
         if (p->bp_rt) (void)hipFree(p->bp_rt);
     }
     delete p;
@@ -2867,8 +2817,7 @@ int tsx_plan_info_get(const tsx_plan *p, tsx_plan_info *info)
     info->plan_bytes = sub_bytes + (p->dev ? (int64_t)(sizeof(AngleParams) * 2 * p->host.size()) *
                                         (1 + (int64_t)p->slabs.size()) +
                                     (p->bp_rt ? p->bp_rt_stride * p->n_angles * 4 : 0) +
-                                    (p->flat_dev ? (int64_t)(sizeof(FlatAngle) * p->flat_host.size() +
-                                                             sizeof(int32_t) * p->flat_groups.size()) : 0)
+                                    (p->flat_dev ? (int64_t)(sizeof(FlatAngle) * p->flat_host.size()) : 0)
                               : 0);
     for (int c = 0; c < 3; ++c) info->axis_count[c] = p->axis_count[c];
     // the plan whose forward kernels run
