@@ -45,8 +45,7 @@ __host__ __device__ inline int fdk_factor_reach(int cols)
 }
 constexpr int fdk_filter_floats(int nt) { return 2 * (FDK_ROWS * (32 * nt + 4) + 16) + 64 * nt + 16; }
 
-// With `pair`, q is written row-paired: element (i, a, j) holds the filtered
-// values of rows i and i + 1 (0 past the last row), 8 bytes.
+// q is written as [row][angle][column], or by_angle as [angle][row][column].
 //
 // The ramp filter couples columns of opposite parity only. With c_p[y] the
 // weighted pixel 2 y + p, and E[y] = c_p[y] - c_p[y - 1] the differences of
@@ -75,7 +74,7 @@ constexpr int fdk_filter_floats(int nt) { return 2 * (FDK_ROWS * (32 * nt + 4) +
 template <int NT>
 __global__ void __launch_bounds__(FDK_FILTER_THREADS, NT > 8 ? 3 : 4)
 fdk_filter(const FdkAngle *__restrict__ angles, int n_angles, int rows, int cols, const float *__restrict__ factors,
-           const float *__restrict__ proj, float *__restrict__ q, int pair)
+           const float *__restrict__ proj, float *__restrict__ q, int by_angle)
 {
     typedef float f4 __attribute__((ext_vector_type(4)));
     constexpr int HALF = 32 * NT, S = HALF + 4, PAR = FDK_ROWS * S + 16, W = 2 * HALF + 4, OUT = 2 * HALF + 4;
@@ -174,18 +173,7 @@ fdk_filter(const FdkAngle *__restrict__ angles, int n_angles, int rows, int cols
             const int r = e / (2 * HALF), k = e - r * 2 * HALF, j = 2 * ub + k, i = i0 + r;
             if (j >= cols || i >= rows) continue;
             const float v = lds[r * OUT + k];
-            const int64_t o = (int64_t)i * pitch + (int64_t)a * cols + j;
-            if (!pair) {
-                q[o] = v;
-            } else {
-                if (i == rows - 1)
-                    reinterpret_cast<float2 *>(q)[o] = make_float2(v, 0.0f);
-                else if (r < FDK_ROWS - 1)
-                    reinterpret_cast<float2 *>(q)[o] = make_float2(v, lds[(r + 1) * OUT + k]);
-                else
-                    q[2 * o] = v;
-                if (r == 0 && i > 0) q[2 * (o - pitch) + 1] = v;
-            }
+            q[by_angle ? ((int64_t)a * rows + i) * cols + j : (int64_t)i * pitch + (int64_t)a * cols + j] = v;
         }
     }
 }
@@ -232,98 +220,164 @@ fdk_bp(const FdkAngle *__restrict__ angles, int n_angles, int rows, int cols,
 }
 
 // Upright detectors (v parallel to z, detector normal perpendicular to z, every
-// angle; at least 2 detector columns; row-paired q): along a voxel column (x, y) the depth,
-// the detector column and the weight are constant and the detector row is
-// affine in z. One thread per (x, y) and FDK_ZC voxels along z: FP64 setup
-// once per angle, FP32 per voxel; the waves of a block go through the angles
-// in step (a barrier per angle).
-constexpr int FDK_ZC = 16;
+// angle; q as [angle][row][column]): along a voxel column (x, y) the depth, the
+// detector column and the weight are constant and the detector row is affine
+// in z. A block takes 16 x 16 columns and ZC voxels of each: FP64 setup
+// once per column and angle, FP32 per voxel.
+//
+// The pixels that the block's voxels read at an angle lie between those of its
+// corners (formed for eight angles at a time, a corner per lane); they are
+// staged in LDS with zeros around the detector, the next angle's while the
+// present one's are summed (two buffers, one barrier per angle). Where they
+// are more than the buffer holds (pixels far finer than the voxels) or a
+// corner is not in front of the source, the angle's pixels are read from
+// memory, each with its own bounds.
+//
+// Bound: LDS reads (two of 8 bytes per voxel and angle) and vector ALU issue
+// (12 instructions and the setup). A 16-byte gather from row-paired memory
+// took 16 cycles of the L1 port per wave: 512^3, 720 angles, 512 x 768
+// pixels 49.0 ms; 39.7 ms so.
+//
+// ZC voxels per column; staged are at most SP columns (the pitch) and SR rows.
+// 32 voxels share a set-up better than 16 (39.7 and 42.0 ms); detectors with
+// pixels finer than about a voxel take 8 and larger pieces.
+constexpr int FDK_T = 16;
 
-__global__ void __launch_bounds__(FDK_BX *FDK_BY)
+template <int ZC, int SP, int SR>
+__global__ void __launch_bounds__(FDK_T *FDK_T)
 fdk_bp_upright(const FdkAngle *__restrict__ angles, int n_angles, int rows, int cols,
                const float *__restrict__ q, float *__restrict__ vol, int nx, int ny, int nz,
                double lo_x, double lo_y, double lo_z, double h_x, double h_y, double h_z, int additive)
 {
-    const int x = blockIdx.x * FDK_BX + threadIdx.x;
-    const int y = blockIdx.y * FDK_BY + threadIdx.y;
-    const int z0 = blockIdx.z * FDK_ZC;
-    const bool active = x < nx && y < ny;  // every thread takes part in the barriers
-    const double X = lo_x + (x + 0.5) * h_x, Y = lo_y + (y + 0.5) * h_y, Z0 = lo_z + (z0 + 0.5) * h_z;
-    // the row-paired filtered projections are addressed with 32-bit byte offsets (< 4 GiB)
-    const uint32_t rbytes = (uint32_t)n_angles * (uint32_t)cols * 8u;
-    const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
-        (void *)q, (short)0, (int)(rbytes * (uint32_t)rows), 0x00020000);
-    float acc[FDK_ZC];
+    constexpr int THREADS = FDK_T * FDK_T, LOADS = (SP * SR + THREADS - 1) / THREADS;
+    __shared__ float pixels[2][LOADS * THREADS];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int x0 = blockIdx.x * FDK_T, y0 = blockIdx.y * FDK_T, z0 = blockIdx.z * ZC;
+    const int x = x0 + (tid & (FDK_T - 1)), y = y0 + tid / FDK_T;
+    // (threads past the volume repeat its last column: positions stay between the corners')
+    const double X = lo_x + (min(x, nx - 1) + 0.5) * h_x, Y = lo_y + (min(y, ny - 1) + 0.5) * h_y;
+    const double Z0 = lo_z + (z0 + 0.5) * h_z;
+    float acc[ZC];
 #pragma unroll
-    for (int k = 0; k < FDK_ZC; ++k) acc[k] = 0.0f;
+    for (int k = 0; k < ZC; ++k) acc[k] = 0.0f;
+    // lane 8 e + c: corner c of the block at angle a0 + e, then the angle's first
+    // staged column and row and their numbers (0 columns: not staged)
+    int first_j = 0, first_i = 0, wide = 0, high = 0;
+    auto corners = [&](int a0) {
+        const FdkAngle &A = angles[min(a0 + (lane >> 3), n_angles - 1)];
+        const double cx = lo_x + (x0 + (lane & 1 ? FDK_T - 1 : 0) + 0.5) * h_x;
+        const double cy = lo_y + (y0 + (lane & 2 ? FDK_T - 1 : 0) + 0.5) * h_y;
+        const double cz = lo_z + (z0 + (lane & 4 ? ZC - 1 : 0) + 0.5) * h_z;
+        const double wx = cx - A.s[0], wy = cy - A.s[1], wz = cz - A.s[2];
+        const double den = wx * A.n[0] + wy * A.n[1];
+        int bad = !(den > 1e-6 * A.D);
+        const double lam = bad ? 0.0 : A.D / den;
+        double j_lo = A.cj + lam * (wx * A.Bj[0] + wy * A.Bj[1]);
+        double i_lo = A.ci + lam * (wx * A.Bi[0] + wy * A.Bi[1] + wz * A.Bi[2]);
+        double j_hi = j_lo, i_hi = i_lo;
+#pragma unroll
+        for (int d = 1; d < 8; d *= 2) {
+            j_lo = fmin(j_lo, __shfl_xor(j_lo, d, 64));
+            j_hi = fmax(j_hi, __shfl_xor(j_hi, d, 64));
+            i_lo = fmin(i_lo, __shfl_xor(i_lo, d, 64));
+            i_hi = fmax(i_hi, __shfl_xor(i_hi, d, 64));
+            bad |= __shfl_xor(bad, d, 64);
+        }
+        // (the margins exceed the rounding of the voxels' positions, FP64 and FP32)
+        bad |= !(j_hi - j_lo < SP - 3.0 && i_hi - i_lo < SR - 3.0 && fabs(j_lo) < 1e8 && fabs(i_lo) < 1e8);
+        first_j = bad ? 0 : (int)floor(j_lo - 1e-6);
+        first_i = bad ? 0 : (int)floor(i_lo - 1e-3);
+        wide = bad ? 0 : (int)floor(j_hi + 1e-6) + 2 - first_j;
+        high = bad ? 0 : (int)floor(i_hi + 1e-3) + 2 - first_i;
+    };
+    float next[LOADS];
+    int count = 0;
+    // pixel e = (row e / SP, column e % SP) of the staged ones of angle a
+    auto load = [&](int a) {
+        const int e8 = (a & 7) * 8;
+        const int fj = __builtin_amdgcn_readlane(first_j, e8), fi = __builtin_amdgcn_readlane(first_i, e8);
+        const int w = __builtin_amdgcn_readlane(wide, e8), h = __builtin_amdgcn_readlane(high, e8);
+        const float *src = q + (int64_t)a * rows * cols;
+        count = w ? h * SP : 0;
+#pragma unroll
+        for (int l = 0; l < LOADS; ++l) {
+            if (l * THREADS >= count) break;
+            const int e = l * THREADS + tid, r = e / SP, c = e - r * SP, i = fi + r, j = fj + c;
+            next[l] = 0.0f;
+            if (c < w && (unsigned)i < (unsigned)rows && (unsigned)j < (unsigned)cols) next[l] = src[i * cols + j];
+        }
+    };
+    corners(0);
+    load(0);
     for (int a = 0; a < n_angles; ++a) {
-        auto one_angle = [&]() {
-            const FdkAngle &A = angles[a];
-            const double wx = X - A.s[0], wy = Y - A.s[1], wz = Z0 - A.s[2];
-            const double den = wx * A.n[0] + wy * A.n[1];
-            if (!(den > 0.0)) return;
-            const double lam = A.D * rcp64(den);
-            const double fj = A.cj + lam * (wx * A.Bj[0] + wy * A.Bj[1]);
-            if (!(fj > -1.0 && fj < (double)cols)) return;
-            // rows relative to the first voxel's, floor(fi): FP32 holds their fractions
-            const double fi = fmin(fmax(A.ci + lam * (wx * A.Bi[0] + wy * A.Bi[1] + wz * A.Bi[2]), -1e9), 1e9);
-            const int ib = (int)floor(fi);
-            const float fi0 = (float)(fi - ib);
-            const float dfi = (float)(lam * h_z * A.Bi[2]);
-            const float wgt = (float)(A.half_dbeta * lam * lam);
-            const double fj0 = floor(fj);
-            const int j0 = (int)fj0;
-            const float wj = (float)(fj - fj0);
-            // columns (jb, jb + 1), jb = j0 clamped into [0, cols - 2], read as one
-            // 8-byte pair; the weights of columns outside the detector are 0
-            const int jb = min(max(j0, 0), max(cols - 2, 0));
-            float ca, cb;
-            if (j0 == jb) {
-                ca = 1.0f - wj;
-                cb = j0 + 1 < cols ? wj : 0.0f;
-            } else if (j0 < jb) {  // j0 = -1: only column 0 = jb, weight wj
-                ca = wj;
-                cb = 0.0f;
-            } else {               // j0 = cols - 1: only column jb + 1, weight 1 - wj
-                ca = 0.0f;
-                cb = 1.0f - wj;
-            }
-            // q is row-paired: the 16 bytes at (row i, column jb) are
-            // q[i][jb], q[i+1][jb], q[i][jb+1], q[i+1][jb+1]
-            const uint32_t cboff = ((uint32_t)a * (uint32_t)cols + (uint32_t)jb) * 8u;
-    #pragma unroll
-            for (int k = 0; k < FDK_ZC; ++k) {
-                const float fi = fmaf((float)k, dfi, fi0);
-                const float fi0f = floorf(fi);
-                const int i0 = ib + (int)fi0f;
-                const float wi = fi - fi0f;
-                // rows i0, i0 + 1 from the element of row max(i0, 0) (inside the
-                // buffer); for i0 = -1 that element's first row is row i0 + 1
-                const uint32_t o = (uint32_t)min(max(i0, 0), rows - 1) * rbytes + cboff;
-                const float x0 = bload(rs, o), y0 = bload(rs, o + 4u);
-                const float x1 = bload(rs, o + 8u), y1 = bload(rs, o + 12u);
-                const float first = fmaf(ca, x0, cb * x1), second = fmaf(ca, y0, cb * y1);
-                const bool in = i0 >= 0 && i0 < rows;
-                const float top = in ? first : 0.0f;
-                const float bot = in ? second : (i0 == -1 ? first : 0.0f);
+        float *buf = pixels[a & 1];
+        const int e8 = (a & 7) * 8;
+        const bool staged = __builtin_amdgcn_readlane(wide, e8) > 0;
+        const int fj0 = __builtin_amdgcn_readlane(first_j, e8), fi0 = __builtin_amdgcn_readlane(first_i, e8);
+#pragma unroll
+        for (int l = 0; l < LOADS; ++l) {
+            if (l * THREADS >= count) break;
+            buf[l * THREADS + tid] = next[l];
+        }
+        __syncthreads();
+        if (a + 1 < n_angles) {
+            if (((a + 1) & 7) == 0) corners(a + 1);
+            load(a + 1);
+        }
+        const FdkAngle &A = angles[a];
+        const double wx = X - A.s[0], wy = Y - A.s[1], wz = Z0 - A.s[2];
+        const double den = wx * A.n[0] + wy * A.n[1];
+        const double lam = A.D * rcp64(den);
+        const double fj = A.cj + lam * (wx * A.Bj[0] + wy * A.Bj[1]) - fj0;
+        const double fi = A.ci + lam * (wx * A.Bi[0] + wy * A.Bi[1] + wz * A.Bi[2]) - fi0;
+        const float dfi = (float)(lam * h_z * A.Bi[2]), wgt = (float)(A.half_dbeta * lam * lam);
+        if (staged) {
+            const double fl = floor(fj);
+            const float cb = (float)(fj - fl), ca = 1.0f - cb, f0 = (float)fi;
+            const float *col = buf + (int)fl;
+#pragma unroll
+            for (int k = 0; k < ZC; ++k) {
+                const float f = fmaf((float)k, dfi, f0), ff = floorf(f), wi = f - ff;
+                const float *p = col + (int)__umul24((uint32_t)(int)ff, SP);
+                const float top = fmaf(ca, p[0], cb * p[1]), bot = fmaf(ca, p[SP], cb * p[SP + 1]);
                 acc[k] = fmaf(wgt, fmaf(wi, bot - top, top), acc[k]);
             }
-        };
-        if (active) one_angle();
-        // The block's waves stay at one angle together: their voxels read
-        // neighbouring pixels of the same filtered projection, which the
-        // waves then share in L1 (17 % faster at 512^3 than free-running).
-        __syncthreads();
-
+        } else if (x < nx && y < ny && den > 0.0 && fj > -1.0 && fj < (double)cols) {
+            const double fl = floor(fj);
+            const int j0 = (int)fl;
+            const float wj = (float)(fj - fl);
+            const float *src = q + (int64_t)a * rows * cols;
+            const bool j_lo = j0 >= 0, j_hi = j0 + 1 < cols;
+            const double step = lam * h_z * A.Bi[2];
+            for (int k = 0; k < ZC; ++k) {
+                const double f = fma((double)k, step, fi), ff = floor(f);
+                if (!(f > -1.0 && f < (double)rows)) continue;
+                const int i0 = (int)ff;
+                const float wi = (float)(f - ff);
+                const float *r0 = src + (int64_t)i0 * cols + j0, *r1 = r0 + cols;
+                const bool i_lo = i0 >= 0, i_hi = i0 + 1 < rows;
+                const float v00 = (i_lo && j_lo) ? r0[0] : 0.0f, v01 = (i_lo && j_hi) ? r0[1] : 0.0f;
+                const float v10 = (i_hi && j_lo) ? r1[0] : 0.0f, v11 = (i_hi && j_hi) ? r1[1] : 0.0f;
+                const float top = fmaf(1.0f - wj, v00, wj * v01), bot = fmaf(1.0f - wj, v10, wj * v11);
+                const float t = wgt * fmaf(wi, bot - top, top);
+#pragma unroll
+                for (int e = 0; e < ZC; ++e)
+                    if (e == k) acc[e] += t;
+            }
+        }
     }
 #pragma unroll
-    for (int k = 0; k < FDK_ZC; ++k) {
+    for (int k = 0; k < ZC; ++k) {
         const int z = z0 + k;
-        if (active && z < nz) {
+        if (x < nx && y < ny && z < nz) {
             float *o = vol + ((int64_t)z * ny + y) * nx + x;
             *o = additive ? *o + acc[k] : acc[k];
         }
     }
 }
+
+using FdkKernel = void (*)(const FdkAngle *, int, int, int, const float *, float *, int, int, int, double, double, double,
+                           double, double, double, int);
+constexpr int FDK_ZC = 32, FDK_SP = 41, FDK_SR = 62, FDK_FINE_ZC = 8, FDK_FINE_SP = 83, FDK_FINE_SR = 58;
 
 }  // namespace tsx

@@ -207,6 +207,7 @@ struct tsx_plan {
     std::vector<FdkAngle> fdk_host;
     FdkAngle *fdk_dev = nullptr;
     const float *fdk_factors = nullptr;  // the ramp filter's factors (after fdk_dev's entries)
+    bool fdk_fine = false;     // ... and the pixels are so fine that its kernel takes short columns
     bool fdk_upright = false;  // every angle: v parallel to z, normal perpendicular to z
     double vlo[3] = {0, 0, 0}, vh[3] = {0, 0, 0};
 };
@@ -366,6 +367,16 @@ void build_fdk(const tsx_geometry *g, tsx_plan *p)
             db = 0.5 * std::fabs(beta[a + 1] - beta[a - 1]);
         F.half_dbeta = 0.5 * db;
         F.inv_du = 1.0 / std::sqrt(dot(U, U));
+        // pixels that a block's 16 x 16 columns of FDK_ZC voxels span, with the
+        // voxels nearest to the source (corners of the volume) as large as they get
+        double near = F.D;
+        for (int k = 0; k < 4; ++k)
+            near = std::min(near, ((k & 1 ? g->window_max[0] : g->window_min[0]) - s[0]) * n[0] +
+                                      ((k & 2 ? g->window_max[1] : g->window_min[1]) - s[1]) * n[1]);
+        const double most = near > 0.0 ? F.D / near : 1e9;
+        const double across = (FDK_T - 1) * (std::fabs(Bj[0]) * p->vh[0] + std::fabs(Bj[1]) * p->vh[1]);
+        const double along = (FDK_ZC - 1) * std::fabs(Bi[2]) * p->vh[2];
+        if (most * across > FDK_SP - 6 || 1.1 * most * along > FDK_SR - 6) p->fdk_fine = true;
     }
 }
 
@@ -2624,9 +2635,9 @@ tsx_geometry refined_geometry(const tsx_geometry *g, std::vector<double> &vec)
     return fg;
 }
 
-// The upright FDK backprojector reads row-paired filtered projections (8 bytes
-// per pixel, addressed with 32-bit offsets); the general one plain ones.
-bool fdk_paired(const tsx_plan *p)
+// The upright FDK backprojector, where its kernel takes the plan. (Its workspace
+// stays at 8 bytes per pixel, as callers size their buffers, of which it uses 4.)
+bool fdk_staged(const tsx_plan *p)
 {
     return p->fdk_upright && !force_general() && p->cols >= 2 &&
            (int64_t)p->rows * p->n_angles * p->cols * 8 < ((int64_t)1 << 32);
@@ -2845,7 +2856,7 @@ int tsx_plan_info_get(const tsx_plan *p, tsx_plan_info *info)
 int tsx_fdk_workspace_size(const tsx_plan *p, int64_t *bytes)
 {
     if (!p || !bytes) return fail(TSX_ERR_INVALID_ARGUMENT, "plan and bytes must not be NULL");
-    *bytes = (int64_t)p->rows * p->n_angles * p->cols * (fdk_paired(p) ? 8 : 4);
+    *bytes = (int64_t)p->rows * p->n_angles * p->cols * (fdk_staged(p) ? 8 : 4);
     return TSX_OK;
 }
 
@@ -2869,7 +2880,7 @@ int tsx_fdk(const tsx_plan *p, float *vol, const float *proj, int additive, void
     if (!dg.ok) return fail(TSX_ERR_HIP, "cannot select the plan's device");
     EntryTimer entry_timer_("tsx_fdk", stream);
     hipStream_t s = (hipStream_t)stream;
-    const bool upright = fdk_paired(p);
+    const bool upright = fdk_staged(p);
     const int64_t need = (int64_t)p->rows * p->n_angles * p->cols * (upright ? 8 : 4);
     Scratch owned;
     void *wptr = nullptr;
@@ -2883,12 +2894,16 @@ int tsx_fdk(const tsx_plan *p, float *vol, const float *proj, int additive, void
                        q, upright ? 1 : 0);
     TSX_HIP_CHECK(hipGetLastError());
     const unsigned gx = (unsigned)((p->nx + FDK_BX - 1) / FDK_BX), gy = (unsigned)((p->ny + FDK_BY - 1) / FDK_BY);
-    if (upright)
-        hipLaunchKernelGGL(fdk_bp_upright, dim3(gx, gy, (unsigned)((p->nz + FDK_ZC - 1) / FDK_ZC)),
-                           dim3(FDK_BX, FDK_BY), 0, s, p->fdk_dev, p->n_angles, p->rows, p->cols, q, vol,
+    if (upright) {
+        const int zc = p->fdk_fine ? FDK_FINE_ZC : FDK_ZC;
+        const FdkKernel kernel = p->fdk_fine ? fdk_bp_upright<FDK_FINE_ZC, FDK_FINE_SP, FDK_FINE_SR>
+                                             : fdk_bp_upright<FDK_ZC, FDK_SP, FDK_SR>;
+        hipLaunchKernelGGL(kernel, dim3((unsigned)((p->nx + FDK_T - 1) / FDK_T), (unsigned)((p->ny + FDK_T - 1) / FDK_T),
+                                        (unsigned)((p->nz + zc - 1) / zc)),
+                           dim3(FDK_T * FDK_T), 0, s, p->fdk_dev, p->n_angles, p->rows, p->cols, q, vol,
                            p->nx, p->ny, p->nz, p->vlo[0], p->vlo[1], p->vlo[2], p->vh[0], p->vh[1],
                            p->vh[2], additive ? 1 : 0);
-    else
+    } else
         hipLaunchKernelGGL(fdk_bp, dim3(gx, gy, (unsigned)p->nz), dim3(FDK_BX, FDK_BY), 0, s, p->fdk_dev,
                            p->n_angles, p->rows, p->cols, q, vol, p->nx, p->ny, p->nz, p->vlo[0],
                            p->vlo[1], p->vlo[2], p->vh[0], p->vh[1], p->vh[2], additive ? 1 : 0);
