@@ -2496,13 +2496,14 @@ int autotune(tsx_plan *p, hipStream_t stream)
     }
     if (p->bp_separable && !force_general() && !bp_flat_used) {
         float best_ms = 1e30f;
-        for (int bz : {32, 24, 16}) {
+        // (a depth replaces an earlier one where it is faster by more than the trials scatter)
+        for (int bz : {32, 16, 24}) {
             sub.bp_bz = bz;
             float ms = 0.0f;
             int rc = time_launches([&] { return launch_bp(&sub, vol, 0, proj, 0, 1, ep, stream); },
                                    stream, t.e0, t.e1, 2, &ms);
             if (rc) return rc;
-            if (ms < best_ms) {
+            if (ms < 0.96f * best_ms) {
                 best_ms = ms;
                 best.bp_bz = bz;
             }
@@ -2895,8 +2896,11 @@ int tsx_fdk(const tsx_plan *p, float *vol, const float *proj, int additive, void
     TSX_HIP_CHECK(hipGetLastError());
     const unsigned gx = (unsigned)((p->nx + FDK_BX - 1) / FDK_BX), gy = (unsigned)((p->ny + FDK_BY - 1) / FDK_BY);
     if (upright) {
-        const int zc = p->fdk_fine ? FDK_FINE_ZC : FDK_ZC;
-        const FdkKernel kernel = p->fdk_fine ? fdk_bp_upright<FDK_FINE_ZC, FDK_FINE_SP, FDK_FINE_SR>
+        // (short columns also where long ones leave CUs idle: 100^3, 120 angles 0.20 against 0.28 ms)
+        const int64_t tiles = (int64_t)((p->nx + FDK_T - 1) / FDK_T) * ((p->ny + FDK_T - 1) / FDK_T);
+        const bool fine = p->fdk_fine || tiles * ((p->nz + FDK_ZC - 1) / FDK_ZC) < 256;
+        const int zc = fine ? FDK_FINE_ZC : FDK_ZC;
+        const FdkKernel kernel = fine ? fdk_bp_upright<FDK_FINE_ZC, FDK_FINE_SP, FDK_FINE_SR>
                                              : fdk_bp_upright<FDK_ZC, FDK_SP, FDK_SR>;
         hipLaunchKernelGGL(kernel, dim3((unsigned)((p->nx + FDK_T - 1) / FDK_T), (unsigned)((p->ny + FDK_T - 1) / FDK_T),
                                         (unsigned)((p->nz + zc - 1) / zc)),
