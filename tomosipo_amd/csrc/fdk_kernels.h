@@ -68,7 +68,7 @@ constexpr int fdk_filter_floats(int nt) { return 2 * (FDK_ROWS * (32 * nt + 4) +
 //
 // Bound: the matrix cores' FP32 rate (157 TFLOP/s; 2 cols FLOP per output,
 // half of the full product), with three blocks per CU at 768 columns so that
-// one loads while another multiplies. 512 x 720 rows of 768 columns: FIGURE ms (the sum
+// one loads while another multiplies. 512 x 720 rows of 768 columns: 3.0 ms (the sum
 // of factor (c[j - m] + c[j + m] - 2 c[j]) on the vector ALUs, register-tiled:
 // 10.4 ms; in this form there: 9.5 ms).
 template <int NT>

@@ -2089,6 +2089,14 @@ int multi_fp(const tsx_plan *const *plans, const float *const *vols, float *cons
     return flush();
 }
 
+// Bricks of a fused backprojection below which instances in angle parts run
+// alone: it runs a brick's parts in turn, so that fewer than about four blocks
+// per CU leave it idle, while their own launches run the parts in separate
+// blocks (two 105^3 cones beside two parallel scans: the pass 386 and 283 us
+// with its forward projections; eight scans of 64^3 to 128^3, 880 bricks: 1.35
+// and 1.25 ms). Either order of a part's sums gives the same bits.
+constexpr int64_t MULTI_BP_BRICKS = 1024;
+
 int multi_bp(const tsx_plan *const *plans, float *const *vols, const float *const *projs,
              const Epilogue *eps, int n, void *wsp, int64_t ws_bytes, hipStream_t stream)
 {
@@ -2164,6 +2172,15 @@ int multi_bp(const tsx_plan *const *plans, float *const *vols, const float *cons
         const int rc = fb.backward(f, plans[k]->flat_nc);
         if (rc) return rc;
     }
+    // Separable instances in angle parts whose bricks together are few take
+    // their own launches, which run the parts in separate blocks.
+    const auto bricks_of = [](const tsx_plan *p) {
+        const int bz = bp_brick_z_of(p);
+        return (int64_t)((p->nx + BR - 1) / BR) * ((p->ny + BR - 1) / BR) * ((p->nz + bz - 1) / bz);
+    };
+    int64_t in_parts = 0;
+    for (int k = 0; k < n; ++k)
+        if (!taken[k] && bp_parts_of(plans[k]) > 1) in_parts += bricks_of(plans[k]);
     for (size_t pass = 0; pass < keys.size(); ++pass)
     for (int k = 0; k < n; ++k) {
         if (taken[k]) continue;
@@ -2182,7 +2199,7 @@ int multi_bp(const tsx_plan *const *plans, float *const *vols, const float *cons
         const int64_t tblocks = scale_job_blocks(job);
         const int64_t cap = max_blocks(BR * BR);
         if (!(fast && p->bp_separable && bp_chunk_of(p) == p->n_angles) || blocks > cap ||
-            tblocks > max_blocks(256) || flat_bp(p, 1).ok) {
+            tblocks > max_blocks(256) || flat_bp(p, 1).ok || (bp_parts_of(p) > 1 && in_parts < MULTI_BP_BRICKS)) {
             if (pass > 0) continue;  // (its own launch, in the first pass)
             int rc = launch_bp(p, vols[k], 0, projs[k], 0, 1, eps[k], stream, wptr ? (char *)wptr + woff : nullptr, wb);
             if (rc) return rc;
