@@ -91,6 +91,8 @@ def request_bytes(req):
     vol = 4 * s ** 3
     sino = 4 * s * req.n_angles * (3 * s // 2)
     pad = 8 * (s + 4) ** 2 * s * 2       # row-paired padded volume copies of the forward projector
+    if req.kind == "parallel":           # or the turned volume and its line sums (all angles within 64 MiB)
+        pad = max(pad, min(vol + sino, 1 << 26))
     ly = 4 * (s + 6) * req.n_angles * (3 * s // 2)  # length-weighted projections (padded rows)
     if req.op == "fp":
         return vol + sino + pad
