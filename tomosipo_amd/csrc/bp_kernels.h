@@ -31,6 +31,7 @@
 
 #include "tsx_plan.h"
 #include "fp_kernels.h"
+#include "tilted_box.h"
 
 namespace tsx {
 
@@ -280,8 +281,10 @@ __global__ void scale_by_length(const AngleParams *__restrict__ angles, int n_an
 // are largest at an end, so that one box size, from the two ends, serves all
 // of them. A pixel's weight takes its ray's in-slice offset, as in bp_general:
 // (dj A1j + di A1i) / (1 + dj fBj + di fBi) along c1, likewise along c2.
-// Angles stepping along z and voxels near the source's planes (W . N under 16
-// times its steps, |W_m| under 16) take the FP64 set-up for each voxel.
+// Angles stepping along z, voxels near the source's planes (W . N under 16
+// times its steps, |W_m| under 16) and positions or boxes beyond TILTED_REACH
+// take the FP64 set-up for each voxel and cut its box in FP64 (FAR: a
+// parallel scan has angles whose positions are; it has none else).
 //
 // Bound: vector ALU issue (1.2 per CU-cycle). 192^3 cone, 240 angles, 192 x
 // 288 tilted by 0.2 rad: 4.17 ms (103 instructions per 64 voxels and angle); with the set-up of every voxel in FP64 and
@@ -352,7 +355,7 @@ __device__ __forceinline__ float tilted_sum(__amdgpu_buffer_rsrc_t rs, const Til
     return sum;
 }
 
-template <bool CONE, int ZV>
+template <bool CONE, int ZV, bool FAR>
 __global__ void __launch_bounds__(BP_BX *BP_BY)
 bp_tilted(const AngleParams *__restrict__ angles, int n_angles, int rows, int cols, int nx, int ny, int nz,
           float *__restrict__ vol, int64_t vol_stride, const float *__restrict__ ly, int64_t ly_stride, Epilogue ep)
@@ -365,6 +368,7 @@ bp_tilted(const AngleParams *__restrict__ angles, int n_angles, int rows, int co
     ConstAngle *table = (ConstAngle *)angles;
     const float *entry = uniform_ptr(ly + (int64_t)b * ly_stride);
     const uint32_t bytes = (uint32_t)rows * (uint32_t)cols * 4u, pitch = (uint32_t)cols * 4u;
+    constexpr float REACH = (float)TILTED_REACH;
     float acc[ZV];
 #pragma unroll
     for (int k = 0; k < ZV; ++k) acc[k] = 0.0f;
@@ -374,10 +378,10 @@ bp_tilted(const AngleParams *__restrict__ angles, int n_angles, int rows, int co
         if (!CONE && !(A.par_b[0] >= 0.0f)) continue;  // singular map
         const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
             (void *)(entry + (int64_t)a * rows * cols), (short)0, (int)bytes, 0x00020000);
-        // FP64 set-up of the voxel z; false: no position
-        auto setup = [&](int z, TiltedVoxel &V) {
+        // FP64 position (cj, ci) of the voxel z and its map; false: no position
+        auto position = [&](int z, TiltedVoxel &V, double &cj, double &ci) {
             const double km = sel3(m, x, y, z), k1 = sel3(m == 2 ? 1 : 2, x, y, z), k2 = sel3(m == 0 ? 1 : 0, x, y, z);
-            double cj, ci;
+            cj = ci = 0.0;
             V.tj = V.ti = V.dn = V.W0 = V.W1 = V.W2 = 0.0f;
             if constexpr (CONE) {
                 const double W0 = km - A.S[0], W1 = k1 - A.S[1], W2 = k2 - A.S[2];
@@ -393,53 +397,57 @@ bp_tilted(const AngleParams *__restrict__ angles, int n_angles, int rows, int co
                 V.W0 = (float)W0;
                 V.W1 = (float)W1;
                 V.W2 = (float)W2;
-                if (dn == 0.0 || W0 == 0.0) return false;
+                return dn != 0.0 && W0 != 0.0;
             } else {
                 cj = fma(k2, A.par_c[3], fma(k1, A.par_c[2], fma(km, A.par_c[1], A.par_c[0])));
                 ci = fma(k2, A.par_c[7], fma(k1, A.par_c[6], fma(km, A.par_c[5], A.par_c[4])));
+                return true;
             }
-            const double fj = floor(fmin(fmax(cj, -1e9), 1e9)), fi = floor(fmin(fmax(ci, -1e9), 1e9));
-            V.j0 = (int)fj;
-            V.i0 = (int)fi;
-            V.pj = (float)(cj - fj);
-            V.pi = (float)(ci - fi);
-            return true;
+        };
+        // the position relative to pixel (j0, i0)
+        auto relative = [&](TiltedVoxel &V, double cj, double ci, int j0, int i0) {
+            V.j0 = j0;
+            V.i0 = i0;
+            V.pj = (float)(cj - (double)j0);
+            V.pi = (float)(ci - (double)i0);
         };
         // the box of half-widths (mj, mi) around the position, cut to the detector
         auto box = [&](const TiltedVoxel &V, float mj, float mi, TiltedMap &T) {
-            T.jl = -min(floor_to_int(mj - T.pj), V.j0);
-            T.jh = min(floor_to_int(T.pj + mj), cols - 1 - V.j0);
-            T.il = -min(floor_to_int(mi - T.pi), V.i0);
-            T.ih = min(floor_to_int(T.pi + mi), rows - 1 - V.i0);
+            const PixelRange j = tilted_near_pixels(V.j0, floor_to_int(mj - T.pj), floor_to_int(T.pj + mj), cols);
+            const PixelRange i = tilted_near_pixels(V.i0, floor_to_int(mi - T.pi), floor_to_int(T.pi + mi), rows);
+            T.jl = j.lo;
+            T.jh = j.hi;
+            T.il = i.lo;
+            T.ih = i.hi;
         };
         // (offsets of pixels far outside the detector wrap around; their boxes are empty)
         auto origin = [&](const TiltedVoxel &V) { return (uint32_t)V.i0 * pitch + (uint32_t)V.j0 * 4u; };
         TiltedVoxel V;
-        const bool ok = setup(z0, V);
-        const bool near = CONE && (!ok || m == 2 || !(fabsf(V.dn) > A.freach) || !(fabsf(V.W0) > 16.0f));
+        double cj, ci;
+        const bool ok = position(z0, V, cj, ci), reached = CONE ? tilted_in_reach(cj, ci) : !FAR || A.freach <= REACH;
+        // (a position out of reach: any, as the box is cut in FP64 then)
+        relative(V, cj, ci, reached ? (int)floor(cj) : 0, reached ? (int)floor(ci) : 0);
         TiltedMap T;
-        if (!CONE) {
-            T.A1j = A.par_a[0];
-            T.A1i = A.par_a[1];
-            T.A2j = A.par_a[2];
-            T.A2i = A.par_a[3];
-            T.fBj = T.fBi = 0.0f;
+        bool apart = ok && reached;
+        float mj = 0.0f, mi = 0.0f;  // half-widths of the boxes
+        float gj, gi;                // the position's step per voxel, cone: (B_e - N_e (W . B) / (W . N))
+        if constexpr (!CONE) {
             const int zc = m == 2 ? 0 : 1;
-            const float gj = A.fBj[zc], gi = A.fBi[zc], mj = A.par_b[0] + 1e-3f, mi = A.par_b[1] + 1e-3f;
-            const uint32_t o = origin(V);
-#pragma unroll
-            for (int k = 0; k < ZV; ++k) {
-                T.pj = fmaf((float)k, gj, V.pj);
-                T.pi = fmaf((float)k, gi, V.pi);
-                box(V, mj, mi, T);
-                acc[k] += tilted_sum<CONE>(rs, T, o, pitch);
-            }
-        } else if (__builtin_amdgcn_ballot_w64(near) == 0) {
-            // (m = 0 or 1: the voxels differ along c1)
+            gj = A.fBj[zc];
+            gi = A.fBi[zc];
+            mj = A.par_b[0] + 1e-3f;
+            mi = A.par_b[1] + 1e-3f;
+        } else if (m == 2) {
+            apart = false;
+            gj = gi = 0.0f;
+        } else {
+            // (the voxels differ along c1)
             const float Nz = A.fN[1];
-            const float gj = fmaf(-Nz, V.tj, A.fBj[1]), gi = fmaf(-Nz, V.ti, A.fBi[1]);
+            gj = fmaf(-Nz, V.tj, A.fBj[1]);
+            gi = fmaf(-Nz, V.ti, A.fBi[1]);
+            apart = apart && fabsf(V.dn) > A.freach && fabsf(V.W0) > 16.0f;
             // box size from the two ends
-            float mj = 0.0f, mi = 0.0f, s = 0.0f;
+            float s = 0.0f;
 #pragma unroll
             for (int e = 0; e < 2; ++e) {
                 if (e == 1 && ZV == 1) break;
@@ -455,56 +463,83 @@ bp_tilted(const AngleParams *__restrict__ angles, int n_angles, int rows, int co
             s *= fmaf(1.1f * A.fspan, s, 1.0f);  // 1 / (1 - c) <= 1 + 1.1 c for c <= 1 / 16
             mj = fmaf(mj, s, 1e-3f);
             mi = fmaf(mi, s, 1e-3f);
-            const float iW0 = __builtin_amdgcn_rcpf(V.W0), r1 = V.W1 * iW0, r2 = V.W2 * iW0;
-            const float uj = A.fU[0] * iW0, ui = A.fV[0] * iW0;
-            const float c1j = fmaf(-r1, A.fU[0], A.fU[1]), c1i = fmaf(-r1, A.fV[0], A.fV[1]);
-            const float c2j = fmaf(-r2, A.fU[0], A.fU[2]), c2i = fmaf(-r2, A.fV[0], A.fV[2]);
+        }
+        if (CONE ? __builtin_amdgcn_ballot_w64(!(apart && fmaxf(mj, mi) <= REACH)) == 0 : apart) {
             const uint32_t o = origin(V);
+            if constexpr (!CONE) {
+                T.A1j = A.par_a[0];
+                T.A1i = A.par_a[1];
+                T.A2j = A.par_a[2];
+                T.A2i = A.par_a[3];
+                T.fBj = T.fBi = 0.0f;
 #pragma unroll
-            for (int k = 0; k < ZV; ++k) {
-                const float fk = (float)k, dn = k ? fmaf(fk, Nz, V.dn) : V.dn, Tc = dn * A.finv_kappa;
-                T.pj = V.pj;
-                T.pi = V.pi;
-                if (k) {
-                    const float kl = fk * A.fkappa * __builtin_amdgcn_rcpf(dn);
-                    T.pj = fmaf(kl, gj, V.pj);
-                    T.pi = fmaf(kl, gi, V.pi);
+                for (int k = 0; k < ZV; ++k) {
+                    T.pj = fmaf((float)k, gj, V.pj);
+                    T.pi = fmaf((float)k, gi, V.pi);
+                    box(V, mj, mi, T);
+                    acc[k] += tilted_sum<CONE>(rs, T, o, pitch);
                 }
-                T.A1j = Tc * fmaf(-fk, uj, c1j);
-                T.A1i = Tc * fmaf(-fk, ui, c1i);
-                T.A2j = Tc * c2j;
-                T.A2i = Tc * c2i;
-                T.fBj = Tc * uj;
-                T.fBi = Tc * ui;
-                box(V, mj, mi, T);
-                acc[k] += tilted_sum<CONE>(rs, T, o, pitch);
+            } else {
+                const float Nz = A.fN[1];
+                const float iW0 = __builtin_amdgcn_rcpf(V.W0), r1 = V.W1 * iW0, r2 = V.W2 * iW0;
+                const float uj = A.fU[0] * iW0, ui = A.fV[0] * iW0;
+                const float c1j = fmaf(-r1, A.fU[0], A.fU[1]), c1i = fmaf(-r1, A.fV[0], A.fV[1]);
+                const float c2j = fmaf(-r2, A.fU[0], A.fU[2]), c2i = fmaf(-r2, A.fV[0], A.fV[2]);
+#pragma unroll
+                for (int k = 0; k < ZV; ++k) {
+                    const float fk = (float)k, dn = k ? fmaf(fk, Nz, V.dn) : V.dn, Tc = dn * A.finv_kappa;
+                    T.pj = V.pj;
+                    T.pi = V.pi;
+                    if (k) {
+                        const float kl = fk * A.fkappa * __builtin_amdgcn_rcpf(dn);
+                        T.pj = fmaf(kl, gj, V.pj);
+                        T.pi = fmaf(kl, gi, V.pi);
+                    }
+                    T.A1j = Tc * fmaf(-fk, uj, c1j);
+                    T.A1i = Tc * fmaf(-fk, ui, c1i);
+                    T.A2j = Tc * c2j;
+                    T.A2i = Tc * c2i;
+                    T.fBj = Tc * uj;
+                    T.fBi = Tc * ui;
+                    box(V, mj, mi, T);
+                    acc[k] += tilted_sum<CONE>(rs, T, o, pitch);
+                }
             }
-        } else {
+        } else if constexpr (FAR) {
 #pragma unroll 1
             for (int k = 0; k < ZV; ++k) {
                 float sum = 0.0f;
-                if (setup(z0 + k, V)) {
-                    const float lam = A.fkappa * __builtin_amdgcn_rcpf(V.dn), c = A.fspan * fabsf(lam);
-                    const float M00 = fmaf(-A.fN[1], V.tj, A.fBj[1]), M01 = fmaf(-A.fN[2], V.tj, A.fBj[2]);
-                    const float M10 = fmaf(-A.fN[1], V.ti, A.fBi[1]), M11 = fmaf(-A.fN[2], V.ti, A.fBi[2]);
-                    const float s = fabsf(lam) * __builtin_amdgcn_rcpf(1.0f - c);
-                    const float iW0 = __builtin_amdgcn_rcpf(V.W0), r1 = V.W1 * iW0, r2 = V.W2 * iW0;
-                    const float Tc = V.dn * A.finv_kappa, TW = Tc * iW0;
+                if (z0 + k < nz && position(z0 + k, V, cj, ci)) {
+                    if constexpr (!CONE) {
+                        T.A1j = A.par_a[0];
+                        T.A1i = A.par_a[1];
+                        T.A2j = A.par_a[2];
+                        T.A2i = A.par_a[3];
+                        T.fBj = T.fBi = 0.0f;
+                    } else {
+                        const float lam = A.fkappa * __builtin_amdgcn_rcpf(V.dn), c = A.fspan * fabsf(lam);
+                        const float M00 = fmaf(-A.fN[1], V.tj, A.fBj[1]), M01 = fmaf(-A.fN[2], V.tj, A.fBj[2]);
+                        const float M10 = fmaf(-A.fN[1], V.ti, A.fBi[1]), M11 = fmaf(-A.fN[2], V.ti, A.fBi[2]);
+                        const float s = fabsf(lam) * __builtin_amdgcn_rcpf(1.0f - c);
+                        const float iW0 = __builtin_amdgcn_rcpf(V.W0), r1 = V.W1 * iW0, r2 = V.W2 * iW0;
+                        const float Tc = V.dn * A.finv_kappa, TW = Tc * iW0;
+                        T.A1j = Tc * fmaf(-r1, A.fU[0], A.fU[1]);
+                        T.A1i = Tc * fmaf(-r1, A.fV[0], A.fV[1]);
+                        T.A2j = Tc * fmaf(-r2, A.fU[0], A.fU[2]);
+                        T.A2i = Tc * fmaf(-r2, A.fV[0], A.fV[2]);
+                        T.fBj = A.fU[0] * TW;
+                        T.fBi = A.fV[0] * TW;
+                        const bool bounded = c < 1.0f - 1e-6f;
+                        mj = bounded ? fmaf(fabsf(M00) + fabsf(M01), s, 1e-3f) : INFINITY;
+                        mi = bounded ? fmaf(fabsf(M10) + fabsf(M11), s, 1e-3f) : INFINITY;
+                    }
+                    const PixelRange j = tilted_pixels(cj, mj, cols), i = tilted_pixels(ci, mi, rows);
+                    relative(V, cj, ci, j.lo, i.lo);
                     T.pj = V.pj;
                     T.pi = V.pi;
-                    T.A1j = Tc * fmaf(-r1, A.fU[0], A.fU[1]);
-                    T.A1i = Tc * fmaf(-r1, A.fV[0], A.fV[1]);
-                    T.A2j = Tc * fmaf(-r2, A.fU[0], A.fU[2]);
-                    T.A2i = Tc * fmaf(-r2, A.fV[0], A.fV[2]);
-                    T.fBj = A.fU[0] * TW;
-                    T.fBi = A.fV[0] * TW;
-                    box(V, fmaf(fabsf(M00) + fabsf(M01), s, 1e-3f), fmaf(fabsf(M10) + fabsf(M11), s, 1e-3f), T);
-                    if (!(c < 1.0f - 1e-6f)) {  // an unbounded image
-                        T.jl = -V.j0;
-                        T.jh = cols - 1 - V.j0;
-                        T.il = -V.i0;
-                        T.ih = rows - 1 - V.i0;
-                    }
+                    T.jl = T.il = 0;
+                    T.jh = j.hi - j.lo;
+                    T.ih = i.hi - i.lo;
                     sum = tilted_sum<CONE>(rs, T, origin(V), pitch);
                 }
 #pragma unroll

@@ -300,6 +300,21 @@ void parallel_map(AngleParams &A)
     A.par_b[1] = (float)((std::fabs(a2j) + std::fabs(a1j)) / std::fabs(det));
 }
 
+// The largest of a parallel scan's detector positions over the voxels of the
+// volume (and those beyond its end that a block of bp_tilted also forms), of
+// their steps per voxel and of the half-widths of their boxes.
+float parallel_reach(const AngleParams &A, const tsx_geometry *g)
+{
+    double most = std::max((double)A.par_b[0], (double)A.par_b[1]);
+    const double n = 64.0 + std::max(g->grid_col_count, std::max(g->grid_row_count, g->grid_slice_count));
+    for (int r = 0; r < 8; r += 4) {
+        const double *c = A.par_c + r;
+        const double v = std::fabs(c[0]) + n * (std::fabs(c[1]) + std::fabs(c[2]) + std::fabs(c[3]));
+        if (!(v <= most)) most = v;
+    }
+    return most <= 1e30 ? (float)most : 1e30f;
+}
+
 // Dominant axis: argmax |e_c|, ties resolved in the order x, y, z.
 int dominant_axis(V3 e)
 {
@@ -595,7 +610,8 @@ int build_angles(const tsx_geometry *g, tsx_plan *p)
         A.fkappa = (float)A.kappa;
         A.finv_kappa = (float)A.inv_kappa;
         A.fspan = (float)((std::fabs(A.N[1]) + std::fabs(A.N[2])) * std::fabs(A.inv_kappa));
-        A.freach = (float)(16.0 * (std::fabs(A.N[0]) + std::fabs(A.N[1]) + std::fabs(A.N[2])));
+        A.freach = cone ? (float)(16.0 * (std::fabs(A.N[0]) + std::fabs(A.N[1]) + std::fabs(A.N[2])))
+                        : parallel_reach(A, g);
         tile_slopes(A, g->det_row_count, g->det_col_count, &slope_j[a], &slope_i[a]);
         p->axis_count[m] += 1;
     }
@@ -1779,11 +1795,22 @@ int launch_bp_general(const tsx_plan *p, T *vol, int64_t vs, const T *proj, int6
     return TSX_OK;
 }
 
+// Whether a parallel scan has a direction so near its detector's plane that
+// bp_tilted has to cut boxes in FP64.
+bool tilted_far(const tsx_plan *p)
+{
+    if (p->kind == TSX_CONE_VEC) return false;
+    for (const AngleParams &A : p->host)
+        if (!(A.freach <= TILTED_REACH)) return true;
+    return false;
+}
+
 // Voxels per thread of bp_tilted: eight share a set-up, or two, or none where
 // more would leave fewer than four blocks per CU (of one entry: the choice
 // changes the rounding of positions, so it depends on the plan alone).
 int tilted_voxels(const tsx_plan *p)
 {
+    if (tilted_far(p)) return 1;
     const int64_t columns = (int64_t)((p->nx + BP_BX - 1) / BP_BX) * ((p->ny + BP_BY - 1) / BP_BY);
     for (int zv : {8, 2})
         if (columns * ((p->nz + zv - 1) / zv) >= 1024) return zv;
@@ -1799,9 +1826,10 @@ int launch_bp_tilted(const tsx_plan *p, float *vol, int64_t vs, const float *ly,
     const int zv = tilted_voxels(p);
     const int64_t groups = (p->nz + zv - 1) / zv, bc = GRID_DIM_MAX / groups;  // entries per launch
     const bool cone = p->kind == TSX_CONE_VEC;
-    auto kernel = zv == 8   ? (cone ? bp_tilted<true, 8> : bp_tilted<false, 8>)
-                  : zv == 2 ? (cone ? bp_tilted<true, 2> : bp_tilted<false, 2>)
-                            : (cone ? bp_tilted<true, 1> : bp_tilted<false, 1>);
+    auto kernel = zv == 8   ? (cone ? bp_tilted<true, 8, true> : bp_tilted<false, 8, false>)
+                  : zv == 2 ? (cone ? bp_tilted<true, 2, true> : bp_tilted<false, 2, false>)
+                            : (cone ? bp_tilted<true, 1, true> : bp_tilted<false, 1, false>);
+    if (tilted_far(p)) kernel = bp_tilted<false, 1, true>;
     for (int64_t b0 = 0; b0 < batch; b0 += bc) {
         const int64_t nb = std::min(bc, batch - b0);
         dim3 grid((unsigned)((p->nx + BP_BX - 1) / BP_BX), (unsigned)((p->ny + BP_BY - 1) / BP_BY),
