@@ -45,6 +45,8 @@ extern "C" int near_box(double c, float step, int k, float half, int n, int *out
     out[2] = j0;
     return 1;
 }
+extern "C" double apart(const double *N) { return tilted_apart(N); }
+extern "C" float growth(float c) { return tilted_growth(c); }
 """
 
 
@@ -61,6 +63,10 @@ def boxes(tmp_path_factory):
     lib.far_box.argtypes = [ctypes.c_double, ctypes.c_float, ctypes.c_int, ctypes.c_void_p]
     lib.near_box.argtypes = [ctypes.c_double, ctypes.c_float, ctypes.c_int, ctypes.c_float, ctypes.c_int,
                              ctypes.c_void_p]
+    lib.apart.restype = ctypes.c_double
+    lib.apart.argtypes = [ctypes.c_void_p]
+    lib.growth.restype = ctypes.c_float
+    lib.growth.argtypes = [ctypes.c_float]
     return lib
 
 
@@ -109,3 +115,16 @@ def test_boxes_within_reach_never_leave_the_detector(boxes, n):
                             elif want:
                                 assert hi < lo or (lo + j0 >= want[0] and hi + j0 <= want[1])
     assert taken > 1000
+
+
+def test_box_growth_covers_every_voxel_of_a_thread(boxes):
+    """The image of a voxel's square is at most 1 / (1 - c) of its linear part,
+    c = (|N1| + |N2|) / |W . N|; the thread's voxels lie k N1 further, k < 8."""
+    rng = np.random.default_rng(7)
+    normals = np.concatenate([rng.standard_normal((500, 3)), [[0, 1, 0], [0.01, 1, 0.01], [0, 1, 1], [1, 0, 0]]])
+    for N in normals:
+        N = np.ascontiguousarray(N)
+        dn = boxes.apart(N.ctypes.data) * (1 + 1e-6)
+        for sign in (1, -1):
+            c = (abs(N[1]) + abs(N[2])) / np.abs(sign * dn + np.arange(8) * N[1])
+            assert c.max() <= 1 / 16 + 1e-9 and boxes.growth(c.max()) >= 1 / (1 - c.max()), (N, c.max())

@@ -281,8 +281,8 @@ __global__ void scale_by_length(const AngleParams *__restrict__ angles, int n_an
 // are largest at an end, so that one box size, from the two ends, serves all
 // of them. A pixel's weight takes its ray's in-slice offset, as in bp_general:
 // (dj A1j + di A1i) / (1 + dj fBj + di fBi) along c1, likewise along c2.
-// Angles stepping along z, voxels near the source's planes (W . N under 16
-// times its steps, |W_m| under 16) and positions or boxes beyond TILTED_REACH
+// Angles stepping along z, voxels near the source's planes (W . N under
+// tilted_apart, |W_m| under 16) and positions or boxes beyond TILTED_REACH
 // take the FP64 set-up for each voxel and cut its box in FP64 (FAR: a
 // parallel scan has angles whose positions are; it has none else).
 //
@@ -360,6 +360,7 @@ __global__ void __launch_bounds__(BP_BX *BP_BY)
 bp_tilted(const AngleParams *__restrict__ angles, int n_angles, int rows, int cols, int nx, int ny, int nz,
           float *__restrict__ vol, int64_t vol_stride, const float *__restrict__ ly, int64_t ly_stride, Epilogue ep)
 {
+    static_assert(ZV <= TILTED_VOXELS, "tilted_apart covers the voxels of a thread");
     const int x = blockIdx.x * BP_BX + threadIdx.x;
     const int y = blockIdx.y * BP_BY + threadIdx.y;
     const int zb = (nz + ZV - 1) / ZV;
@@ -460,7 +461,7 @@ bp_tilted(const AngleParams *__restrict__ angles, int n_angles, int rows, int co
                 mi = fmaxf(mi, fabsf(M10) + fabsf(M11));
                 s = fmaxf(s, fabsf(lam));
             }
-            s *= fmaf(1.1f * A.fspan, s, 1.0f);  // 1 / (1 - c) <= 1 + 1.1 c for c <= 1 / 16
+            s *= tilted_growth(A.fspan * s);
             mj = fmaf(mj, s, 1e-3f);
             mi = fmaf(mi, s, 1e-3f);
         }

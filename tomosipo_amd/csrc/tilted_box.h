@@ -47,4 +47,17 @@ TSX_BOX_FN PixelRange tilted_pixels(double c, double half, int n)
     return r;
 }
 
+// Cone beams, |W . N| (W from the source to a voxel, N the detector's normal in
+// voxel steps along m, c1, c2) above which up to TILTED_VOXELS voxels along c1
+// from it on have c = (|N1| + |N2|) / |W . N| <= 1 / 16, the last ones too.
+constexpr int TILTED_VOXELS = 8;
+
+TSX_BOX_FN double tilted_apart(const double *N)
+{
+    return 16.0 * (fabs(N[0]) + fabs(N[1]) + fabs(N[2])) + (TILTED_VOXELS - 1) * fabs(N[1]);
+}
+
+// 1 / (1 - c) or a little more, for c <= 1 / 16 (it holds up to 1 / 11).
+TSX_BOX_FN float tilted_growth(float c) { return fmaf(1.1f, c, 1.0f); }
+
 }  // namespace tsx

@@ -610,8 +610,7 @@ int build_angles(const tsx_geometry *g, tsx_plan *p)
         A.fkappa = (float)A.kappa;
         A.finv_kappa = (float)A.inv_kappa;
         A.fspan = (float)((std::fabs(A.N[1]) + std::fabs(A.N[2])) * std::fabs(A.inv_kappa));
-        A.freach = cone ? (float)(16.0 * (std::fabs(A.N[0]) + std::fabs(A.N[1]) + std::fabs(A.N[2])))
-                        : parallel_reach(A, g);
+        A.freach = cone ? (float)tilted_apart(A.N) : parallel_reach(A, g);
         tile_slopes(A, g->det_row_count, g->det_col_count, &slope_j[a], &slope_i[a]);
         p->axis_count[m] += 1;
     }

@@ -32,7 +32,7 @@ struct AngleParams {
     float fU[3], fV[3];   // U and V rounded to float
     double sBj, sBi;      // cone: (S - P0) . Bj, (S - P0) . Bi
     // cone: floats of N, Bj, Bi, kappa and 1 / kappa; (|N1| + |N2|) / |kappa|;
-    // 16 (|N0| + |N1| + |N2|). parallel: the position's steps (fBj, fBi)
+    // tilted_apart(N). parallel: the position's steps (fBj, fBi)
     // along (m, c1, c2), and in freach the largest position, step or half-width
     float fN[3], fBj[3], fBi[3], fkappa, finv_kappa, fspan, freach;
     // parallel beam: detector position of grid point k = (k_m, k_c1, k_c2),
