@@ -1118,11 +1118,13 @@ FlatPlan flat_bp(const tsx_plan *p, int64_t batch)
 }
 
 // Angle parts of the flat backprojector, for the plans that bp_part_len_of
-// cuts into parts (never more of them: they use its workspace): two halves,
-// which round less than one running sum (180 angles: 1.7e-7 of the result
-// against 2.7e-7; the separable kernel's four parts 1.9e-7), or parts of at
-// least 4 angles, about 256 blocks of 8 waves per launch of one entry, where
-// the bricks alone give fewer than 128.
+// cuts into parts (never more of them: they use its workspace): parts of at
+// least 4 angles, about 256 blocks of 8 waves per launch of one entry where the
+// bricks alone give fewer than 128, and of no more angles than round least: n
+// angles in parts of L round with the variance 2 n L^2 / 3 within the parts and
+// n^3 / (3 L) where these are added, least at L = (n^2 / 4)^(1/3). Longer
+// parts only where the separable kernel's are (128^3 and slices of 256^2, 180
+// angles: two halves 1.6e-7 of the result, its parts of 45 1.0e-7).
 int flat_part_len(const tsx_plan *p)
 {
     const int cut = bp_part_len_of(p);
@@ -1130,7 +1132,8 @@ int flat_part_len(const tsx_plan *p)
     const int zl = flat_zl(p->nz);
     const int64_t blocks = std::min<int64_t>(128, flat_blocks(p, 8, (p->nz + 64 * zl - 1) / (64 * zl)));
     const int64_t len = std::max<int64_t>(4, ((int64_t)p->n_angles * blocks + 255) / 256);
-    return (int)std::min<int64_t>(std::max<int64_t>(len, cut), p->n_angles);
+    const int64_t least = (int64_t)std::ceil(std::cbrt(0.25 * p->n_angles * p->n_angles));
+    return (int)std::max<int64_t>(cut, std::min(len, least));
 }
 
 int64_t workspace_bytes(const tsx_plan *p, int op, int64_t batch)
@@ -1596,7 +1599,7 @@ struct FlatBatch {
         rc = main_pass(f.direct ? bp_flat_direct_kernel(nc) : bp_flat_kernel(f.zl, nc), by, 10, 2048,
                        [](const FlatView &v) { return (int64_t)v.bx * v.by * v.chunks * v.parts; });
         if (rc || !sums) return rc;
-        hipLaunchKernelGGL(flat_parts_reduce, dim3((unsigned)((ve + 255) / 256), (unsigned)entries, (unsigned)m.n),
+        hipLaunchKernelGGL(flat_parts_reduce, dim3((unsigned)((ve + FLAT_REDUCE - 1) / FLAT_REDUCE), (unsigned)entries, (unsigned)m.n),
                            dim3(256), 0, stream, m);
         TSX_HIP_CHECK(hipGetLastError());
         return TSX_OK;
