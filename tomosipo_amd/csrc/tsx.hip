@@ -197,13 +197,16 @@ struct tsx_plan {
     std::string bp_reason;      // why bp_separable is off
     // kernel variants chosen by tsx_plan_autotune (-1: library default)
     int32_t fp_variant = -1, bp_bz = -1, fp_by = -1;
-    // FDK (cone plans): per-angle quantities and the volume window
     // flat parallel-beam kernels (fp_flat, bp_flat): the angles ordered by
     // stepping axis (empty: the plan is not flat), and the columns they stage
     std::vector<FlatAngle> flat_host;
     FlatAngle *flat_dev = nullptr;
     int32_t flat_nc = 0;                // backward: detector columns per voxel column
     int32_t flat_stage_bp = 0;          // detector columns staged per angle
+    // bytes that the plan holding this one (refined detector, swapped axes)
+    // puts before its workspace, for one entry of TSX_OP_FP and TSX_OP_BP
+    int64_t outer[2] = {0, 0};
+    // FDK (cone plans): per-angle quantities and the volume window
     std::vector<FdkAngle> fdk_host;
     FdkAngle *fdk_dev = nullptr;
     const float *fdk_factors = nullptr;  // the ramp filter's factors (after fdk_dev's entries)
@@ -1018,18 +1021,24 @@ int64_t flat_turned_elems(const tsx_plan *p, int64_t batch)
     return ((int64_t)p->nx * p->ny + 1) * flat_pitch(p, batch);
 }
 
-// Workspace floats of the forward projector. The flat kernels' turned volume
-// and sums G live in that of the padded layouts (which is two to four times
-// the volume), G for as many angles at a time as it holds; it is grown to
-// flat_angles of them, unless 64 took the plan past the static buffer of
-// tsx_direct_fpbp3d_noalloc: it then stays on the padded kernels.
+// The least workspace floats of the flat forward projector: the turned volume
+// and the sums of 16 angles.
+int64_t flat_fp_least(const tsx_plan *p)
+{
+    return flat_turned_elems(p, 1) + (int64_t)p->cols * flat_pitch(p, 1) * std::min(p->n_angles, 16);
+}
+
+// The flat kernels' turned volume and sums G live in the workspace of the
+// padded layouts (which is two to four times the volume), G for as many angles
+// at a time as it holds; it is grown to flat_angles of them. A plan whose padded
+// layouts fit the static buffer of tsx_direct_fpbp3d_noalloc, but not the
+// flat kernels' least, stays on the padded kernels.
 bool flat_fp_ok(const tsx_plan *p)
 {
     if (p->flat_host.empty() || force_general() || env_int("TSX_FP_VARIANT") >= 2 || !p->fp_padded) return false;
     if (flat_turned_elems(p, 1) * 4 >= (int64_t)1 << 32) return false;  // 32-bit byte offsets
-    const int64_t need = flat_turned_elems(p, 1) + (int64_t)p->cols * flat_pitch(p, 1) * std::min(p->n_angles, 64);
-    return need * 4 <= TSX_NOALLOC_SCRATCH_BYTES || fp_workspace_elems(p) * 4 > TSX_NOALLOC_SCRATCH_BYTES ||
-           need <= fp_workspace_elems(p);
+    const int64_t buffer = TSX_NOALLOC_SCRATCH_BYTES - p->outer[TSX_OP_FP];
+    return flat_fp_least(p) * 4 <= buffer || fp_workspace_elems(p) * 4 > buffer;
 }
 
 // Angles whose sums G the workspace has to hold: all of them within 64 MiB per
@@ -1041,10 +1050,14 @@ int64_t flat_angles(const tsx_plan *p)
     return std::min<int64_t>(p->n_angles, std::max<int64_t>(64, room / ((int64_t)p->cols * flat_pitch(p, 1))));
 }
 
-int64_t fp_elems(const tsx_plan *p, int64_t batch)
+// Workspace floats of the forward projector; with `least`, those that it can do
+// with (tsx_direct_fpbp3d_noalloc, one entry: more launches of fewer angles,
+// whose results are the same).
+int64_t fp_elems(const tsx_plan *p, int64_t batch, bool least = false)
 {
     const int64_t padded = fp_workspace_elems(p) * batch;
     if (!flat_fp_ok(p)) return padded;
+    if (least) return std::max(padded, flat_fp_least(p));
     return std::max(padded, flat_turned_elems(p, batch) + (int64_t)p->cols * flat_pitch(p, batch) * flat_angles(p));
 }
 
@@ -1054,13 +1067,14 @@ int64_t flat_fp_blocks(int angles, int cols, int rays, int chunks)
     return (int64_t)((angles + 3) / 4) * ((cols + rays - 1) / rays) * chunks;
 }
 
-FlatPlan flat_fp(const tsx_plan *p, int64_t batch)
+// elems: the workspace's floats, where they are not those of fp_elems
+FlatPlan flat_fp(const tsx_plan *p, int64_t batch, int64_t elems = 0)
 {
     FlatPlan f;
     const int64_t W = p->nz * batch, Wp = flat_pitch(p, batch);
     if (!flat_fp_ok(p) || W > (1 << 28)) return f;
     f.per_launch = (int)std::min<int64_t>(
-        p->n_angles, (fp_elems(p, batch) - flat_turned_elems(p, batch)) / ((int64_t)p->cols * Wp));
+        p->n_angles, ((elems ? elems : fp_elems(p, batch)) - flat_turned_elems(p, batch)) / ((int64_t)p->cols * Wp));
     // Chunks of w: one up to 127; of 64, whole cache lines, where they fit
     // (512^3, 360 angles: 9.9 ms, chunks of 76 17.1); else at most 80 (134^3,
     // 360 angles: chunks of 68 0.26 ms, one 0.32). As many rays as fill a wave;
@@ -1080,7 +1094,9 @@ FlatPlan flat_fp(const tsx_plan *p, int64_t batch)
 // The backprojector's lines U take the workspace of the transposed
 // projections (grown where the volume is higher than the detector).
 // Where that growth would take a plan past the static buffer of
-// tsx_direct_fpbp3d_noalloc, the plan keeps the separable kernel and the buffer.
+// tsx_direct_fpbp3d_noalloc, the plan keeps the separable kernel and the buffer
+// (for every caller, as that entry point's results are tsx_direct_fpbp3d's:
+// angles in several launches would add up in another order).
 bool flat_bp_ok(const tsx_plan *p)
 {
     if (p->flat_host.empty() || !p->bp_separable || force_general() || env_int("TSX_BP_BRICK_Z") >= 0 ||
@@ -1088,7 +1104,8 @@ bool flat_bp_ok(const tsx_plan *p)
         return false;
     const int64_t sums = bp_parts_of(p) > 1 ? (int64_t)bp_parts_of(p) * p->nx * p->ny * p->nz * 4 + 256 : 0;
     const int64_t lines = ((int64_t)bp_chunk_of(p) * p->cols + 1) * flat_pitch(p, 1) * 4;
-    return lines + sums <= TSX_NOALLOC_SCRATCH_BYTES || bp_workspace_elems(p) * 4 + sums > TSX_NOALLOC_SCRATCH_BYTES;
+    const int64_t buffer = TSX_NOALLOC_SCRATCH_BYTES - p->outer[TSX_OP_BP];
+    return lines + sums <= buffer || bp_workspace_elems(p) * 4 + sums > buffer;
 }
 
 int64_t flat_line_elems(const tsx_plan *p, int64_t batch)
@@ -1136,16 +1153,17 @@ int flat_part_len(const tsx_plan *p)
     return (int)std::max<int64_t>(cut, std::min(len, least));
 }
 
-int64_t workspace_bytes(const tsx_plan *p, int op, int64_t batch)
+// (least: as for fp_elems)
+int64_t workspace_bytes(const tsx_plan *p, int op, int64_t batch, bool least = false)
 {
     if (force_general()) return 0;
     // the axis-swapped plan's volume, then that plan's workspace
     if (op == TSX_OP_FP && fp_swapped(p))
-        return align_ws((int64_t)p->nx * p->ny * p->nz * batch * 4) + workspace_bytes(p->perm, op, batch);
+        return align_ws((int64_t)p->nx * p->ny * p->nz * batch * 4) + workspace_bytes(p->perm, op, batch, least);
     // the refined detector's projections, then that plan's workspace
     if (op == TSX_OP_FP && fp_refined(p))
-        return align_ws(refined_sino(p) * batch * 4) + workspace_bytes(p->fine, op, batch);
-    if (op == TSX_OP_FP) return p->fp_padded ? fp_elems(p, batch) * 4 : 0;
+        return align_ws(refined_sino(p) * batch * 4) + workspace_bytes(p->fine, op, batch, least);
+    if (op == TSX_OP_FP) return p->fp_padded ? fp_elems(p, batch, least) * 4 : 0;
     if (op == TSX_OP_BP && bp_refined(p)) return workspace_bytes(p->fine, op, batch);
     if (p->perm)
         return align_ws((int64_t)p->nx * p->ny * p->nz * batch * 4) + workspace_bytes(p->perm, op, batch);
@@ -1615,14 +1633,14 @@ int64_t flat_entries(const tsx_plan *p)
 }
 
 int launch_fp_flat(const tsx_plan *p, const float *vol, int64_t vs, float *proj, int64_t ps, int64_t batch,
-                   Epilogue ep, float *base, hipStream_t stream)
+                   Epilogue ep, float *base, int64_t elems, hipStream_t stream)
 {
     // (the turned volume of a launch is addressed with 32-bit byte offsets)
     const int64_t room = (((int64_t)1 << 30) - 1) / ((int64_t)p->nx * p->ny + 1) - 3;
     const int64_t bc = std::max<int64_t>(1, std::min(flat_entries(p), room / p->nz));
     for (int64_t b0 = 0; b0 < batch; b0 += bc) {
         const int64_t nb = std::min(bc, batch - b0);
-        const FlatPlan f = flat_fp(p, nb);
+        const FlatPlan f = flat_fp(p, nb, elems);
         for (int k0 = 0; k0 < p->n_angles; k0 += f.per_launch) {
             FlatBatch fb(stream);
             FlatView v = flat_view(p, f, nb, k0, std::min(f.per_launch, p->n_angles - k0), ep_from(ep, b0));
@@ -1678,10 +1696,11 @@ int launch_bp_flat(const tsx_plan *p, float *vol, int64_t vs, const float *proj,
 
 // Forward projection of `batch` volumes: the padded kernels on the whole
 // volume or slab by slab (each slab's sums added to the projections of the
-// previous ones), else the general kernel.
+// previous ones), else the general kernel. least: the workspace given holds
+// workspace_bytes(.., true) or more, and all of it may be used.
 int launch_fp(const tsx_plan *p, const float *vol, int64_t vs, float *proj, int64_t ps,
               int64_t batch, Epilogue ep, hipStream_t stream, void *wsp = nullptr,
-              int64_t ws_bytes = 0)
+              int64_t ws_bytes = 0, bool least = false)
 {
     if (batch <= 0) return TSX_OK;
     if (fp_refined(p)) {
@@ -1692,13 +1711,14 @@ int launch_fp(const tsx_plan *p, const float *vol, int64_t vs, float *proj, int6
         // (the requirement formed here from its two parts, so that a short
         // workspace is refused rather than overrun)
         const int64_t fe = refined_sino(p);
-        const int64_t fine_bytes = align_ws(fe * batch * 4), rest_bytes = workspace_bytes(p->fine, TSX_OP_FP, batch);
+        const int64_t fine_bytes = align_ws(fe * batch * 4), rest_bytes = workspace_bytes(p->fine, TSX_OP_FP, batch, least);
         Scratch owned;
         void *wptr = nullptr;
         int rc = get_workspace(p, fine_bytes + rest_bytes, wsp, ws_bytes, stream, owned, &wptr);
         if (rc) return rc;
         float *fine = (float *)wptr;
-        rc = launch_fp(p->fine, vol, vs, fine, fe, batch, plain(0), stream, (char *)wptr + fine_bytes, rest_bytes);
+        rc = launch_fp(p->fine, vol, vs, fine, fe, batch, plain(0), stream, (char *)wptr + fine_bytes,
+                       least ? ws_bytes - fine_bytes : rest_bytes, least);
         if (rc) return rc;
         const int64_t blocks = (int64_t)((p->cols + 255) / 256) * p->rows * p->n_angles;
         const int64_t cap = max_blocks(256);
@@ -1715,7 +1735,7 @@ int launch_fp(const tsx_plan *p, const float *vol, int64_t vs, float *proj, int6
     if (fp_swapped(p)) {
         const int64_t ve = (int64_t)p->nx * p->ny * p->nz;
         const tsx_plan *q = p->perm;
-        const int64_t tmp_bytes = align_ws(ve * batch * 4), rest_bytes = workspace_bytes(q, TSX_OP_FP, batch);
+        const int64_t tmp_bytes = align_ws(ve * batch * 4), rest_bytes = workspace_bytes(q, TSX_OP_FP, batch, least);
         Scratch owned;
         void *wptr = nullptr;
         int rc = get_workspace(p, tmp_bytes + rest_bytes, wsp, ws_bytes, stream, owned, &wptr);
@@ -1723,17 +1743,18 @@ int launch_fp(const tsx_plan *p, const float *vol, int64_t vs, float *proj, int6
         float *tmp = (float *)wptr;
         rc = launch_unswap(vol, vs, tmp, ve, q->nx, q->ny, q->nz, p->swap, batch, plain(0), stream);
         if (rc) return rc;
-        return launch_fp(q, tmp, ve, proj, ps, batch, ep, stream, (char *)wptr + tmp_bytes, rest_bytes);
+        return launch_fp(q, tmp, ve, proj, ps, batch, ep, stream, (char *)wptr + tmp_bytes,
+                         least ? ws_bytes - tmp_bytes : rest_bytes, least);
     }
     if (!p->fp_padded || force_general() || p->ss > 4)
         return launch_fp_general<float>(p, vol, vs, proj, ps, batch, ep, stream);
     const int variant = fp_variant_of(p), by = fp_tile_rows_of(p);
     Scratch owned;
     void *wptr = nullptr;
-    int rc = get_workspace(p, fp_elems(p, batch) * 4, wsp, ws_bytes, stream, owned, &wptr);
+    int rc = get_workspace(p, fp_elems(p, batch, least) * 4, wsp, ws_bytes, stream, owned, &wptr);
     if (rc) return rc;
     if (flat_fp(p, 1).ok && flat_fp(p, std::min(batch, flat_entries(p))).ok)
-        return launch_fp_flat(p, vol, vs, proj, ps, batch, ep, (float *)wptr, stream);
+        return launch_fp_flat(p, vol, vs, proj, ps, batch, ep, (float *)wptr, least ? ws_bytes / 4 : 0, stream);
     const bool shear = fp_shear_on(p);  // (slabs: each with its own row offset bound)
     if (p->slabs.empty())
         return launch_fp_padded(p, variant, by, shear, vol, vs, proj, ps, batch, ep, (float *)wptr, stream);
@@ -2683,6 +2704,17 @@ tsx_geometry refined_geometry(const tsx_geometry *g, std::vector<double> &vec)
     return fg;
 }
 
+// The bytes before the workspaces of a plan and of those that it holds
+// (tsx_plan::outer, in the order of launch_fp and launch_bp).
+void set_outer(tsx_plan *p, int64_t fp, int64_t bp)
+{
+    p->outer[TSX_OP_FP] = fp;
+    p->outer[TSX_OP_BP] = bp;
+    const int64_t vol = align_ws((int64_t)p->nx * p->ny * p->nz * 4);
+    if (p->perm) set_outer(p->perm, fp + vol, bp + vol);
+    if (p->fine) set_outer(p->fine, fp + align_ws(refined_sino(p) * 4), bp);
+}
+
 // The upright FDK backprojector, where its kernel takes the plan. (Its workspace
 // stays at 8 bytes per pixel, as callers size their buffers, of which it uses 4.)
 bool fdk_staged(const tsx_plan *p)
@@ -2839,6 +2871,7 @@ int tsx_plan_create(const tsx_geometry *g, int device, tsx_plan **out)
         }
         g_last_error.clear();
     }
+    set_outer(p, 0, 0);
     *out = p;
     return TSX_OK;
 }
@@ -3271,7 +3304,7 @@ int tsx_direct_fpbp3d_noalloc(const tsx_plan *p, float *vol, float *proj, int mo
     if (op != TSX_OP_FP && op != TSX_OP_BP)
         return fail(TSX_ERR_INVALID_ARGUMENT, "op must be TSX_OP_FP (0) or TSX_OP_BP (1)");
     if (!vol || !proj) return fail(TSX_ERR_INVALID_ARGUMENT, "data pointers must not be NULL");
-    const int64_t need = workspace_bytes(p, op, 1);
+    const int64_t need = workspace_bytes(p, op, 1, true);
     if (need > TSX_NOALLOC_SCRATCH_BYTES)
         return fail(TSX_ERR_UNSUPPORTED, "tsx_direct_fpbp3d_noalloc: the plan needs " + std::to_string(need) +
                                              " bytes of workspace, more than the " +
@@ -3286,7 +3319,7 @@ int tsx_direct_fpbp3d_noalloc(const tsx_plan *p, float *vol, float *proj, int mo
     if (rc) return rc;
     const Epilogue ep = plain(mode == TSX_MODE_ADD);
     if (op == TSX_OP_FP)
-        return launch_fp(p, vol, 0, proj, 0, 1, ep, (hipStream_t)stream, ws, TSX_NOALLOC_SCRATCH_BYTES);
+        return launch_fp(p, vol, 0, proj, 0, 1, ep, (hipStream_t)stream, ws, TSX_NOALLOC_SCRATCH_BYTES, true);
     return launch_bp(p, vol, 0, proj, 0, 1, ep, (hipStream_t)stream, ws, TSX_NOALLOC_SCRATCH_BYTES);
 }
 
