@@ -1288,4 +1288,16 @@ __attribute__((amdgpu_waves_per_eu(PARTS ? 1 : bp_waves_per_eu(BZ)))) bp_wave_mu
     bp_wave_work<BZ, PARTS>(m.v[k], logical - m.begin[k], sh);
 }
 
+// bp_parts_reduce for every instance of a fused launch: grid (voxels / 256 of
+// the largest one, instances).
+__global__ void __launch_bounds__(256) bp_parts_reduce_multi(BpMulti m)
+{
+    const BpView &v = m.v[blockIdx.y];
+    const int64_t ve = (int64_t)v.nx * v.ny * v.nz, o = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (o >= ve) return;
+    float t = v.partial[o];
+    for (int s = 1; s < v.parts; ++s) t += v.partial[(int64_t)s * ve + o];
+    emit(v.vol, o, 0, t, v.ep);
+}
+
 }  // namespace tsx

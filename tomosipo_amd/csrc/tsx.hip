@@ -2140,13 +2140,29 @@ int multi_fp(const tsx_plan *const *plans, const float *const *vols, float *cons
     return flush();
 }
 
-// Bricks of a fused backprojection below which instances in angle parts run
-// alone: it runs a brick's parts in turn, so that fewer than about four blocks
-// per CU leave it idle, while their own launches run the parts in separate
-// blocks (two 105^3 cones beside two parallel scans: the pass 386 and 283 us
-// with its forward projections; eight scans of 64^3 to 128^3, 880 bricks: 1.35
-// and 1.25 ms). Either order of a part's sums gives the same bits.
-constexpr int64_t MULTI_BP_BRICKS = 1024;
+// Whether the angle parts of a fused launch's instances run in separate blocks
+// with a reduction after them, or a brick's parts in turn in its block (either
+// order of the sums gives the same bits). In separate blocks the chip is full,
+// at 4 ns per brick and angle and 20 ns per brick and part (its sums written and
+// read); in turn an angle takes the latency of a brick, 3.2 us and a little more
+// the more bricks run beside it, for every 1024 bricks (four per CU). Measured, in
+// turn and apart: 8 x 32^3, 40 angles 140 and 44 us, 12 x 64^3, 90 angles 348
+// and 311, 16 of them 355 and 415, 8 x 96^3, 120 angles 537 and 573, 3 x
+// 140^3, 200 angles 1319 and 1014.
+bool parts_apart(const BpMulti &m)
+{
+    double apart = 0.0;
+    int64_t bricks = 0;
+    int angles = 0;
+    for (int k = 0; k < m.n; ++k) {
+        const BpView &v = m.v[k];
+        const int64_t b = (int64_t)v.bricks_x * v.bricks_y * v.bricks_z;
+        apart += (double)b * (4.0 * v.n_angles + 20.0 * v.parts);
+        bricks += b;
+        angles = std::max(angles, v.n_angles);
+    }
+    return apart < (double)angles * ((bricks + 1023) / 1024) * (3150.0 + 1.25 * std::min<int64_t>(bricks, 1024));
+}
 
 int multi_bp(const tsx_plan *const *plans, float *const *vols, const float *const *projs,
              const Epilogue *eps, int n, void *wsp, int64_t ws_bytes, hipStream_t stream)
@@ -2164,20 +2180,33 @@ int multi_bp(const tsx_plan *const *plans, float *const *vols, const float *cons
     BpMulti m;
     m.n = 0;
     m.begin[0] = 0;
+    float *part_sums[MAX_FUSED];  // room for the sums of the instances' angle parts
     ScaleJobs sj;
     int sj_max = 0;  // blocks of the largest job in sj
     auto flush = [&]() -> int {
         if (m.n == 0) return TSX_OK;
         sj.n = m.n;
-        pad_begin(m.begin, m.n);
         hipLaunchKernelGGL(scale_by_length_t_multi, dim3((unsigned)sj_max, (unsigned)sj.n), dim3(32, 8), 0, stream,
                            sj);
         sj_max = 0;
+        const bool apart = PM && parts_apart(m);
+        int64_t ve = 0;
+        for (int k = 0; apart && k < m.n; ++k) {
+            BpView &v = m.v[k];
+            v.partial = part_sums[k];
+            m.begin[k + 1] = m.begin[k] + v.bricks_x * v.bricks_y * v.bricks_z * v.parts;
+            ve = std::max(ve, (int64_t)v.nx * v.ny * v.nz);
+        }
+        pad_begin(m.begin, m.n);
         const unsigned grid = xcd_grid(m.begin[m.n], &m.shift);
-        auto kern = BZ == 32 ? (PM ? bp_wave_multi<32, true> : bp_wave_multi<32, false>)
-                  : BZ == 24 ? (PM ? bp_wave_multi<24, true> : bp_wave_multi<24, false>)
-                             : (PM ? bp_wave_multi<16, true> : bp_wave_multi<16, false>);
+        const bool in_turn = PM && !apart;
+        auto kern = BZ == 32 ? (in_turn ? bp_wave_multi<32, true> : bp_wave_multi<32, false>)
+                  : BZ == 24 ? (in_turn ? bp_wave_multi<24, true> : bp_wave_multi<24, false>)
+                             : (in_turn ? bp_wave_multi<16, true> : bp_wave_multi<16, false>);
         hipLaunchKernelGGL(kern, dim3(grid), dim3(BR, BR), 0, stream, m);
+        if (apart)
+            hipLaunchKernelGGL(bp_parts_reduce_multi, dim3((unsigned)((ve + 255) / 256), (unsigned)m.n), dim3(256), 0,
+                               stream, m);
         TSX_HIP_CHECK(hipGetLastError());
         m.n = 0;
         return TSX_OK;
@@ -2223,15 +2252,6 @@ int multi_bp(const tsx_plan *const *plans, float *const *vols, const float *cons
         const int rc = fb.backward(f, plans[k]->flat_nc);
         if (rc) return rc;
     }
-    // Separable instances in angle parts whose bricks together are few take
-    // their own launches, which run the parts in separate blocks.
-    const auto bricks_of = [](const tsx_plan *p) {
-        const int bz = bp_brick_z_of(p);
-        return (int64_t)((p->nx + BR - 1) / BR) * ((p->ny + BR - 1) / BR) * ((p->nz + bz - 1) / bz);
-    };
-    int64_t in_parts = 0;
-    for (int k = 0; k < n; ++k)
-        if (!taken[k] && bp_parts_of(plans[k]) > 1) in_parts += bricks_of(plans[k]);
     for (size_t pass = 0; pass < keys.size(); ++pass)
     for (int k = 0; k < n; ++k) {
         if (taken[k]) continue;
@@ -2250,7 +2270,7 @@ int multi_bp(const tsx_plan *const *plans, float *const *vols, const float *cons
         const int64_t tblocks = scale_job_blocks(job);
         const int64_t cap = max_blocks(BR * BR);
         if (!(fast && p->bp_separable && bp_chunk_of(p) == p->n_angles) || blocks > cap ||
-            tblocks > max_blocks(256) || flat_bp(p, 1).ok || (bp_parts_of(p) > 1 && in_parts < MULTI_BP_BRICKS)) {
+            tblocks > max_blocks(256) || flat_bp(p, 1).ok) {
             if (pass > 0) continue;  // (its own launch, in the first pass)
             int rc = launch_bp(p, vols[k], 0, projs[k], 0, 1, eps[k], stream, wptr ? (char *)wptr + woff : nullptr, wb);
             if (rc) return rc;
@@ -2275,6 +2295,7 @@ int multi_bp(const tsx_plan *const *plans, float *const *vols, const float *cons
         if (parts > 1) {
             m.v[m.n].parts = parts;
             m.v[m.n].part_len = bp_part_len_of(p);
+            part_sums[m.n] = (float *)((char *)ly + align_ws(sino_t * 4));
         }
         m.begin[m.n + 1] = m.begin[m.n] + (int)blocks;
         m.n += 1;
