@@ -69,3 +69,42 @@ def test_outputs_of_any_alignment_and_stride_hold_the_same_bits(shape):
                     got = out[shift + k * (m + extra):][:m]
                     assert torch.equal(got, want_f[k] + 2.0 if additive else want_f[k]), (shift, extra, additive, k)
                 assert (out[:shift] == 2.0).all() and (out[shift + 2 * (m + extra) + m:] == 2.0).all()
+
+
+@pytest.mark.parametrize("nz,n,batches", [(1, 36, (2, 3, 4, 5, 60, 64, 65)), (8, 300, (6, 9)), (3, 30, (2, 21, 22))])
+def test_short_and_long_lines_hold_the_same_bits(nz, n, batches):
+    """A batch's entries lengthen the lines: through the kernel of short lines, one and four values
+    per lane, its angle parts in blocks of their own and in turn, to the one that stages lines."""
+    A = _operator((nz, n, n - 3), (nz, n + 9), 50)
+    plan, s = A.projector.plan(0), torch.cuda.current_stream().cuda_stream
+    gen = torch.Generator(device=DEV)
+    gen.manual_seed(n)
+    ys = torch.randn((max(batches),) + A.range_shape, generator=gen, device=DEV)
+    want = [A.T(ys[k]) for k in range(max(batches))]
+    for batch in batches:
+        out = torch.empty((batch,) + A.domain_shape, device=DEV)
+        plan.backward(out.data_ptr(), ys.data_ptr(), False, s, batch, out[0].numel(), ys[0].numel())
+        for k in range(batch):
+            assert torch.equal(out[k], want[k]), (batch, k)
+
+
+@pytest.mark.parametrize("nz", [1, 2, 3, 4, 7, 20, 24, 36, 41, 48, 61, 64])
+@pytest.mark.parametrize("pitch,pixels", [(1.3, 40), (0.8, 60), (0.55, 90)])
+def test_short_lines_match_oracle(nz, pitch, pixels):
+    """Lines of 1 to 64 (lanes per voxel column from 1 to 16, tiles of every width), two to four detector
+    columns per voxel. Tolerance: that of the flat kernels' own tests, 2e-6 of the result's norm."""
+    A = _operator((nz, 33, 29), (nz + 1, pixels), 21, pitch)
+    y = np.random.default_rng(nz).standard_normal(A.range_shape).astype(np.float32)
+    b = A.T(torch.from_numpy(y).to(DEV)).cpu().numpy()
+    assert rel_l2(b, oracle.bp(oracle.oracle_geometry(A.volume_geometry, A.projection_geometry), y)) <= 2e-6
+
+
+@pytest.mark.parametrize("nz", [1, 5, 30])
+def test_infinite_pixels_in_short_lines(nz):
+    A = _operator((nz, 24, 24), (nz, 36), 12, 1.3)
+    y = torch.zeros(A.range_shape, device=DEV)
+    y[nz // 2, 5, 18] = 1.0
+    met = A.T(y) > 0
+    y[nz // 2, 5, 18] = float("inf")
+    b = A.T(y)
+    assert met.any() and torch.equal(~torch.isfinite(b), met)

@@ -306,7 +306,6 @@ __global__ void __launch_bounds__(256) flat_splat(FlatMulti M)
         const int jc = j0 + c, w = w0 + tx;
         if (jc < v.cols && w < v.Wp) v.lines[((int64_t)k * v.cols + jc) * v.Wp + w] = tile[tx][c];
     }
-    if (j0 == 0 && k == 0) flat_zero_line(v.lines, (int64_t)v.kn * v.cols, v.Wp, w0);
 }
 
 // ---------------------------------------------------------------------------
@@ -682,18 +681,34 @@ __global__ void __launch_bounds__(64 * FLAT_BY) bp_flat(FlatMulti M)
     flat_write<ZL, FLAT_BX>(v, part, x0, y0 + wv, w, acc);
 }
 
-// The same without staging, for short lines (64 of w per wave, one per lane):
-// each wave reads the two (or NC) lines of every voxel column from global
-// memory. A line is then 256 bytes or less, its read from L1 takes no longer
-// than the 2 NC + 2 instructions that use it, and no barrier or staging
-// latency is left; the waves of small volumes hide each other's latency only
-// with many loads in flight. Columns without weight read the line of zeros
-// after the last one. 64^3, 96 angles, 64 x 96: 20 us, 16 slices of 256^2, 180
-// angles, 384 columns: 281 us (bp_flat 23 and 334).
-template <int NC>
-__global__ void __launch_bounds__(256) bp_flat_direct(FlatMulti M)
+// The same without staging, for short lines: a wave takes `rays` voxel columns
+// and `quads` lanes of V consecutive w for each, so that lines of any length
+// fill its lanes (one w per lane over 64 of them left 63 of 64 idle on a single
+// slice), a block four waves' columns in a tile. The weights
+// and places of up to 32 angles are formed by all lanes, a (column, angle) per
+// lane, and passed on through LDS; columns of no weight are read past the end
+// of the buffer, which gives zeros, so that an infinite pixel reaches no voxel
+// that its ray does not meet. The angle parts run in blocks of their own, or in
+// turn with their sums in registers, whose parts are then of a multiple of UN.
+//
+// Bound: the L1 port (two 16-byte loads of 16 cycles each per 64 lanes; its
+// address unit 81 % busy at 64 x 256^2). Whole backprojection, 180 angles,
+// pixel pitch 1, in brackets one w per lane: 256^2 46 us (250), 16 slices of it
+// 91 (260), 64 209 (290, kernel alone); 512^2 130 (870).
+// Columns along x of a block's tile of 4 rays (any shape takes the same time).
+__host__ __device__ inline int flat_tile(int rays) { return rays % 4 == 0 ? 16 : (rays % 2 == 0 ? 8 : 4); }
+
+template <int V, int NC>
+__global__ void __launch_bounds__(256) bp_flat_short(FlatMulti M)
 {
-    constexpr int AL = 4;
+    constexpr int EN = NC == 2 ? 512 : 256;  // (angle, column) entries of a wave at a time
+    constexpr int UN = NC == 2 ? 8 : 4;  // angles whose lines are in flight together
+    constexpr uint32_t NONE = 0x80000000u;
+    struct Entry {
+        float w[NC];
+        uint32_t at[NC];
+    };
+    __shared__ __align__(16) Entry entry[4][EN];
     const int logical = xcd_logical(M.shift);
     if (logical >= M.begin[M.n]) return;
     const int inst = owner_of(M.begin, logical);
@@ -703,48 +718,97 @@ __global__ void __launch_bounds__(256) bp_flat_direct(FlatMulti M)
     id /= v.bx;
     const int by = id % v.by;
     id /= v.by;
-    const int w0 = (id % v.chunks) * 64, part = id / v.chunks;
+    const int L = v.quads, R = v.rays, TX = flat_tile(R), rows = 4 * R / TX, cols = v.cols, Wp = v.Wp;
+    const int w0 = (id % v.chunks) * V * L, part = id / v.chunks;
     const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int x0 = bx * FLAT_BX, y = by * 4 + wv, kn = v.kn, cols = v.cols, Wp = v.Wp;
-    const int ka = part * v.part_len, kb = min(kn, ka + v.part_len);
-    const int w = w0 + lane;
-    const FlatAngle *ang = v.ang;
-    const float *src = v.lines + min(w, Wp - 1);
-    const int zero = kn * cols;
-    FlatVec<1> acc[FLAT_BX];
+    // (a block per angle part, or all parts in turn)
+    const int ka = v.partial ? part * v.part_len : 0, kb = v.partial ? min(v.kn, ka + v.part_len) : v.kn;
+    const int r = lane / L, w = w0 + (lane - r * L) * V;
+    const int t0 = wv * R;  // the wave's first column of the tile
+    const int x = bx * TX + (t0 + r) % TX, y = by * rows + (t0 + r) / TX;
+    const bool live = r < R && w < Wp;
+    const uint32_t lane_bytes = (uint32_t)w * 4u, line_bytes = (uint32_t)Wp * 4u, angle_bytes = (uint32_t)cols * line_bytes;
+    // angles whose entries are formed together; (angle, column) of the lane's first one, and the way to the next
+    const int NS = min(32, EN / R) / UN * UN;
+    const int h0 = lane / R, c0 = lane - h0 * R, step_h = 64 / R, step_c = 64 - step_h * R;
+    FlatVec<V> acc, sum;  // of the present part, of those before it
 #pragma unroll
-    for (int c = 0; c < FLAT_BX; ++c) acc[c].v[0] = 0.0f;
-    for (int k = ka; k < kb; k += AL) {
-        int row[NC];
-        float wt[NC];
-        {
-            const int ke = k + lane / FLAT_BX;
-            const FlatAngle &A = ang[min(ke, kn - 1)];
-            const double jc = flat_column(A, x0 + lane % FLAT_BX, y), j0 = flat_first<NC>(A, jc);
+    for (int z = 0; z < V; ++z) acc.v[z] = sum.v[z] = 0.0f;
+    int left = v.part_len;  // angles of the present part (a multiple of UN where several run in turn)
+    for (int k0 = ka; k0 < kb; k0 += NS) {
+        const int n = min(NS, kb - k0);
+        int h = h0, c = c0;
+        for (int e = lane; e < (n + UN - 1) / UN * UN * R; e += 64) {
+            Entry t;
+            const FlatAngle &A = v.ang[min(k0 + h, kb - 1)];
+            const double jc = flat_column(A, bx * TX + (t0 + c) % TX, by * rows + (t0 + c) / TX);
+            const double j0 = flat_first<NC>(A, jc);
 #pragma unroll
-            for (int e = 0; e < NC; ++e) {
-                const int j = (int)j0 + e;
-                wt[e] = ke < kb && (unsigned)j < (unsigned)cols ? flat_weight(A, j0, jc, e) : 0.0f;
-                row[e] = wt[e] > 0.0f ? ke * cols + j : zero;
+            for (int i = 0; i < NC; ++i) {
+                const int j = (int)j0 + i;
+                const float f = flat_weight(A, j0, jc, i);
+                const bool some = h < n && f > 0.0f && (unsigned)j < (unsigned)cols;
+                t.w[i] = some ? f : 0.0f;
+                t.at[i] = some ? (uint32_t)h * angle_bytes + (uint32_t)j * line_bytes : NONE;
+            }
+            entry[wv][e] = t;
+            c += step_c;
+            h += step_h;
+            if (c >= R) {
+                c -= R;
+                ++h;
             }
         }
+        const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
+            (void *)(v.lines + (int64_t)k0 * cols * Wp), (short)0, (int)((uint32_t)n * angle_bytes), 0x00020000);
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        if (live) {
+            const Entry *in = entry[wv] + r;
+            for (int h = 0; h < n; h += UN) {
+                Entry t[UN];
+                FlatVec<V> u[UN][NC];
 #pragma unroll
-        for (int h = 0; h < AL; ++h) {
-            float u[FLAT_BX][NC];
+                for (int e = 0; e < UN; ++e) t[e] = in[(h + e) * R];
 #pragma unroll
-            for (int c = 0; c < FLAT_BX; ++c)
+                for (int e = 0; e < UN; ++e)
 #pragma unroll
-                for (int e = 0; e < NC; ++e) u[c][e] = src[(int64_t)lane_i(row[e], h * FLAT_BX + c) * Wp];
-            __builtin_amdgcn_sched_barrier(0);
+                    for (int i = 0; i < NC; ++i) u[e][i] = flat_bload<V>(rs, t[e].at[i] + lane_bytes);
+                __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-            for (int c = 0; c < FLAT_BX; ++c)
+                for (int e = 0; e < UN; ++e)
 #pragma unroll
-                for (int e = 0; e < NC; ++e)
-                    acc[c].v[0] = fmaf(lane_f(wt[e], h * FLAT_BX + c), u[c][e], acc[c].v[0]);
-            __builtin_amdgcn_sched_barrier(0);
+                    for (int i = 0; i < NC; ++i)
+#pragma unroll
+                        for (int z = 0; z < V; ++z) acc.v[z] = fmaf(t[e].w[i], u[e][i].v[z], acc.v[z]);
+                __builtin_amdgcn_sched_barrier(0);
+                left -= UN;
+                if (left == 0) {
+                    left = v.part_len;
+#pragma unroll
+                    for (int z = 0; z < V; ++z) {
+                        sum.v[z] += acc.v[z];
+                        acc.v[z] = 0.0f;
+                    }
+                }
+            }
         }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
     }
-    flat_write<1, FLAT_BX>(v, part, x0, y, w, acc);
+#pragma unroll
+    for (int z = 0; z < V; ++z) acc.v[z] = sum.v[z] + acc.v[z];
+    if (!live || x >= v.nx || y >= v.ny) return;
+#pragma unroll
+    for (int z = 0; z < V; ++z) {
+        if (w + z >= v.W) break;
+        const int b = (w + z) / v.nz, iz = (w + z) - b * v.nz;
+        const int64_t o = ((int64_t)iz * v.ny + y) * v.nx + x;
+        if (v.partial)
+            v.partial[((int64_t)b * v.parts + part) * ((int64_t)v.nx * v.ny * v.nz) + o] = acc.v[z];
+        else
+            emit(v.vol + b * v.vs, o, b, acc.v[z], v.ep);
+    }
 }
 
 // The sums of the angle parts added in order and written through the
@@ -789,9 +853,10 @@ inline FlatKernel bp_flat_kernel(int zl, int nc)
     return nc == 2 ? bp_flat<2, 2> : (nc == 3 ? bp_flat<2, 3> : bp_flat<2, 4>);
 }
 
-inline FlatKernel bp_flat_direct_kernel(int nc)
+inline FlatKernel bp_flat_short_kernel(int v, int nc)
 {
-    return nc == 2 ? bp_flat_direct<2> : (nc == 3 ? bp_flat_direct<3> : bp_flat_direct<4>);
+    if (v == 4) return nc == 2 ? bp_flat_short<4, 2> : (nc == 3 ? bp_flat_short<4, 3> : bp_flat_short<4, 4>);
+    return nc == 2 ? bp_flat_short<1, 2> : (nc == 3 ? bp_flat_short<1, 3> : bp_flat_short<1, 4>);
 }
 
 }  // namespace tsx

@@ -993,9 +993,11 @@ bool fp_refined(const tsx_plan *p)
 // The choice only cuts the work into blocks: no result depends on it.
 struct FlatPlan {
     bool ok = false;
-    int v = 4, quads = 1, rays = 1;  // forward: w per lane, lanes per ray, rays per wave
-    int zl = 1;      // backward: consecutive w per lane
-    bool direct = false;  // backward, short lines: the kernel without staging
+    // forward: w per lane, lanes per ray, rays per wave; backward, short lines:
+    // w per lane, lanes per voxel column, voxel columns per wave
+    int v = 4, quads = 1, rays = 1;
+    bool shrt = false;  // backward: the kernel of short lines
+    int zl = 2;      // backward, the others: consecutive w per lane
     int stage = 0;   // backward: columns staged at a time
     int chunks = 1;  // chunks of w
     int per_launch = 0;  // angles per launch
@@ -1010,10 +1012,15 @@ int64_t flat_pitch(const tsx_plan *p, int64_t batch)
     return W < 4 ? W : (W + 3) / 4 * 4;
 }
 
-// Backward, lanes: the fewest w per lane that cover W in one chunk, at most 4
-// (W = 64: 1, on the kernels without staging; 128: 2). Fewer w per lane than
-// that cost more instructions per w.
-int flat_zl(int64_t W) { return W > 128 ? 4 : (W > 64 ? 2 : 1); }
+// Backward, staged lines: the fewest w per lane that cover W in one chunk, at
+// most 4. Fewer w per lane than that cost more instructions per w.
+int flat_zl(int64_t W) { return W > 128 ? 4 : 2; }
+
+// Backward: whether lines of W take the kernel of short lines (staged lines
+// leave lanes idle there; 256^2, 180 angles: W = 16 91 and 323 us, 64 209 and
+// 373, 100 409 and 385; 128^2, 90 angles: 64 64 and 70, 70 80 and 70), which
+// addresses 32 angles with 31 bits.
+bool flat_short(const tsx_plan *p, int64_t W) { return W <= 64 && p->cols * ((W + 3) / 4 * 4) < (int64_t)1 << 24; }
 
 // The turned volume and its line of zeros.
 int64_t flat_turned_elems(const tsx_plan *p, int64_t batch)
@@ -1103,14 +1110,14 @@ bool flat_bp_ok(const tsx_plan *p)
         p->flat_nc > 4 || p->flat_stage_bp > FLAT_BSC)
         return false;
     const int64_t sums = bp_parts_of(p) > 1 ? (int64_t)bp_parts_of(p) * p->nx * p->ny * p->nz * 4 + 256 : 0;
-    const int64_t lines = ((int64_t)bp_chunk_of(p) * p->cols + 1) * flat_pitch(p, 1) * 4;
+    const int64_t lines = (int64_t)bp_chunk_of(p) * p->cols * flat_pitch(p, 1) * 4;
     const int64_t buffer = TSX_NOALLOC_SCRATCH_BYTES - p->outer[TSX_OP_BP];
     return lines + sums <= buffer || bp_workspace_elems(p) * 4 + sums > buffer;
 }
 
 int64_t flat_line_elems(const tsx_plan *p, int64_t batch)
 {
-    return flat_bp_ok(p) ? ((int64_t)bp_chunk_of(p) * p->cols + 1) * flat_pitch(p, batch) : 0;
+    return flat_bp_ok(p) ? (int64_t)bp_chunk_of(p) * p->cols * flat_pitch(p, batch) : 0;
 }
 
 // Blocks of the backprojector (by: voxel columns per block along y).
@@ -1124,11 +1131,19 @@ FlatPlan flat_bp(const tsx_plan *p, int64_t batch)
     FlatPlan f;
     const int64_t W = p->nz * batch;
     if (!flat_bp_ok(p) || W > (1 << 28)) return f;
-    f.zl = flat_zl(W);
-    f.direct = f.zl == 1;
-    f.chunks = (int)((W + 64 * f.zl - 1) / (64 * f.zl));
-    f.stage = p->flat_stage_bp;
-    f.lds = f.direct ? 0 : (size_t)2 * (f.stage + 1) * f.zl * 256;
+    f.shrt = flat_short(p, W);
+    if (f.shrt) {
+        f.v = W < 4 ? 1 : 4;
+        const int q = (int)(flat_pitch(p, batch) / f.v);
+        f.chunks = (q + 31) / 32;
+        f.quads = (q + f.chunks - 1) / f.chunks;
+        f.rays = 64 / f.quads;
+    } else {
+        f.zl = flat_zl(W);
+        f.chunks = (int)((W + 64 * f.zl - 1) / (64 * f.zl));
+        f.stage = p->flat_stage_bp;
+        f.lds = (size_t)2 * (f.stage + 1) * f.zl * 256;
+    }
     f.per_launch = bp_chunk_of(p);
     f.ok = true;
     return f;
@@ -1150,7 +1165,8 @@ int flat_part_len(const tsx_plan *p)
     const int64_t blocks = std::min<int64_t>(128, flat_blocks(p, 8, (p->nz + 64 * zl - 1) / (64 * zl)));
     const int64_t len = std::max<int64_t>(4, ((int64_t)p->n_angles * blocks + 255) / 256);
     const int64_t least = (int64_t)std::ceil(std::cbrt(0.25 * p->n_angles * p->n_angles));
-    return (int)std::max<int64_t>(cut, std::min(len, least));
+    const int64_t part = (std::max<int64_t>(cut, std::min(len, least)) + 7) / 8 * 8;  // (groups of bp_flat_short)
+    return (int)std::min<int64_t>(part, p->n_angles);
 }
 
 // (least: as for fp_elems)
@@ -1602,22 +1618,37 @@ struct FlatBatch {
     {
         int rc = pass(flat_splat, flat_splat_blocks);
         if (rc) return rc;
-        int64_t ve = 0;
-        int entries = 0;
-        bool sums = false;
-        const int by = f.direct ? 4 : FLAT_BY;
+        int64_t ve = 0, blocks = 0;
+        int entries = 0, angles = 0;
+        double sums = 0.0;  // floats of the parts' sums
         for (int k = 0; k < m.n; ++k) {
             FlatView &v = m.v[k];
-            v.bx = (v.nx + FLAT_BX - 1) / FLAT_BX;
+            const int bx = f.shrt ? flat_tile(v.rays) : FLAT_BX, by = f.shrt ? 4 * v.rays / bx : FLAT_BY;
+            v.bx = (v.nx + bx - 1) / bx;
             v.by = (v.ny + by - 1) / by;
-            sums = sums || v.partial;
+            blocks += (int64_t)v.bx * v.by * v.chunks;
             ve = std::max(ve, (int64_t)v.nx * v.ny * v.nz);
             entries = std::max(entries, v.W / v.nz);
+            angles = std::max(angles, v.kn);
+            if (v.partial) sums += (double)v.nx * v.ny * v.W * v.parts;
         }
-        rc = main_pass(f.direct ? bp_flat_direct_kernel(nc) : bp_flat_kernel(f.zl, nc), by, 10, 2048,
+        // Short lines: parts in turn within a block (same bits) rather than in
+        // blocks of their own where the sums to write and read, 4e-6 us a float
+        // and 4 us for the reduction, cost more than the idle CUs, 0.1 us an angle
+        // for the part of four blocks per CU that is missing. Measured, in turn
+        // and apart: 64^3, 90 angles 21 and 26 us, 16 of them 140 and 199; 64^3,
+        // 360 angles 56 and 53; 256^2, 180 angles 69 and 45, 16 slices of it 77 and 82.
+        if (f.shrt && 4e-6 * sums + 4.0 > 0.1 * angles * std::max(0.0, 1.0 - blocks / 1024.0))
+            for (int k = 0; k < m.n; ++k) {
+                m.v[k].partial = nullptr;
+                m.v[k].parts = 1;
+                sums = 0.0;
+            }
+        rc = main_pass(f.shrt ? bp_flat_short_kernel(f.v, nc) : bp_flat_kernel(f.zl, nc), f.shrt ? 4 : FLAT_BY, 10, 2048,
                        [](const FlatView &v) { return (int64_t)v.bx * v.by * v.chunks * v.parts; });
-        if (rc || !sums) return rc;
-        hipLaunchKernelGGL(flat_parts_reduce, dim3((unsigned)((ve + FLAT_REDUCE - 1) / FLAT_REDUCE), (unsigned)entries, (unsigned)m.n),
+        if (rc || sums == 0.0) return rc;
+        hipLaunchKernelGGL(flat_parts_reduce,
+                           dim3((unsigned)((ve + FLAT_REDUCE - 1) / FLAT_REDUCE), (unsigned)entries, (unsigned)m.n),
                            dim3(256), 0, stream, m);
         TSX_HIP_CHECK(hipGetLastError());
         return TSX_OK;
@@ -1999,7 +2030,7 @@ bool flat_one_launch(const tsx_plan *p, int op)
     if (op == TSX_OP_FP && (fp_refined(p) || fp_swapped(p))) return false;
     if (op == TSX_OP_BP && (bp_refined(p) || p->perm)) return false;
     return f.ok && f.per_launch >= p->n_angles && std::max(tiles, turn) <= most &&
-           flat_blocks(p, 4, f.chunks) * bp_parts_of(p) <= most;
+           (int64_t)p->nx * p->ny * f.chunks * bp_parts_of(p) <= 4 * most;
 }
 
 // Scratch of a fused launch: each instance's workspace.
@@ -2233,7 +2264,7 @@ int multi_bp(const tsx_plan *const *plans, float *const *vols, const float *cons
             if (taken[e] || !flat_one_launch(plans[e], TSX_OP_BP)) continue;
             const tsx_plan *p = plans[e];
             const FlatPlan fe = flat_bp(p, 1);
-            if (fe.zl != f.zl || p->flat_nc != plans[k]->flat_nc) continue;
+            if (fe.shrt != f.shrt || (f.shrt ? fe.v != f.v : fe.zl != f.zl) || p->flat_nc != plans[k]->flat_nc) continue;
             taken[e] = 1;
             FlatView &v = fb.m.v[fb.m.n++];
             v = flat_view(p, fe, 1, 0, p->n_angles, eps[e]);
