@@ -28,7 +28,6 @@
 namespace tsx {
 
 constexpr int FLAT_MAX = MAX_FUSED;  // instances of one launch
-constexpr int FLAT_RAYS = 32;        // forward projector: most rays per wave
 constexpr int FLAT_STRIP = 8;        // forward projector: column tiles per strip
 // forward: slices (n / FLAT_SUM of the volume) summed before they join the rest of a ray's sum.
 // One running sum over the 256 slices of a slice stack rounds to 3.6e-7 of the result, the
@@ -46,7 +45,7 @@ struct FlatView {
     int W, Wp;              // batch entries x nz, and the pitch of a line
     float *vol, *proj;      // caller's data: read or written, entries vs and ps floats apart
     int64_t vs, ps;
-    float *turned;          // forward: the volume as [x][y][Wp]
+    float *turned, *across; // forward: the volume as [x][y][Wp], and as [y][x][Wp] (or null)
     float *lines;           // G or U as [kn][cols][Wp]
     Epilogue ep;
     int up;                 // backward: pixels per coarse pixel edge (refined detector), else 1
@@ -101,22 +100,6 @@ __device__ __forceinline__ void flat_store(float *p, const FlatVec<ZL> &r)
         *p = r.v[0];
 }
 
-// A line's values = r (first) or += r; r = 0 after it.
-template <int ZL>
-__device__ __forceinline__ void flat_join(float *p, FlatVec<ZL> &r, bool first)
-{
-    FlatVec<ZL> t;
-#pragma unroll
-    for (int z = 0; z < ZL; ++z) t.v[z] = 0.0f;
-    if (!first) t = flat_load<ZL>(p);
-#pragma unroll
-    for (int z = 0; z < ZL; ++z) {
-        t.v[z] += r.v[z];
-        r.v[z] = 0.0f;
-    }
-    flat_store<ZL>(p, t);
-}
-
 __device__ __forceinline__ float lane_f(float v, int lane)
 {
     return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), lane));
@@ -128,8 +111,8 @@ __device__ __forceinline__ int lane_i(int v, int lane) { return __builtin_amdgcn
 // layout passes: 32 x 32 tiles through LDS, blocks of 32 x 8 threads
 // ---------------------------------------------------------------------------
 
-// turned[x][y][w] from vol[z][y][x] of every entry: a block per tile of 32 x
-// by 32 w of one y.
+// turned[x][y][w], and across[y][x][w] where it is asked for, from vol[z][y][x]
+// of every entry: a block per tile of 32 x by 32 w of one y.
 __host__ __device__ inline int64_t flat_turn_blocks(const FlatView &v)
 {
     return (int64_t)((v.nx + 31) / 32) * ((v.W + 31) / 32) * v.ny;
@@ -164,9 +147,15 @@ __global__ void __launch_bounds__(256) flat_turn(FlatMulti M)
     __syncthreads();
     for (int r = ty; r < 32; r += 8) {
         const int x = x0 + r, w = w0 + tx;
-        if (x < v.nx && w < v.Wp) v.turned[((int64_t)x * v.ny + y) * v.Wp + w] = tile[tx][r];
+        if (x < v.nx && w < v.Wp) {
+            v.turned[((int64_t)x * v.ny + y) * v.Wp + w] = tile[tx][r];
+            if (v.across) v.across[((int64_t)y * v.nx + x) * v.Wp + w] = tile[tx][r];
+        }
     }
-    if (x0 == 0 && y == 0) flat_zero_line(v.turned, (int64_t)v.nx * v.ny, v.Wp, w0);
+    if (x0 == 0 && y == 0) {
+        flat_zero_line(v.turned, (int64_t)v.nx * v.ny, v.Wp, w0);
+        if (v.across) flat_zero_line(v.across, (int64_t)v.nx * v.ny, v.Wp, w0);
+    }
 }
 
 // y[i, a, j] = l lerp_t G[a, j, .] through the epilogue: a block per tile of
@@ -316,19 +305,26 @@ __device__ __forceinline__ FlatVec<V> flat_bload(__amdgpu_buffer_rsrc_t rs, uint
 {
     if constexpr (V == 4)
         return __builtin_bit_cast(FlatVec<4>, __builtin_amdgcn_raw_buffer_load_b128(rs, bytes, 0, 0));
+    else if constexpr (V == 2)
+        return __builtin_bit_cast(FlatVec<2>, __builtin_amdgcn_raw_buffer_load_b64(rs, bytes, 0, 0));
     else
         return __builtin_bit_cast(FlatVec<1>, __builtin_amdgcn_raw_buffer_load_b32(rs, bytes, 0, 0));
 }
 
-// A wave takes `rays` neighbouring detector columns of one angle and 4 quads
-// of w (lane: ray lane / quads, V = 4 consecutive w at 4 (lane % quads); V = 1
-// on lines of fewer than 4 w), a block four neighbouring angles, whose rays
-// meet nearly the same voxel columns. Slice by slice every ray takes the two
-// voxel columns beside it straight from memory (the line of zeros after the
-// last one where they lie beyond the volume), with the weights and addresses
-// of up to 32 slices formed by all lanes (FP64 positions) and passed on through
-// LDS. The launch goes through chunks of at most 80 of w, in a chunk through strips
-// of 8 column tiles, in a strip through the angles: the blocks that an XCD runs
+// A wave takes `rays` neighbouring detector columns of one angle and V quads
+// of w (lane: ray lane / quads, V consecutive w at V (lane % quads); V = 1 and
+// 2 on lines of one and two w). Slice by slice every ray takes the two voxel
+// columns beside it straight from memory (the line of zeros after the last one
+// where they lie beyond the volume). Where a ray has several lanes, the weights
+// and addresses of up to 32 slices are formed by all lanes (FP64 positions) and
+// passed on through LDS; where it has one (OWN), that lane forms its own.
+// Slices are summed in groups of FLAT_SUM, whose sums are added in order.
+//
+// A block takes four neighbouring angles, whose rays meet nearly the same voxel
+// columns, or one angle, whose groups its four waves take in turn (SPLIT: few
+// rays, which would leave the chip waiting on one wave's loads per SIMD). The
+// launch goes through chunks of at most 80 of w, in a chunk through strips of 8
+// column tiles, in a strip through the angles: the blocks that an XCD runs
 // together meet few voxel columns, so that its L2 holds them (512^3, 360
 // angles: 9.9 ms; angles before tiles, chunks of 256 of w: 19.4 ms).
 //
@@ -340,120 +336,173 @@ __device__ __forceinline__ FlatVec<V> flat_bload(__amdgpu_buffer_rsrc_t rs, uint
 //   256^3, 360 angles    2.17 (3.39) and 1.11 (1.43) ms
 //   512^3, 360 angles    15.4 and 10.0 ms
 //   75 x 441 x 441, 361  1.79 (2.81) and 1.28 (1.44) ms
-//   16 x (256 x 256), 180 angles 0.64 and 0.09 ms; one slice 69 and 74 us
+//   16 x (256 x 256), 180 angles 123 (137) and 69 (77) us
+//   1 x (256 x 256), 180 angles 60 (68) and 36 (35) us, 4 of them 65 (74) and 37 (41)
+//   1 x (512 x 512), 360 angles 292 (372) and 141 (127) us
+//   2 x (1024 x 1024), 720 angles 1.15 (1.32) and 0.73 (0.89) ms
 // Taken back: lines staged in LDS by blocks that go through the slices in step
 // (a barrier per slice: 200^3, 360 angles, pitch sqrt 2 1.07 ms against 0.72
 // here; few blocks on small volumes: 80^3, 60 angles 0.09 against 0.03); one ray
 // per wave with weights from readlane (1.15 ms).
-template <int V>
+template <int V, bool OWN, bool SPLIT>
 __global__ void __launch_bounds__(256) fp_flat(FlatMulti M)
 {
-    constexpr int EN = 256;  // (ray, slice) entries of a wave at a time
-    constexpr int UN = 8;    // slices whose columns are in flight together
-    __shared__ float4 entry[4][EN];
+    constexpr int UN = 8;  // slices whose columns are in flight together
+    extern __shared__ __align__(16) float flat_lds[];
     const int logical = xcd_logical(M.shift);
     if (logical >= M.begin[M.n]) return;
     const int inst = owner_of(M.begin, logical);
     const FlatView &v = M.v[inst];
     const int id = logical - M.begin[inst];
-    const int cols = v.cols, Wp = v.Wp, L = v.quads, R = v.rays;
-    const int tiles = (cols + R - 1) / R, ks = (v.kn + 3) / 4;
+    const int cols = v.cols, Wp = v.Wp, L = OWN ? 1 : v.quads, R = v.rays, NS = OWN ? UN : v.stage;
+    const int tiles = (cols + R - 1) / R, ks = SPLIT ? v.kn : (v.kn + 3) / 4;
     const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     constexpr int T = FLAT_STRIP;
     const int per = ks * tiles, chunk = id / per, in_chunk = id - chunk * per;
     const int strip = in_chunk / (ks * T), width = min(T, tiles - strip * T), in_strip = in_chunk - strip * ks * T;
-    const int jb = (strip * T + in_strip % width) * R, w0 = chunk * V * L, k = in_strip / width * 4 + wv;
-    if (k >= v.kn) return;
+    const int jb = (strip * T + in_strip % width) * R, w0 = chunk * V * L;
+    const int k = SPLIT ? in_strip / width : in_strip / width * 4 + wv;
+    if (k >= v.kn) return;  // (never with SPLIT, whose waves meet at barriers)
+    float4 *entry = reinterpret_cast<float4 *>(flat_lds) + wv * NS * R;
     typedef const __attribute__((address_space(4))) FlatAngle ConstAngle;
     ConstAngle &A = ((ConstAngle *)v.ang)[k];
     const int m = A.m;
     const int nm = m == 0 ? v.nx : v.ny, nc = m == 0 ? v.ny : v.nx;
-    const int sn = m == 0 ? v.ny : 1, sc = m == 0 ? 1 : v.ny;  // voxel column (n, c) is n sn + c sc
+    const bool turned = m == 0 || !v.across;
+    // voxel column (n, c) is n sn + c sc
+    const int sn = m == 0 ? v.ny : (turned ? 1 : v.nx), sc = m == 0 || !turned ? 1 : v.ny;
     const int nref = nm / 2, zero = v.nx * v.ny;
     // the ray of column j: q(n) = base + j qj + (n - nref) qm, slices with q in (-1, nc)
     const double base = fma(A.qm, (double)nref, A.q0);
+    const auto ray_at = [&](int ray) {  // (held where the voxel columns' numbers are exact)
+        return fmin(fmax(fma(A.qj, (double)min(jb + ray, cols - 1), base), -1e8), 1e8);
+    };
+    const double Rd = ray_at(lane % R);
     int lo = 0, hi = nm - 1;
-    {
-        const double Rd = fma(A.qj, (double)min(jb + lane % R, cols - 1), base);
-        if (A.qm != 0.0) {
-            const double t0 = (-1.0 - Rd) / A.qm, t1 = ((double)nc - Rd) / A.qm;
-            lo = max(0, (int)fmax(ceil(fmin(t0, t1) + nref), -1e9));
-            hi = min(nm - 1, (int)fmin(floor(fmax(t0, t1) + nref), 1e9));
-        } else if (!(Rd > -1.0 && Rd < (double)nc)) {
-            lo = nm;
-            hi = -1;
-        }
-        if (lo > hi) {
-            lo = nm;
-            hi = -1;
-        }
+    if (A.qm != 0.0) {
+        const double t0 = (-1.0 - Rd) / A.qm, t1 = ((double)nc - Rd) / A.qm;
+        lo = max(0, (int)fmin(fmax(ceil(fmin(t0, t1) + nref), -1e9), 1e9));
+        hi = min(nm - 1, (int)fmax(fmin(floor(fmax(t0, t1) + nref), 1e9), -1e9));
+    } else if (!(Rd > -1.0 && Rd < (double)nc)) {
+        hi = -1;
+    }
+    if (lo > hi) {
+        lo = nm;
+        hi = -1;
     }
     lo = __builtin_amdgcn_readfirstlane(wave_min(lo));
     hi = __builtin_amdgcn_readfirstlane(wave_max(hi));
     const int r = lane / L, w = w0 + (lane - r * L) * V;
     const bool live = r < R && w < Wp;
     const uint32_t lane_bytes = (uint32_t)w * 4u, line_bytes = (uint32_t)Wp * 4u;
+    const uint32_t n_bytes = (uint32_t)sn * line_bytes, c_bytes = (uint32_t)sc * line_bytes, none = (uint32_t)zero * line_bytes;
     const __amdgpu_buffer_rsrc_t rs =
-        __builtin_amdgcn_make_buffer_rsrc((void *)v.turned, (short)0, (int)((uint32_t)(zero + 1) * line_bytes), 0x00020000);
-    FlatVec<V> acc;
-#pragma unroll
-    for (int z = 0; z < V; ++z) acc.v[z] = 0.0f;
-    float *out = v.lines + ((int64_t)k * cols + jb + r) * Wp + w;
-    bool first = true;
-    auto flush = [&]() {
-        if (live && jb + r < cols) flat_join<V>(out, acc, first);
-        first = false;
+        __builtin_amdgcn_make_buffer_rsrc((void *)(turned ? v.turned : v.across), (short)0,
+                                          (int)((uint32_t)(zero + 1) * line_bytes), 0x00020000);
+    // weight and addresses of the two voxel columns beside a ray in slice n (byte offset at)
+    const bool narrow = c_bytes < 1u << 24 && nc < 1 << 24;
+    const auto place = [&](double q, uint32_t at, bool inside, float &wh, uint32_t &ra, uint32_t &rb) {
+        const double f = floor(q);
+        const int c = (int)f;
+        wh = (float)(q - f);
+        rb = at + (narrow ? __umul24((uint32_t)(c + 1), c_bytes) : (uint32_t)(c + 1) * c_bytes);
+        ra = inside && (unsigned)c < (unsigned)nc ? rb - c_bytes : none;
+        rb = inside && (unsigned)(c + 1) < (unsigned)nc ? rb : none;
     };
-    // slices whose entries are formed together (a power of two from UN to FLAT_SUM; NS R <= EN)
-    const int NS = R <= 8 ? 32 : (R <= 16 ? 16 : 8);
+    // acc += the slices of (1 - wh, wh, ra, rb)
+    const auto sample = [&](const float4 (&t)[UN], FlatVec<V> &acc) {
+        FlatVec<V> a[UN], b[UN];
+#pragma unroll
+        for (int e = 0; e < UN; ++e) {
+            a[e] = flat_bload<V>(rs, __builtin_bit_cast(uint32_t, t[e].z) + lane_bytes);
+            b[e] = flat_bload<V>(rs, __builtin_bit_cast(uint32_t, t[e].w) + lane_bytes);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int e = 0; e < UN; ++e)
+#pragma unroll
+            for (int z = 0; z < V; ++z) acc.v[z] = fmaf(t[e].y, b[e].v[z], fmaf(t[e].x, a[e].v[z], acc.v[z]));
+        __builtin_amdgcn_sched_barrier(0);
+    };
     // (ray, slice) of the lane's first entry of a step, and the way from one to the next
     const int h0 = lane / R, ray0 = lane - h0 * R, step_h = 64 / R, step_r = 64 - step_h * R;
-    for (int n0 = lo / NS * NS; n0 <= hi; n0 += NS) {
-        int h = h0, ray = ray0;
-        for (int e = lane; e < NS * R; e += 64) {
-            const int n = n0 + h;
-            const double Rd = fma(A.qj, (double)min(jb + ray, cols - 1), base);
-            const double q = fma((double)(n - nref), A.qm, Rd), f = floor(q);
-            ray += step_r;
-            h += step_h;
-            if (ray >= R) {
-                ray -= R;
-                ++h;
-            }
-            const float wh = (float)(q - f);
-            const int c = (int)fmin(fmax(f, -1e8), 1e8);
-            const uint32_t ra = (uint32_t)(n < nm && (unsigned)c < (unsigned)nc ? n * sn + c * sc : zero) * line_bytes;
-            const uint32_t rb =
-                (uint32_t)(n < nm && (unsigned)(c + 1) < (unsigned)nc ? n * sn + (c + 1) * sc : zero) * line_bytes;
-            entry[wv][e] = make_float4(1.0f - wh, wh, __builtin_bit_cast(float, ra), __builtin_bit_cast(float, rb));
-        }
-        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        if (live) {
-            const float4 *in = entry[wv] + r;
-            for (int h = 0; h < NS && n0 + h <= hi; h += UN) {
-                float4 t[UN];
-                FlatVec<V> a[UN], b[UN];
+    // the sum over the slices of one group of FLAT_SUM
+    const auto group = [&](int g, FlatVec<V> &acc) {
 #pragma unroll
-                for (int e = 0; e < UN; ++e) t[e] = in[(h + e) * R];
+        for (int z = 0; z < V; ++z) acc.v[z] = 0.0f;
+        const int end = min(hi, g * FLAT_SUM + FLAT_SUM - 1);
+        for (int n0 = max(g * FLAT_SUM, lo / NS * NS); n0 <= end; n0 += NS) {
+            if constexpr (OWN) {
+                if (!live) continue;
+                const double dn = (double)(n0 - nref);
+                float4 t[UN];
 #pragma unroll
                 for (int e = 0; e < UN; ++e) {
-                    a[e] = flat_bload<V>(rs, __builtin_bit_cast(uint32_t, t[e].z) + lane_bytes);
-                    b[e] = flat_bload<V>(rs, __builtin_bit_cast(uint32_t, t[e].w) + lane_bytes);
+                    float wh;
+                    uint32_t ra, rb;
+                    place(fma(dn + (double)e, A.qm, Rd), (uint32_t)(n0 + e) * n_bytes, n0 + e <= end, wh, ra, rb);
+                    t[e] = make_float4(1.0f - wh, wh, __builtin_bit_cast(float, ra), __builtin_bit_cast(float, rb));
                 }
-                __builtin_amdgcn_sched_barrier(0);
+                sample(t, acc);
+            } else {
+                int h = h0, ray = ray0;
+                for (int e = lane; e < NS * R; e += 64) {
+                    const int n = n0 + h;
+                    float wh;
+                    uint32_t ra, rb;
+                    place(fma((double)(n - nref), A.qm, step_r ? ray_at(ray) : Rd), (uint32_t)n * n_bytes, n <= end, wh, ra, rb);
+                    entry[e] = make_float4(1.0f - wh, wh, __builtin_bit_cast(float, ra), __builtin_bit_cast(float, rb));
+                    ray += step_r;
+                    h += step_h;
+                    if (ray >= R) {
+                        ray -= R;
+                        ++h;
+                    }
+                }
+                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                __builtin_amdgcn_wave_barrier();
+                if (live) {
+                    const float4 *in = entry + r;
+                    for (int h = 0; h < NS && n0 + h <= end; h += UN) {
+                        float4 t[UN];
 #pragma unroll
-                for (int e = 0; e < UN; ++e)
-#pragma unroll
-                    for (int z = 0; z < V; ++z) acc.v[z] = fmaf(t[e].y, b[e].v[z], fmaf(t[e].x, a[e].v[z], acc.v[z]));
-                __builtin_amdgcn_sched_barrier(0);
+                        for (int e = 0; e < UN; ++e) t[e] = in[(h + e) * R];
+                        sample(t, acc);
+                    }
+                }
+                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                __builtin_amdgcn_wave_barrier();
             }
         }
-        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        if ((n0 + NS) % FLAT_SUM == 0) flush();
+    };
+    FlatVec<V> sum;  // of the groups, in their order
+#pragma unroll
+    for (int z = 0; z < V; ++z) sum.v[z] = 0.0f;
+    const int last = hi / FLAT_SUM;
+    if constexpr (SPLIT) {
+        // a group per wave; their sums are added in order by the first wave
+        FlatVec<V> *part = reinterpret_cast<FlatVec<V> *>(flat_lds + (OWN ? 0 : 4 * 4 * NS * R));
+        int buf = 0;
+        for (int g = lo / FLAT_SUM; lo <= hi && g <= last; g += 4, buf ^= 1) {
+            FlatVec<V> acc;
+            group(g + wv, acc);  // (past the last one: nothing)
+            part[(buf * 4 + wv) * 64 + lane] = acc;
+            __syncthreads();
+            if (wv == 0)
+                for (int s = 0; s < 4 && g + s <= last; ++s)
+#pragma unroll
+                    for (int z = 0; z < V; ++z) sum.v[z] += part[(buf * 4 + s) * 64 + lane].v[z];
+        }
+        if (wv != 0) return;
+    } else {
+        for (int g = lo / FLAT_SUM; lo <= hi && g <= last; ++g) {
+            FlatVec<V> acc;
+            group(g, acc);
+#pragma unroll
+            for (int z = 0; z < V; ++z) sum.v[z] += acc.v[z];
+        }
     }
-    if (lo > hi || (hi / NS + 1) * NS % FLAT_SUM) flush();
+    if (live && jb + r < cols) flat_store<V>(v.lines + ((int64_t)k * cols + jb + r) * Wp + w, sum);
 }
 
 // ---------------------------------------------------------------------------
@@ -846,6 +895,14 @@ __global__ void __launch_bounds__(256) flat_parts_reduce(FlatMulti M)
 }
 
 using FlatKernel = void (*)(FlatMulti);
+
+inline FlatKernel fp_flat_kernel(int v, bool own, bool split)
+{
+    if (!own) return split ? fp_flat<4, false, true> : fp_flat<4, false, false>;
+    if (v == 4) return split ? fp_flat<4, true, true> : fp_flat<4, true, false>;
+    if (v == 2) return split ? fp_flat<2, true, true> : fp_flat<2, true, false>;
+    return split ? fp_flat<1, true, true> : fp_flat<1, true, false>;
+}
 
 inline FlatKernel bp_flat_kernel(int zl, int nc)
 {

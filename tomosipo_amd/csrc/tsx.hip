@@ -997,19 +997,19 @@ struct FlatPlan {
     // w per lane, lanes per voxel column, voxel columns per wave
     int v = 4, quads = 1, rays = 1;
     bool shrt = false;  // backward: the kernel of short lines
+    bool own = false;    // forward: a lane per ray
     int zl = 2;      // backward, the others: consecutive w per lane
-    int stage = 0;   // backward: columns staged at a time
+    int stage = 0;   // forward: slices per step; backward: columns staged at a time
     int chunks = 1;  // chunks of w
     int per_launch = 0;  // angles per launch
     size_t lds = 0;
 };
 
-// Pitch of a line of w: a multiple of 4, and of the forward projector's 16-byte
-// loads, unless the line is shorter.
+// Pitch of a line of w: 1, 2 or a multiple of 4, as the loads take them.
 int64_t flat_pitch(const tsx_plan *p, int64_t batch)
 {
     const int64_t W = p->nz * batch;
-    return W < 4 ? W : (W + 3) / 4 * 4;
+    return W < 3 ? W : (W + 3) / 4 * 4;
 }
 
 // Backward, staged lines: the fewest w per lane that cover W in one chunk, at
@@ -1023,9 +1023,32 @@ int flat_zl(int64_t W) { return W > 128 ? 4 : 2; }
 bool flat_short(const tsx_plan *p, int64_t W) { return W <= 64 && p->cols * ((W + 3) / 4 * 4) < (int64_t)1 << 24; }
 
 // The turned volume and its line of zeros.
-int64_t flat_turned_elems(const tsx_plan *p, int64_t batch)
+int64_t flat_layout_elems(const tsx_plan *p, int64_t batch)
 {
     return ((int64_t)p->nx * p->ny + 1) * flat_pitch(p, batch);
+}
+
+// Short lines, of which a wave reads many, are laid out for either stepping
+// axis, so that its rays meet neighbouring ones (360 angles, one layout and two:
+// 512^2 284 and 127 us, 4 slices of it 328 and 173, 12 slices of 256^2, 180 angles 80
+// and 67, 16 77 and 78).
+constexpr int FLAT_ACROSS = 16;
+
+bool flat_across(const tsx_plan *p, int64_t batch)
+{
+    return p->nz * batch < FLAT_ACROSS && p->axis_count[0] > 0 && p->axis_count[1] > 0;
+}
+
+int64_t flat_turned_elems(const tsx_plan *p, int64_t batch)
+{
+    return flat_layout_elems(p, batch) * (flat_across(p, batch) ? 2 : 1);
+}
+
+// (and no less than those of fewer entries)
+int64_t flat_turned_room(const tsx_plan *p, int64_t batch)
+{
+    const int64_t few = std::min<int64_t>(batch, (FLAT_ACROSS - 1) / p->nz);
+    return std::max(flat_turned_elems(p, batch), few > 0 ? flat_turned_elems(p, few) : 0);
 }
 
 // The least workspace floats of the flat forward projector: the turned volume
@@ -1043,7 +1066,7 @@ int64_t flat_fp_least(const tsx_plan *p)
 bool flat_fp_ok(const tsx_plan *p)
 {
     if (p->flat_host.empty() || force_general() || env_int("TSX_FP_VARIANT") >= 2 || !p->fp_padded) return false;
-    if (flat_turned_elems(p, 1) * 4 >= (int64_t)1 << 32) return false;  // 32-bit byte offsets
+    if (flat_layout_elems(p, 1) * 4 >= (int64_t)1 << 32) return false;  // 32-bit byte offsets
     const int64_t buffer = TSX_NOALLOC_SCRATCH_BYTES - p->outer[TSX_OP_FP];
     return flat_fp_least(p) * 4 <= buffer || fp_workspace_elems(p) * 4 > buffer;
 }
@@ -1065,13 +1088,7 @@ int64_t fp_elems(const tsx_plan *p, int64_t batch, bool least = false)
     const int64_t padded = fp_workspace_elems(p) * batch;
     if (!flat_fp_ok(p)) return padded;
     if (least) return std::max(padded, flat_fp_least(p));
-    return std::max(padded, flat_turned_elems(p, batch) + (int64_t)p->cols * flat_pitch(p, batch) * flat_angles(p));
-}
-
-// Blocks of the forward projector (four angles and `rays` columns each).
-int64_t flat_fp_blocks(int angles, int cols, int rays, int chunks)
-{
-    return (int64_t)((angles + 3) / 4) * ((cols + rays - 1) / rays) * chunks;
+    return std::max(padded, flat_turned_room(p, batch) + (int64_t)p->cols * flat_pitch(p, batch) * flat_angles(p));
 }
 
 // elems: the workspace's floats, where they are not those of fp_elems
@@ -1084,16 +1101,13 @@ FlatPlan flat_fp(const tsx_plan *p, int64_t batch, int64_t elems = 0)
         p->n_angles, ((elems ? elems : fp_elems(p, batch)) - flat_turned_elems(p, batch)) / ((int64_t)p->cols * Wp));
     // Chunks of w: one up to 127; of 64, whole cache lines, where they fit
     // (512^3, 360 angles: 9.9 ms, chunks of 76 17.1); else at most 80 (134^3,
-    // 360 angles: chunks of 68 0.26 ms, one 0.32). As many rays as fill a wave;
-    // fewer where that leaves fewer than 512 blocks (one slice, whose waves
-    // spend most of their time on weights: 2048. 512 x 512, 360 angles: 0.41
-    // ms with 64 rays, 0.35 so).
-    f.v = W < 4 ? 1 : 4;
+    // 360 angles: chunks of 68 0.26 ms, one 0.32). As many rays as fill a wave.
+    f.v = W < 3 ? (int)W : 4;
     f.chunks = (int)(W < 128 ? 1 : (W % 64 == 0 ? W / 64 : (W + 79) / 80));
     f.quads = (int)((Wp / f.v + f.chunks - 1) / f.chunks);
-    f.rays = std::min(FLAT_RAYS, 64 / f.quads);
-    while (f.rays > 8 && flat_fp_blocks(std::min(p->n_angles, f.per_launch), p->cols, f.rays, f.chunks) < (f.v == 1 ? 2048 : 512))
-        f.rays = (f.rays + 1) / 2;
+    f.own = f.quads == 1;
+    f.rays = 64 / f.quads;
+    f.stage = f.own ? 0 : (f.rays <= 8 ? 32 : (f.rays <= 16 ? 16 : 8));
     f.ok = true;
     return f;
 }
@@ -1133,7 +1147,7 @@ FlatPlan flat_bp(const tsx_plan *p, int64_t batch)
     if (!flat_bp_ok(p) || W > (1 << 28)) return f;
     f.shrt = flat_short(p, W);
     if (f.shrt) {
-        f.v = W < 4 ? 1 : 4;
+        f.v = W < 3 ? 1 : 4;
         const int q = (int)(flat_pitch(p, batch) / f.v);
         f.chunks = (q + 31) / 32;
         f.quads = (q + f.chunks - 1) / f.chunks;
@@ -1564,6 +1578,14 @@ FlatView flat_view(const tsx_plan *p, const FlatPlan &f, int64_t batch, int k0, 
     return v;
 }
 
+// The forward projector's layouts and sums in its workspace.
+void flat_place(const tsx_plan *p, int64_t batch, float *base, FlatView &v)
+{
+    v.turned = base;
+    v.across = flat_across(p, batch) ? base + flat_layout_elems(p, batch) : nullptr;
+    v.lines = base + flat_turned_elems(p, batch);
+}
+
 // The instances of one flat launch and the block counts of its passes.
 struct FlatBatch {
     FlatMulti m = {};
@@ -1609,9 +1631,28 @@ struct FlatBatch {
     {
         int rc = turn ? pass(flat_turn, flat_turn_blocks) : TSX_OK;
         if (rc) return rc;
-        rc = main_pass(f.v == 4 ? fp_flat<4> : fp_flat<1>, 4, 8, 128, [](const FlatView &v) {  // (large runs of blocks per XCD: whole strips share its L2)
-            return flat_fp_blocks(v.kn, v.cols, v.rays, v.chunks);
-        });
+        const auto blocks = [](const FlatView &v, bool split) {
+            return (int64_t)(split ? v.kn : (v.kn + 3) / 4) * ((v.cols + v.rays - 1) / v.rays) * v.chunks;
+        };
+        int64_t n = 0;
+        int rays = 64;
+        lds = 0;
+        for (int k = 0; k < m.n; ++k) {
+            n += blocks(m.v[k], false);
+            rays = std::min(rays, m.v[k].rays);
+            lds = std::max(lds, (size_t)(64 * m.v[k].stage * m.v[k].rays));
+        }
+        // Where blocks of four angles are few, a block's waves share the slices of
+        // one instead (same bits): below 4096 of one or two w, below 1536 of more
+        // where a wave has 8 rays or more (16 to 31 of w). Four angles and one, us:
+        // 256^2, 180 angles (270 blocks) 51 and 35; 1024^2, 360 (2160) 447 and 395;
+        // two slices, 720 (4320) 897 and 889; 20 x 256^2, 180 (1440) 106 and 97; 8 x
+        // 512^2, 360 (2160) 254 and 260; 64^3, 360 (2160, 4 rays) 49 and 58.
+        const bool split = f.v < 4 ? n < 4096 : n < 1536 && rays >= 8;
+        if (split) lds += 2 * 4 * 64 * 4 * f.v;
+        // (large runs of blocks per XCD: whole strips share its L2)
+        rc = main_pass(fp_flat_kernel(f.v, f.own, split), 4, 8, 128,
+                       [&](const FlatView &v) { return blocks(v, split); });
         return rc ? rc : pass(flat_rows, flat_rows_blocks);
     }
     int backward(const FlatPlan &f, int nc)
@@ -1679,8 +1720,7 @@ int launch_fp_flat(const tsx_plan *p, const float *vol, int64_t vs, float *proj,
             v.vs = vs;
             v.proj = proj + b0 * ps;
             v.ps = ps;
-            v.turned = base;
-            v.lines = base + flat_turned_elems(p, nb);
+            flat_place(p, nb, base, v);
             fb.m.v[0] = v;
             fb.m.n = 1;
             const int rc = fb.forward(f, k0 == 0);
@@ -2096,14 +2136,13 @@ int multi_fp(const tsx_plan *const *plans, const float *const *vols, float *cons
         for (int e = k; e < n && fb.m.n < FLAT_MAX; ++e) {
             if (taken[e] || !flat_one_launch(plans[e], TSX_OP_FP)) continue;
             const FlatPlan fe = flat_fp(plans[e], 1);
-            if (fe.v != f.v) continue;
+            if (fe.v != f.v || fe.own != f.own) continue;
             taken[e] = 1;
             FlatView &v = fb.m.v[fb.m.n++];
             v = flat_view(plans[e], fe, 1, 0, plans[e]->n_angles, eps[e]);
             v.vol = const_cast<float *>(vols[e]);
             v.proj = projs[e];
-            v.turned = (float *)((char *)wptr + off[e]);
-            v.lines = v.turned + flat_turned_elems(plans[e], 1);
+            flat_place(plans[e], 1, (float *)((char *)wptr + off[e]), v);
         }
         const int rc = fb.forward(f, true);
         if (rc) return rc;
