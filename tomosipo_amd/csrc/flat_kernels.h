@@ -56,12 +56,19 @@ struct FlatView {
     int chunks;             // chunks of w
 };
 
-struct FlatMulti {
-    FlatView v[FLAT_MAX];
-    int begin[FLAT_MAX + 1];
+template <int N>
+struct FlatArgs {
+    FlatView v[N];
+    int begin[N + 1];
     int n;
     int shift;  // chunk size of the XCD order (xcd_logical)
 };
+
+// Kernels take the arguments of one instance or of up to FLAT_MAX: those of a
+// full launch are 3.5 KB, which cost small calls 0.5 us on the host and 3 us
+// until their blocks had read them.
+using FlatOne = FlatArgs<1>;
+using FlatMulti = FlatArgs<FLAT_MAX>;
 
 template <int ZL>
 struct FlatVec {
@@ -126,7 +133,8 @@ __device__ __forceinline__ void flat_zero_line(float *base, int64_t lines, int W
     if (threadIdx.y == 0 && w < Wp) base[lines * Wp + w] = 0.0f;
 }
 
-__global__ void __launch_bounds__(256) flat_turn(FlatMulti M)
+template <typename Args>
+__global__ void __launch_bounds__(256) flat_turn(Args M)
 {
     __shared__ float tile[32][33];
     const int k = owner_of(M.begin, (int)blockIdx.x);
@@ -184,7 +192,8 @@ __device__ __forceinline__ FlatRow flat_row(const FlatAngle &A, int i, int j, in
     return r;
 }
 
-__global__ void __launch_bounds__(256) flat_rows(FlatMulti M)
+template <typename Args>
+__global__ void __launch_bounds__(256) flat_rows(Args M)
 {
     __shared__ float tile[32][33];
     __shared__ FlatRow rows_of[32];
@@ -253,7 +262,8 @@ __device__ __forceinline__ FlatSpan flat_span(const FlatAngle &A, int z, int j, 
     return s;
 }
 
-__global__ void __launch_bounds__(256) flat_splat(FlatMulti M)
+template <typename Args>
+__global__ void __launch_bounds__(256) flat_splat(Args M)
 {
     __shared__ float tile[32][33];
     __shared__ FlatSpan spans[32];
@@ -344,8 +354,8 @@ __device__ __forceinline__ FlatVec<V> flat_bload(__amdgpu_buffer_rsrc_t rs, uint
 // (a barrier per slice: 200^3, 360 angles, pitch sqrt 2 1.07 ms against 0.72
 // here; few blocks on small volumes: 80^3, 60 angles 0.09 against 0.03); one ray
 // per wave with weights from readlane (1.15 ms).
-template <int V, bool OWN, bool SPLIT>
-__global__ void __launch_bounds__(256) fp_flat(FlatMulti M)
+template <int V, bool OWN, bool SPLIT, typename Args>
+__global__ void __launch_bounds__(256) fp_flat(Args M)
 {
     constexpr int UN = 8;  // slices whose columns are in flight together
     extern __shared__ __align__(16) float flat_lds[];
@@ -609,8 +619,8 @@ __device__ __forceinline__ float flat_weight(const FlatAngle &A, double j0, doub
 // angles per step at ZL = 2 cost a block per CU (registers): 2.4 against 2.2
 // ms at 75 x 441 x 441, 361 angles, 75 x 623 (bp_wave: 6.3); 16 x 16 bricks
 // 3.1. 8 x 128^3, 180 angles, 128 x 192: 0.64 ms with the splat against 3.04.
-template <int ZL, int NC>
-__global__ void __launch_bounds__(64 * FLAT_BY) bp_flat(FlatMulti M)
+template <int ZL, int NC, typename Args>
+__global__ void __launch_bounds__(64 * FLAT_BY) bp_flat(Args M)
 {
     extern __shared__ __align__(16) float flat_lds[];
     constexpr int CF = 64 * ZL, AL = 4;  // floats per staged column; angles whose weights a wave holds
@@ -747,8 +757,8 @@ __global__ void __launch_bounds__(64 * FLAT_BY) bp_flat(FlatMulti M)
 // Columns along x of a block's tile of 4 rays (any shape takes the same time).
 __host__ __device__ inline int flat_tile(int rays) { return rays % 4 == 0 ? 16 : (rays % 2 == 0 ? 8 : 4); }
 
-template <int V, int NC>
-__global__ void __launch_bounds__(256) bp_flat_short(FlatMulti M)
+template <int V, int NC, typename Args>
+__global__ void __launch_bounds__(256) bp_flat_short(Args M)
 {
     constexpr int EN = NC == 2 ? 512 : 256;  // (angle, column) entries of a wave at a time
     constexpr int UN = NC == 2 ? 8 : 4;  // angles whose lines are in flight together
@@ -866,7 +876,8 @@ __global__ void __launch_bounds__(256) bp_flat_short(FlatMulti M)
 // voxel per thread, 62 with four.
 constexpr int FLAT_REDUCE = 1024;
 
-__global__ void __launch_bounds__(256) flat_parts_reduce(FlatMulti M)
+template <typename Args>
+__global__ void __launch_bounds__(256) flat_parts_reduce(Args M)
 {
     const FlatView &v = M.v[blockIdx.z];
     const int64_t ve = (int64_t)v.nx * v.ny * v.nz, o0 = (int64_t)blockIdx.x * FLAT_REDUCE;
@@ -894,26 +905,30 @@ __global__ void __launch_bounds__(256) flat_parts_reduce(FlatMulti M)
     }
 }
 
-using FlatKernel = void (*)(FlatMulti);
+template <typename Args>
+using FlatKernel = void (*)(Args);
 
-inline FlatKernel fp_flat_kernel(int v, bool own, bool split)
+template <typename A>
+FlatKernel<A> fp_flat_kernel(int v, bool own, bool split)
 {
-    if (!own) return split ? fp_flat<4, false, true> : fp_flat<4, false, false>;
-    if (v == 4) return split ? fp_flat<4, true, true> : fp_flat<4, true, false>;
-    if (v == 2) return split ? fp_flat<2, true, true> : fp_flat<2, true, false>;
-    return split ? fp_flat<1, true, true> : fp_flat<1, true, false>;
+    if (!own) return split ? fp_flat<4, false, true, A> : fp_flat<4, false, false, A>;
+    if (v == 4) return split ? fp_flat<4, true, true, A> : fp_flat<4, true, false, A>;
+    if (v == 2) return split ? fp_flat<2, true, true, A> : fp_flat<2, true, false, A>;
+    return split ? fp_flat<1, true, true, A> : fp_flat<1, true, false, A>;
 }
 
-inline FlatKernel bp_flat_kernel(int zl, int nc)
+template <typename A>
+FlatKernel<A> bp_flat_kernel(int zl, int nc)
 {
-    if (zl == 4) return nc == 2 ? bp_flat<4, 2> : (nc == 3 ? bp_flat<4, 3> : bp_flat<4, 4>);
-    return nc == 2 ? bp_flat<2, 2> : (nc == 3 ? bp_flat<2, 3> : bp_flat<2, 4>);
+    if (zl == 4) return nc == 2 ? bp_flat<4, 2, A> : (nc == 3 ? bp_flat<4, 3, A> : bp_flat<4, 4, A>);
+    return nc == 2 ? bp_flat<2, 2, A> : (nc == 3 ? bp_flat<2, 3, A> : bp_flat<2, 4, A>);
 }
 
-inline FlatKernel bp_flat_short_kernel(int v, int nc)
+template <typename A>
+FlatKernel<A> bp_flat_short_kernel(int v, int nc)
 {
-    if (v == 4) return nc == 2 ? bp_flat_short<4, 2> : (nc == 3 ? bp_flat_short<4, 3> : bp_flat_short<4, 4>);
-    return nc == 2 ? bp_flat_short<1, 2> : (nc == 3 ? bp_flat_short<1, 3> : bp_flat_short<1, 4>);
+    if (v == 4) return nc == 2 ? bp_flat_short<4, 2, A> : (nc == 3 ? bp_flat_short<4, 3, A> : bp_flat_short<4, 4, A>);
+    return nc == 2 ? bp_flat_short<1, 2, A> : (nc == 3 ? bp_flat_short<1, 3, A> : bp_flat_short<1, 4, A>);
 }
 
 }  // namespace tsx

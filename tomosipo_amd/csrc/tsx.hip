@@ -1606,30 +1606,39 @@ struct FlatBatch {
         pad_begin(m.begin, m.n);
         return n;
     }
-    template <typename K, typename F>
-    int pass(K kernel, F &&blocks)
+    // a kernel in its form for one instance or for all
+    int launch(FlatKernel<FlatOne> one, FlatKernel<FlatMulti> all, dim3 grid, dim3 block, size_t lds = 0)
     {
-        const int64_t n = lay(blocks, 256);
-        if (n < 0) return fail(TSX_ERR_UNSUPPORTED, "flat kernels: too many blocks for one launch");
-        if (n > 0) hipLaunchKernelGGL(kernel, dim3((unsigned)n), dim3(32, 8), 0, stream, m);
+        if (lds > 64 * 1024)
+            TSX_HIP_CHECK(hipFuncSetAttribute(m.n == 1 ? (const void *)one : (const void *)all,
+                                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+        if (m.n == 1) {
+            const FlatOne o = {{m.v[0]}, {m.begin[0], m.begin[1]}, 1, m.shift};
+            hipLaunchKernelGGL(one, grid, block, lds, stream, o);
+        } else {
+            hipLaunchKernelGGL(all, grid, block, lds, stream, m);
+        }
         TSX_HIP_CHECK(hipGetLastError());
         return TSX_OK;
     }
     template <typename F>
-    int main_pass(FlatKernel kernel, int waves, int most, int64_t chunks, F &&blocks)
+    int pass(FlatKernel<FlatOne> one, FlatKernel<FlatMulti> all, F &&blocks)
+    {
+        const int64_t n = lay(blocks, 256);
+        if (n < 0) return fail(TSX_ERR_UNSUPPORTED, "flat kernels: too many blocks for one launch");
+        return n > 0 ? launch(one, all, dim3((unsigned)n), dim3(32, 8)) : TSX_OK;
+    }
+    template <typename F>
+    int main_pass(FlatKernel<FlatOne> one, FlatKernel<FlatMulti> all, int waves, int most, int64_t chunks, F &&blocks)
     {
         const int64_t n = lay(blocks, 64 * waves);
         if (n < 0) return fail(TSX_ERR_UNSUPPORTED, "flat kernels: too many blocks for one launch");
         const unsigned grid = xcd_grid(n, &m.shift, most, chunks);
-        if (lds > 64 * 1024)
-            TSX_HIP_CHECK(hipFuncSetAttribute((const void *)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-        hipLaunchKernelGGL(kernel, dim3(grid), dim3(64 * waves), lds, stream, m);
-        TSX_HIP_CHECK(hipGetLastError());
-        return TSX_OK;
+        return launch(one, all, dim3(grid), dim3(64 * waves), lds);
     }
     int forward(const FlatPlan &f, bool turn)
     {
-        int rc = turn ? pass(flat_turn, flat_turn_blocks) : TSX_OK;
+        int rc = turn ? pass(flat_turn<FlatOne>, flat_turn<FlatMulti>, flat_turn_blocks) : TSX_OK;
         if (rc) return rc;
         const auto blocks = [](const FlatView &v, bool split) {
             return (int64_t)(split ? v.kn : (v.kn + 3) / 4) * ((v.cols + v.rays - 1) / v.rays) * v.chunks;
@@ -1651,13 +1660,13 @@ struct FlatBatch {
         const bool split = f.v < 4 ? n < 4096 : n < 1536 && rays >= 8;
         if (split) lds += 2 * 4 * 64 * 4 * f.v;
         // (large runs of blocks per XCD: whole strips share its L2)
-        rc = main_pass(fp_flat_kernel(f.v, f.own, split), 4, 8, 128,
+        rc = main_pass(fp_flat_kernel<FlatOne>(f.v, f.own, split), fp_flat_kernel<FlatMulti>(f.v, f.own, split), 4, 8, 128,
                        [&](const FlatView &v) { return blocks(v, split); });
-        return rc ? rc : pass(flat_rows, flat_rows_blocks);
+        return rc ? rc : pass(flat_rows<FlatOne>, flat_rows<FlatMulti>, flat_rows_blocks);
     }
     int backward(const FlatPlan &f, int nc)
     {
-        int rc = pass(flat_splat, flat_splat_blocks);
+        int rc = pass(flat_splat<FlatOne>, flat_splat<FlatMulti>, flat_splat_blocks);
         if (rc) return rc;
         int64_t ve = 0, blocks = 0;
         int entries = 0, angles = 0;
@@ -1685,14 +1694,14 @@ struct FlatBatch {
                 m.v[k].parts = 1;
                 sums = 0.0;
             }
-        rc = main_pass(f.shrt ? bp_flat_short_kernel(f.v, nc) : bp_flat_kernel(f.zl, nc), f.shrt ? 4 : FLAT_BY, 10, 2048,
-                       [](const FlatView &v) { return (int64_t)v.bx * v.by * v.chunks * v.parts; });
+        const auto blocks_of = [](const FlatView &v) { return (int64_t)v.bx * v.by * v.chunks * v.parts; };
+        rc = f.shrt ? main_pass(bp_flat_short_kernel<FlatOne>(f.v, nc), bp_flat_short_kernel<FlatMulti>(f.v, nc), 4, 10, 2048,
+                                blocks_of)
+                    : main_pass(bp_flat_kernel<FlatOne>(f.zl, nc), bp_flat_kernel<FlatMulti>(f.zl, nc), FLAT_BY, 10, 2048,
+                                blocks_of);
         if (rc || sums == 0.0) return rc;
-        hipLaunchKernelGGL(flat_parts_reduce,
-                           dim3((unsigned)((ve + FLAT_REDUCE - 1) / FLAT_REDUCE), (unsigned)entries, (unsigned)m.n),
-                           dim3(256), 0, stream, m);
-        TSX_HIP_CHECK(hipGetLastError());
-        return TSX_OK;
+        return launch(flat_parts_reduce<FlatOne>, flat_parts_reduce<FlatMulti>,
+                      dim3((unsigned)((ve + FLAT_REDUCE - 1) / FLAT_REDUCE), (unsigned)entries, (unsigned)m.n), dim3(256));
     }
 };
 
