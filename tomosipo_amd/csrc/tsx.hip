@@ -2815,13 +2815,15 @@ void set_outer(tsx_plan *p, int64_t fp, int64_t bp)
     if (p->fine) set_outer(p->fine, fp + align_ws(refined_sino(p) * 4), bp);
 }
 
-// The upright FDK backprojector, where its kernel takes the plan. (Its workspace
-// stays at 8 bytes per pixel, as callers size their buffers, of which it uses 4.)
+// The upright FDK backprojector, where its kernel takes the plan (the pixels of
+// one angle are numbered with 31 bits).
 bool fdk_staged(const tsx_plan *p)
 {
-    return p->fdk_upright && !force_general() && p->cols >= 2 &&
-           (int64_t)p->rows * p->n_angles * p->cols * 8 < ((int64_t)1 << 32);
+    return p->fdk_upright && !force_general() && p->cols >= 2 && (int64_t)p->rows * p->cols < ((int64_t)1 << 31);
 }
+
+// The filtered projections.
+int64_t fdk_workspace(const tsx_plan *p) { return (int64_t)p->rows * p->n_angles * p->cols * 4; }
 
 }  // namespace
 
@@ -3037,7 +3039,7 @@ int tsx_plan_info_get(const tsx_plan *p, tsx_plan_info *info)
 int tsx_fdk_workspace_size(const tsx_plan *p, int64_t *bytes)
 {
     if (!p || !bytes) return fail(TSX_ERR_INVALID_ARGUMENT, "plan and bytes must not be NULL");
-    *bytes = (int64_t)p->rows * p->n_angles * p->cols * (fdk_staged(p) ? 8 : 4);
+    *bytes = fdk_workspace(p);
     return TSX_OK;
 }
 
@@ -3062,10 +3064,9 @@ int tsx_fdk(const tsx_plan *p, float *vol, const float *proj, int additive, void
     EntryTimer entry_timer_("tsx_fdk", stream);
     hipStream_t s = (hipStream_t)stream;
     const bool upright = fdk_staged(p);
-    const int64_t need = (int64_t)p->rows * p->n_angles * p->cols * (upright ? 8 : 4);
     Scratch owned;
     void *wptr = nullptr;
-    rc = get_workspace(p, need, workspace, workspace_bytes, s, owned, &wptr);
+    rc = get_workspace(p, fdk_workspace(p), workspace, workspace_bytes, s, owned, &wptr);
     if (rc) return rc;
     float *q = (float *)wptr;
     const int nt = fdk_tiles(p->cols);
