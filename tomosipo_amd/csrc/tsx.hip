@@ -2418,22 +2418,31 @@ std::string tune_key(const tsx_plan *p)
            (p->fp_column_waves ? "c" : "r");
 }
 
-// Mean time of `reps` launches after one warm-up launch, in milliseconds.
+// Mean time of `reps` launches after one warm-up launch, in milliseconds; short
+// ones are repeated for half a millisecond, and the least of three means taken.
 template <typename F>
 int time_launches(F &&launch, hipStream_t stream, hipEvent_t e0, hipEvent_t e1, int reps, float *ms)
 {
     int rc = launch();
     if (rc) return rc;
-    TSX_HIP_CHECK(hipEventRecord(e0, stream));
-    for (int r = 0; r < reps; ++r) {
-        rc = launch();
-        if (rc) return rc;
+    *ms = 1e30f;
+    for (int tries = 0, most = 1; tries < most; ++tries) {
+        TSX_HIP_CHECK(hipEventRecord(e0, stream));
+        for (int r = 0; r < reps; ++r) {
+            rc = launch();
+            if (rc) return rc;
+        }
+        TSX_HIP_CHECK(hipEventRecord(e1, stream));
+        TSX_HIP_CHECK(hipEventSynchronize(e1));
+        float t = 0.0f;
+        TSX_HIP_CHECK(hipEventElapsedTime(&t, e0, e1));
+        if (tries == 0 && t < 0.5f) {  // (two launches of 30 us differ by a tenth from one trial to the next)
+            reps = (int)std::min(50.0f, std::ceil(reps * 0.5f / std::max(t, 1e-3f)));
+            most = 4;
+            continue;
+        }
+        *ms = std::min(*ms, t / reps);
     }
-    TSX_HIP_CHECK(hipEventRecord(e1, stream));
-    TSX_HIP_CHECK(hipEventSynchronize(e1));
-    float t = 0.0f;
-    TSX_HIP_CHECK(hipEventElapsedTime(&t, e0, e1));
-    *ms = t / reps;
     return TSX_OK;
 }
 
@@ -2664,14 +2673,16 @@ int autotune(tsx_plan *p, hipStream_t stream)
     }
     if (p->bp_separable && !force_general() && !bp_flat_used) {
         float best_ms = 1e30f;
-        // (a depth replaces an earlier one where it is faster by more than the trials scatter)
-        for (int bz : {32, 16, 24}) {
+        // (a depth replaces an earlier one where it is faster by more than the trials
+        // scatter: 0.5 %, 1 % for launches of 30 us. 24 deep against 32: 300 x 256^2
+        // 0.98, 75 x 441^2 0.99)
+        for (int bz : {32, 24, 16}) {
             sub.bp_bz = bz;
             float ms = 0.0f;
             int rc = time_launches([&] { return launch_bp(&sub, vol, 0, proj, 0, 1, ep, stream); },
                                    stream, t.e0, t.e1, 2, &ms);
             if (rc) return rc;
-            if (ms < 0.96f * best_ms) {
+            if (ms < 0.99f * best_ms) {
                 best_ms = ms;
                 best.bp_bz = bz;
             }
