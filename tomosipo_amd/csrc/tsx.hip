@@ -1908,12 +1908,34 @@ bool tilted_far(const tsx_plan *p)
     return false;
 }
 
+// Whether a cone's source lies so near the volume that the boxes of some voxels
+// span more than 8 times those of the central one, or are unbounded (voxels in
+// the source's plane, or behind it). A thread that goes through several of them
+// holds up the launch: 96^3, 20 angles, a source among the corners 11.5 ms with
+// eight voxels per thread, 0.78 with one; 128^3, 10 angles 0.24 and 0.13 (the
+// source just beyond the corners; at 8 times 0.105 and 0.110).
+bool tilted_uneven(const tsx_plan *p)
+{
+    if (p->kind != TSX_CONE_VEC) return false;
+    for (const AngleParams &A : p->host) {
+        const double c[3] = {0.5 * (A.n[0] - 1), 0.5 * (A.n[1] - 1), 0.5 * (A.n[2] - 1)};
+        double mid = 0.0, reach = 0.0;  // W . N at the centre, and how far it goes to the corners
+        for (int k = 0; k < 3; ++k) {
+            mid += (c[k] - A.S[k]) * A.N[k];
+            reach += c[k] * std::fabs(A.N[k]);
+        }
+        const double far = std::fabs(mid), near = far - reach;
+        if (!(near * 8.0 > far)) return true;
+    }
+    return false;
+}
+
 // Voxels per thread of bp_tilted: eight share a set-up, or two, or none where
 // more would leave fewer than four blocks per CU (of one entry: the choice
 // changes the rounding of positions, so it depends on the plan alone).
 int tilted_voxels(const tsx_plan *p)
 {
-    if (tilted_far(p)) return 1;
+    if (tilted_far(p) || tilted_uneven(p)) return 1;
     const int64_t columns = (int64_t)((p->nx + BP_BX - 1) / BP_BX) * ((p->ny + BP_BY - 1) / BP_BY);
     for (int zv : {8, 2})
         if (columns * ((p->nz + zv - 1) / zv) >= 1024) return zv;
