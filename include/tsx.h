@@ -155,6 +155,11 @@ typedef struct {
                                   backprojector: ss, the backprojection run on the detector
                                   refined ss times (its sub-rays as pixels); 0 otherwise. The
                                   bp_* fields above then describe that plan's kernels */
+    int32_t flat_kernels;      /* parallel scans whose rays stay within slices: 1 if the forward
+                                  projector, 2 if the backprojector, 3 if both run on the flat
+                                  kernels. The padded and separable kernels that the fields
+                                  above describe then run only where a variable asks for one
+                                  of theirs (TSX_FP_VARIANT, TSX_BP_BRICK_Z) */
 } tsx_plan_info;
 
 int tsx_plan_info_get(const tsx_plan *plan, tsx_plan_info *info);

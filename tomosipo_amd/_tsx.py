@@ -105,6 +105,7 @@ class TsxPlanInfo(ctypes.Structure):
         ("fp_column_waves", ctypes.c_int32),
         ("fp_refined_detector", ctypes.c_int32),
         ("bp_refined_detector", ctypes.c_int32),
+        ("flat_kernels", ctypes.c_int32),
     ]
 
 
@@ -236,6 +237,7 @@ class Plan:
             "fp_column_waves": bool(inf.fp_column_waves),
             "fp_refined_detector": inf.fp_refined_detector,
             "bp_refined_detector": inf.bp_refined_detector,
+            "fp_flat": bool(inf.flat_kernels & 1), "bp_flat": bool(inf.flat_kernels & 2),
         }
 
     def fdk_workspace_size(self):

@@ -3066,8 +3066,12 @@ int tsx_plan_info_get(const tsx_plan *p, tsx_plan_info *info)
     info->bp_launch_angles = info->bp_kernel ? bp_chunk_of(bs) : 0;
     info->bp_axis_swap = info->bp_kernel ? b->swap : 0;
     info->bp_refined_detector = b != p ? p->ss : 0;
+    info->flat_kernels = (flat_fp(f, 1).ok ? 1 : 0) | (flat_bp(bs, 1).ok ? 2 : 0);
     return TSX_OK;
 }
+
+// (the last field takes what was padding: callers of the structure without it pass as much room)
+static_assert(sizeof(tsx_plan_info) == 120, "the size of tsx_plan_info is part of the interface");
 
 int tsx_fdk_workspace_size(const tsx_plan *p, int64_t *bytes)
 {
