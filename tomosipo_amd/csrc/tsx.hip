@@ -3076,7 +3076,10 @@ static_assert(sizeof(tsx_plan_info) == 120, "the size of tsx_plan_info is part o
 int tsx_fdk_workspace_size(const tsx_plan *p, int64_t *bytes)
 {
     if (!p || !bytes) return fail(TSX_ERR_INVALID_ARGUMENT, "plan and bytes must not be NULL");
-    *bytes = fdk_workspace(p);
+    // (upright scans below 2^29 pixels: the size that callers have sized their
+    // buffers by, of which tsx_fdk needs half)
+    const bool twice = fdk_staged(p) && fdk_workspace(p) * 2 < ((int64_t)1 << 32);
+    *bytes = fdk_workspace(p) * (twice ? 2 : 1);
     return TSX_OK;
 }
 
