@@ -547,7 +547,7 @@ __device__ __forceinline__ void emit4(float *out, int64_t o, int64_t b, float4 a
 
 // Whether an instance's output rows (or voxels, where `row` is their number)
 // and its epilogue's data can be taken four at a time.
-__device__ __forceinline__ bool flat_quads(const FlatView &v, int64_t row)
+__host__ __device__ __forceinline__ bool flat_quads(const FlatView &v, int64_t row)
 {
     return (row & 3) == 0 && (((uintptr_t)v.vol | (uintptr_t)v.ep.y | (uintptr_t)v.ep.w) & 15) == 0 &&
            ((v.vs | v.ep.stride) & 3) == 0;
@@ -748,7 +748,7 @@ __global__ void __launch_bounds__(64 * FLAT_BY) bp_flat(Args M)
 // lane, and passed on through LDS; columns of no weight are read past the end
 // of the buffer, which gives zeros, so that an infinite pixel reaches no voxel
 // that its ray does not meet. The angle parts run in blocks of their own, or in
-// turn with their sums in registers, whose parts are then of a multiple of UN.
+// turn with their sums in registers (multiples of FLAT_PART angles).
 //
 // Bound: the L1 port (two 16-byte loads of 16 cycles each per 64 lanes; its
 // address unit 81 % busy at 64 x 256^2). Whole backprojection, 180 angles,
@@ -757,11 +757,14 @@ __global__ void __launch_bounds__(64 * FLAT_BY) bp_flat(Args M)
 // Columns along x of a block's tile of 4 rays (any shape takes the same time).
 __host__ __device__ inline int flat_tile(int rays) { return rays % 4 == 0 ? 16 : (rays % 2 == 0 ? 8 : 4); }
 
+constexpr int FLAT_PART = 4;
+
 template <int V, int NC, typename Args>
 __global__ void __launch_bounds__(256) bp_flat_short(Args M)
 {
     constexpr int EN = NC == 2 ? 512 : 256;  // (angle, column) entries of a wave at a time
     constexpr int UN = NC == 2 ? 8 : 4;  // angles whose lines are in flight together
+    constexpr int PART = FLAT_PART;
     constexpr uint32_t NONE = 0x80000000u;
     struct Entry {
         float w[NC];
@@ -793,7 +796,7 @@ __global__ void __launch_bounds__(256) bp_flat_short(Args M)
     FlatVec<V> acc, sum;  // of the present part, of those before it
 #pragma unroll
     for (int z = 0; z < V; ++z) acc.v[z] = sum.v[z] = 0.0f;
-    int left = v.part_len;  // angles of the present part (a multiple of UN where several run in turn)
+    int left = v.part_len;  // angles of the present part (a multiple of PART where several run in turn)
     for (int k0 = ka; k0 < kb; k0 += NS) {
         const int n = min(NS, kb - k0);
         int h = h0, c = c0;
@@ -835,21 +838,23 @@ __global__ void __launch_bounds__(256) bp_flat_short(Args M)
                     for (int i = 0; i < NC; ++i) u[e][i] = flat_bload<V>(rs, t[e].at[i] + lane_bytes);
                 __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-                for (int e = 0; e < UN; ++e)
+                for (int e = 0; e < UN; ++e) {
 #pragma unroll
                     for (int i = 0; i < NC; ++i)
 #pragma unroll
                         for (int z = 0; z < V; ++z) acc.v[z] = fmaf(t[e].w[i], u[e][i].v[z], acc.v[z]);
-                __builtin_amdgcn_sched_barrier(0);
-                left -= UN;
-                if (left == 0) {
-                    left = v.part_len;
+                    if (e % PART != PART - 1) continue;
+                    left -= PART;
+                    if (left == 0) {
+                        left = v.part_len;
 #pragma unroll
-                    for (int z = 0; z < V; ++z) {
-                        sum.v[z] += acc.v[z];
-                        acc.v[z] = 0.0f;
+                        for (int z = 0; z < V; ++z) {
+                            sum.v[z] += acc.v[z];
+                            acc.v[z] = 0.0f;
+                        }
                     }
                 }
+                __builtin_amdgcn_sched_barrier(0);
             }
         }
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
@@ -871,38 +876,38 @@ __global__ void __launch_bounds__(256) bp_flat_short(Args M)
 }
 
 // The sums of the angle parts added in order and written through the
-// epilogue, 1024 voxels per block: grid (voxels / 1024 of the largest instance,
-// entries, instances). Bound: memory; 8 x 128^3, four parts: 94 us with one
-// voxel per thread, 62 with four.
-constexpr int FLAT_REDUCE = 1024;
+// epilogue: grid (voxels of the largest instance / 256 M.shift, entries,
+// instances), M.shift voxels per thread: four where every instance allows it
+// (flat_reduce_quads), or one. Bound: memory; 8 x 128^3, four parts: 94 us with
+// one voxel per thread, 62 with four.
+__host__ __device__ __forceinline__ bool flat_reduce_quads(const FlatView &v)
+{
+    return !v.partial || (flat_quads(v, (int64_t)v.nx * v.ny * v.nz) && ((uintptr_t)v.partial & 15) == 0);
+}
 
 template <typename Args>
 __global__ void __launch_bounds__(256) flat_parts_reduce(Args M)
 {
     const FlatView &v = M.v[blockIdx.z];
-    const int64_t ve = (int64_t)v.nx * v.ny * v.nz, o0 = (int64_t)blockIdx.x * FLAT_REDUCE;
+    const int64_t ve = (int64_t)v.nx * v.ny * v.nz, o = ((int64_t)blockIdx.x * 256 + threadIdx.x) * M.shift;
     const int b = blockIdx.y;
-    if (!v.partial || o0 >= ve || b >= v.W / v.nz) return;
-    const float *pp = v.partial + (int64_t)b * v.parts * ve;
+    if (!v.partial || o >= ve || b >= v.W / v.nz) return;
+    const float *pp = v.partial + (int64_t)b * v.parts * ve + o;
     float *out = v.vol + b * v.vs;
-    if (flat_quads(v, ve) && ((uintptr_t)v.partial & 15) == 0) {
-        const int64_t o = o0 + 4 * threadIdx.x;
-        if (o >= ve) return;
-        FlatVec<4> t = flat_load<4>(pp + o);
+    if (M.shift == 4) {
+        FlatVec<4> t = flat_load<4>(pp);
 #pragma unroll 4
         for (int s = 1; s < v.parts; ++s) {
-            const FlatVec<4> u = flat_load<4>(pp + (int64_t)s * ve + o);
+            const FlatVec<4> u = flat_load<4>(pp + (int64_t)s * ve);
 #pragma unroll
             for (int e = 0; e < 4; ++e) t.v[e] += u.v[e];
         }
         emit4(out, o, b, make_float4(t.v[0], t.v[1], t.v[2], t.v[3]), v.ep);
         return;
     }
-    for (int64_t o = o0 + threadIdx.x; o < min(o0 + FLAT_REDUCE, ve); o += 256) {
-        float t = pp[o];
-        for (int s = 1; s < v.parts; ++s) t += pp[(int64_t)s * ve + o];
-        emit(out, o, b, t, v.ep);
-    }
+    float t = pp[0];
+    for (int s = 1; s < v.parts; ++s) t += pp[(int64_t)s * ve];
+    emit(out, o, b, t, v.ep);
 }
 
 template <typename Args>

@@ -1020,7 +1020,9 @@ int flat_zl(int64_t W) { return W > 128 ? 4 : 2; }
 // leave lanes idle there; 256^2, 180 angles: W = 16 91 and 323 us, 64 209 and
 // 373, 100 409 and 385; 128^2, 90 angles: 64 64 and 70, 70 80 and 70), which
 // addresses 32 angles with 31 bits.
-bool flat_short(const tsx_plan *p, int64_t W) { return W <= 64 && p->cols * ((W + 3) / 4 * 4) < (int64_t)1 << 24; }
+constexpr int FLAT_SHORT = 64;
+
+bool flat_short(const tsx_plan *p, int64_t W) { return W <= FLAT_SHORT && p->cols * ((W + 3) / 4 * 4) < (int64_t)1 << 24; }
 
 // The turned volume and its line of zeros.
 int64_t flat_layout_elems(const tsx_plan *p, int64_t batch)
@@ -1164,23 +1166,31 @@ FlatPlan flat_bp(const tsx_plan *p, int64_t batch)
 }
 
 // Angle parts of the flat backprojector, for the plans that bp_part_len_of
-// cuts into parts (never more of them: they use its workspace): parts of at
-// least 4 angles, about 256 blocks of 8 waves per launch of one entry where the
-// bricks alone give fewer than 128, and of no more angles than round least: n
-// angles in parts of L round with the variance 2 n L^2 / 3 within the parts and
-// n^3 / (3 L) where these are added, least at L = (n^2 / 4)^(1/3). Longer
-// parts only where the separable kernel's are (128^3 and slices of 256^2, 180
-// angles: two halves 1.6e-7 of the result, its parts of 45 1.0e-7).
+// cuts into parts (never more of them: they use its workspace): as many angles
+// as give about 256 blocks of 8 waves per launch of one entry where the bricks
+// alone give fewer than 128, but not so many that their sums round more than
+// the separable kernel's. n angles in parts of L round with the variance
+// 2 n L^2 / 3 within the parts and n^3 / (3 L) where these are added; of equal
+// parts the flat kernel's sums have 1 / 1.22 of the separable one's (128^3 and
+// slices of 256^2, 180 angles: two halves 1.6e-7 of the result, parts of 48 and
+// the separable kernel's of 45 1.0e-7). Volumes of few slices, which may run on
+// bp_flat_short, take the multiple of 4 that rounds least up to that length.
 int flat_part_len(const tsx_plan *p)
 {
-    const int cut = bp_part_len_of(p);
-    if (cut == p->n_angles) return cut;
+    const int cut = bp_part_len_of(p), n = p->n_angles;
+    if (cut == n) return cut;
     const int zl = flat_zl(p->nz);
     const int64_t blocks = std::min<int64_t>(128, flat_blocks(p, 8, (p->nz + 64 * zl - 1) / (64 * zl)));
-    const int64_t len = std::max<int64_t>(4, ((int64_t)p->n_angles * blocks + 255) / 256);
-    const int64_t least = (int64_t)std::ceil(std::cbrt(0.25 * p->n_angles * p->n_angles));
-    const int64_t part = (std::max<int64_t>(cut, std::min(len, least)) + 7) / 8 * 8;  // (groups of bp_flat_short)
-    return (int)std::min<int64_t>(part, p->n_angles);
+    int64_t len = std::max<int64_t>(cut, (n * blocks + 255) / 256);
+    const auto variance = [n](int64_t l) { return 2.0 * n * l * l / 3.0 + (double)n * n * n / (3.0 * l); };
+    while (len > cut && variance(len) > 1.22 * variance(cut)) --len;
+    if (p->nz <= FLAT_SHORT) {
+        const int64_t unit = FLAT_PART, low = (cut + unit - 1) / unit * unit, high = (len + unit - 1) / unit * unit;
+        len = low;
+        for (int64_t l = low; l <= high; l += unit)
+            if (variance(l) < variance(len)) len = l;
+    }
+    return (int)std::min<int64_t>(len, n);
 }
 
 // (least: as for fp_elems)
@@ -1700,8 +1710,12 @@ struct FlatBatch {
                     : main_pass(bp_flat_kernel<FlatOne>(f.zl, nc), bp_flat_kernel<FlatMulti>(f.zl, nc), FLAT_BY, 10, 2048,
                                 blocks_of);
         if (rc || sums == 0.0) return rc;
+        m.shift = 4;  // voxels per thread
+        for (int k = 0; k < m.n; ++k)
+            if (!flat_reduce_quads(m.v[k])) m.shift = 1;
+        const int64_t per = 256 * m.shift;
         return launch(flat_parts_reduce<FlatOne>, flat_parts_reduce<FlatMulti>,
-                      dim3((unsigned)((ve + FLAT_REDUCE - 1) / FLAT_REDUCE), (unsigned)entries, (unsigned)m.n), dim3(256));
+                      dim3((unsigned)((ve + per - 1) / per), (unsigned)entries, (unsigned)m.n), dim3(256));
     }
 };
 
