@@ -286,9 +286,10 @@ __global__ void scale_by_length(const AngleParams *__restrict__ angles, int n_an
 // take the FP64 set-up for each voxel and cut its box in FP64 (FAR: a
 // parallel scan has angles whose positions are; it has none else).
 //
-// Bound: vector ALU issue. 192^3 cone, 240 angles, 192 x 288 tilted by 0.2 rad:
-// 4.17 ms (103 instructions per 64 voxels and angle); with the set-up of every
-// voxel in FP64 and a loop over the pixels of each box 7.46 (234).
+// Bound: vector ALU issue (1.2 instructions per CU-cycle). 192^3 cone, 240
+// angles, 192 x 288 tilted by 0.2 rad: 4.03 ms (103 instructions per 64 voxels
+// and angle); with the set-up of every voxel in FP64 and a loop over the pixels
+// of each box 7.46 (234).
 struct TiltedVoxel {
     int j0, i0;     // pixel near the voxel's position
     float pj, pi;   // position relative to it

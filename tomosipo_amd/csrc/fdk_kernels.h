@@ -66,9 +66,11 @@ constexpr int fdk_filter_floats(int nt) { return 2 * (FDK_ROWS * (32 * nt + 4) +
 // floats apart keep both reads free of bank conflicts; the results go through
 // LDS to be written in rows.
 //
-// Bound: the matrix cores' FP32 rate (157 TFLOP/s; 2 cols FLOP per output,
-// half of the full product), with three blocks per CU at 768 columns so that
-// one loads while another multiplies. 512 x 720 rows of 768 columns: 3.0 ms (the sum
+// Bound: the phases of a block, which loads and weights its rows (an FP64 square
+// root per pixel), multiplies (cols FLOP per output, half of the full product: 1.4
+// ms of the 3.0 below at the matrix cores' 157 TFLOP/s in FP32) and stores;
+// three blocks per CU at 768 columns, so that one loads while another
+// multiplies. 512 x 720 rows of 768 columns: 3.0 ms (the sum
 // of factor (c[j - m] + c[j + m] - 2 c[j]) on the vector ALUs, register-tiled:
 // 10.4 ms; in this form there: 9.5 ms).
 template <int NT>
@@ -233,8 +235,9 @@ fdk_bp(const FdkAngle *__restrict__ angles, int n_angles, int rows, int cols,
 // corner is not in front of the source, the angle's pixels are read from
 // memory, each with its own bounds.
 //
-// Bound: LDS reads (two of 8 bytes per voxel and angle) and vector ALU issue
-// (12 instructions and the setup). A 16-byte gather from row-paired memory
+// Bound: vector ALU issue (1.06 instructions per CU-cycle: 12 per voxel and
+// angle and the setup), with 0.14 LDS reads (two of 8 bytes per voxel and
+// angle) beside it. A 16-byte gather from row-paired memory
 // took 16 cycles of the L1 port per wave: 512^3, 720 angles, 512 x 768
 // pixels 49.0 ms; 39.7 ms so.
 //

@@ -339,17 +339,18 @@ __device__ __forceinline__ FlatVec<V> flat_bload(__amdgpu_buffer_rsrc_t rs, uint
 // angles: 9.9 ms; angles before tiles, chunks of 256 of w: 19.4 ms).
 //
 // Bound: the L1 port and L2 (two 16-byte loads per lane, 8 fma, one LDS read
-// for 4 samples). fp_padded with its layouts against this with both layout
-// passes, pixel pitch sqrt 2 (in brackets 1):
-//   64^3, 180 angles      58 (72) and 35 (36) us
-//   128^3, 360 angles    0.40 (0.55) and 0.17 (0.21) ms
-//   256^3, 360 angles    2.17 (3.39) and 1.11 (1.43) ms
-//   512^3, 360 angles    15.4 and 10.0 ms
-//   75 x 441 x 441, 361  1.79 (2.81) and 1.28 (1.44) ms
-//   16 x (256 x 256), 180 angles 123 (137) and 69 (77) us
-//   1 x (256 x 256), 180 angles 60 (68) and 36 (35) us, 4 of them 65 (74) and 37 (41)
-//   1 x (512 x 512), 360 angles 292 (372) and 141 (127) us
-//   2 x (1024 x 1024), 720 angles 1.15 (1.32) and 0.73 (0.89) ms
+// for 4 samples; its address unit 74 % busy at 8 x 128^3, 85 % at 75 x 441^2).
+// fp_padded with its layouts against this with both layout passes, pixel pitch
+// sqrt 2 (in brackets 1):
+//   64^3, 180 angles      59 (66) and 30 (30) us
+//   128^3, 360 angles    0.38 (0.52) and 0.16 (0.20) ms
+//   256^3, 360 angles    2.06 (3.35) and 1.05 (1.36) ms
+//   512^3, 360 angles    15.1 and 9.3 ms
+//   75 x 441 x 441, 361  1.69 (2.73) and 1.16 (1.37) ms
+//   16 x (256 x 256), 180 angles 123 (137) and 65 (73) us
+//   1 x (256 x 256), 180 angles 60 (68) and 32 (31) us, 4 of them 65 (73) and 33 (37)
+//   1 x (512 x 512), 360 angles 292 (371) and 134 (119) us
+//   2 x (1024 x 1024), 720 angles 1.14 (1.33) and 0.69 (0.87) ms
 // Taken back: lines staged in LDS by blocks that go through the slices in step
 // (a barrier per slice: 200^3, 360 angles, pitch sqrt 2 1.07 ms against 0.72
 // here; few blocks on small volumes: 80^3, 60 angles 0.09 against 0.03); one ray
@@ -613,12 +614,14 @@ __device__ __forceinline__ float flat_weight(const FlatAngle &A, double j0, doub
 // zeros, so that an infinite or NaN pixel reaches no voxel that its ray does
 // not meet.
 //
-// Bound: vector ALU issue; per (voxel column, angle) NC + 1 readlane, NC
-// addresses and NC ZL fma (bp_wave: about 37 instructions per 64 voxels at
-// pixel pitch 1, where its 16-voxel bricks take two chunks of columns). Two
-// angles per step at ZL = 2 cost a block per CU (registers): 2.4 against 2.2
-// ms at 75 x 441 x 441, 361 angles, 75 x 623 (bp_wave: 6.3); 16 x 16 bricks
-// 3.1. 8 x 128^3, 180 angles, 128 x 192: 0.64 ms with the splat against 3.04.
+// Bound: vector ALU and LDS together, in step with the barriers (0.6 vector
+// instructions and 0.09 to 0.12 LDS reads of 8 to 16 bytes per lane and
+// CU-cycle); per (voxel column, angle) NC + 1 readlane, NC addresses, NC reads
+// and NC ZL fma (bp_wave: about 37 instructions per 64 voxels at pixel pitch 1,
+// where its 16-voxel bricks take two chunks of columns). Two angles per step at
+// ZL = 2 cost a block per CU (registers): 2.4 against 2.2 ms at 75 x 441 x 441,
+// 361 angles, 75 x 623 (bp_wave: 5.8); 16 x 16 bricks 3.1. 8 x 128^3, 180
+// angles, 128 x 192: 0.64 ms with the splat against 3.04.
 template <int ZL, int NC, typename Args>
 __global__ void __launch_bounds__(64 * FLAT_BY) bp_flat(Args M)
 {
@@ -751,9 +754,9 @@ __global__ void __launch_bounds__(64 * FLAT_BY) bp_flat(Args M)
 // turn with their sums in registers (multiples of FLAT_PART angles).
 //
 // Bound: the L1 port (two 16-byte loads of 16 cycles each per 64 lanes; its
-// address unit 81 % busy at 64 x 256^2). Whole backprojection, 180 angles,
-// pixel pitch 1, in brackets one w per lane: 256^2 46 us (250), 16 slices of it
-// 91 (260), 64 209 (290, kernel alone); 512^2 130 (870).
+// address unit 81 % busy at 64 x 256^2, 66 % at 16). Whole backprojection, 180
+// angles, pixel pitch 1, in brackets one w per lane and bp_wave: 256^2 42 us (250,
+// 183), 16 slices of it 74 (260, 265), 64 209 (290, 1141).
 // Columns along x of a block's tile of 4 rays (any shape takes the same time).
 __host__ __device__ inline int flat_tile(int rays) { return rays % 4 == 0 ? 16 : (rays % 2 == 0 ? 8 : 4); }
 

@@ -914,8 +914,8 @@ int bp_brick_z_of(const tsx_plan *p);
 // parts of part_len >= 4 consecutive sorted angles, so that bricks x parts
 // reaches about 1024 blocks (four per CU). Single launches run
 // the parts in separate blocks and add their sums in order (bp_parts_reduce);
-// fused launches run them in turn in one block and add them in the same order,
-// so both give the same sums. Volumes of 512 bricks or more, and plans whose
+// fused launches do that too, or run them in turn in one block and add them in
+// the same order (parts_apart), so all give the same sums. Volumes of 512 bricks or more, and plans whose
 // angles take several launches, keep one part. TSX_BP_PARTS=1 keeps one part
 // everywhere.
 int bp_part_len_of(const tsx_plan *p)
@@ -935,8 +935,7 @@ int bp_parts_of(const tsx_plan *p)
 
 // Length-weighted projections of one batch entry: transposed and padded
 // ([sorted angle][col][RPAD + row], scale_by_length_t) for the separable
-// kernel, for the angles of one launch; in the projections' own layout for
-// the general one.
+// kernel, for the angles of one launch; as [angle][row][col] for bp_tilted.
 int64_t bp_workspace_elems(const tsx_plan *p)
 {
     if (p->bp_separable) return (int64_t)bp_chunk_of(p) * p->cols * (p->rows + 2 * RPAD);
