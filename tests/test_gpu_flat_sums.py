@@ -88,6 +88,29 @@ def test_short_and_long_lines_hold_the_same_bits(nz, n, batches):
             assert torch.equal(out[k], want[k]), (batch, k)
 
 
+@pytest.mark.parametrize("nz", [1, 7, 8, 15, 16, 17, 33])
+@pytest.mark.parametrize("nx", [1, 15, 17, 30])
+def test_rows_of_any_length_hold_the_same_bits(nz, nx):
+    """Rows of no multiple of four voxels are written through a tile, 64 lanes' values at a time: lines of
+    two and four values per lane, in which a tile holds part of an entry, some, or many."""
+    A = _operator((nz, 21, nx), (nz, 34), 24)
+    plan, s = A.projector.plan(0), torch.cuda.current_stream().cuda_stream
+    n = int(np.prod(A.domain_shape))
+    gen = torch.Generator(device=DEV)
+    gen.manual_seed(nx)
+    most = 530 // nz
+    ys = torch.randn((most,) + A.range_shape, generator=gen, device=DEV)
+    want = [A.T(ys[k]).reshape(-1) for k in range(most)]
+    for batch in (70 // nz + 1, 130 // nz + 1, 270 // nz + 1, most):
+        for additive in (False, True):
+            out = torch.full((batch * (n + 3) + 8,), 2.0, device=DEV)
+            plan.backward(out[1:].data_ptr(), ys.data_ptr(), additive, s, batch, n + 3, ys[0].numel())
+            rows = out[1:][:batch * (n + 3)].reshape(batch, n + 3)
+            for k in range(batch):
+                assert torch.equal(rows[k, :n], want[k] + 2.0 if additive else want[k]), (batch, additive, k)
+            assert (out[0] == 2.0) and (rows[:, n:] == 2.0).all()
+
+
 @pytest.mark.parametrize("nz", [1, 2, 3, 4, 7, 20, 24, 36, 41, 48, 61, 64])
 @pytest.mark.parametrize("pitch,pixels", [(1.3, 40), (0.8, 60), (0.55, 90)])
 def test_short_lines_match_oracle(nz, pitch, pixels):

@@ -1157,7 +1157,7 @@ FlatPlan flat_bp(const tsx_plan *p, int64_t batch)
         f.zl = flat_zl(W);
         f.chunks = (int)((W + 64 * f.zl - 1) / (64 * f.zl));
         f.stage = p->flat_stage_bp;
-        f.lds = (size_t)2 * (f.stage + 1) * f.zl * 256;
+        f.lds = std::max((size_t)2 * (f.stage + 1) * f.zl * 256, (size_t)FLAT_BY * FLAT_TILE * 4);
     }
     f.per_launch = bp_chunk_of(p);
     f.ok = true;
