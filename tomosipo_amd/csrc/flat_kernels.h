@@ -567,13 +567,13 @@ __device__ __forceinline__ void flat_write(const FlatView &v, int part, int x0, 
                                            const FlatVec<ZL> (&acc)[FLAT_BX], float *tile)
 {
     static_assert(FLAT_BX == 16, "four rows of 16 voxels per store");
-    if (y >= v.ny) return;
     const int lane = threadIdx.x & 63;
     const int64_t ve = (int64_t)v.nx * v.ny * v.nz;
     Epilogue ep = v.ep;
     if (v.partial) ep.mode = EP_SET;
     const auto volume = [&](int b) { return v.partial ? v.partial + ((int64_t)b * v.parts + part) * ve : v.vol + b * v.vs; };
     if (flat_quads(v, v.nx)) {
+        if (y >= v.ny) return;
 #pragma unroll
         for (int z = 0; z < ZL; ++z) {
             const int w = w0 + lane * ZL + z;
@@ -588,6 +588,8 @@ __device__ __forceinline__ void flat_write(const FlatView &v, int part, int x0, 
         }
         return;
     }
+    __syncthreads();  // (the tile lies where the block staged its lines)
+    if (y >= v.ny) return;
     const int col = lane % FLAT_BX, first = lane / FLAT_BX;
     constexpr int STEP = 64 / FLAT_BX * ZL;  // in w, from one store to the next
 #pragma unroll
@@ -766,7 +768,6 @@ __global__ void __launch_bounds__(64 * FLAT_BY) bp_flat(Args M)
             __builtin_amdgcn_sched_barrier(0);
         }
     }
-    __syncthreads();  // (every wave is done with the staged lines)
     flat_write<ZL>(v, part, x0, y0 + wv, w0, acc, flat_lds + wv * FLAT_TILE);
 }
 
